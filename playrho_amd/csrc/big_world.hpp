@@ -20,10 +20,20 @@ constexpr int kBigColorRounds = 40; // colouring rounds before the rest goes to 
 // Indices into BigState::counters.
 // kBigEpoch counts colourings (claim keys are stamped with it); kBigLeft and
 // kBigLeft + 1 hold the uncoloured count of the last two rounds; kBigRounds
-// the rounds the last colouring took.
+// the rounds the last colouring took; kBigWork the contacts left to its last
+// rounds.  kBigStep counts steps (key-set entries carry it), kBigFirstGone is
+// the first destroyed contact, kBigKept the contacts kept, kBigTail the first
+// colour swept by the one-workgroup launch.
 enum : int {
     kBigPairs = 0, kBigColors = 1, kBigTouching = 2, kBigMinSepBits = 3, kBigEpoch = 4, kBigLeft = 5,
-    kBigRounds = 7, kBigCounters = 8
+    kBigRounds = 7, kBigStep = 8, kBigFirstGone = 9, kBigKept = 10, kBigWork = 11, kBigTail = 12, kBigCounters = 13
+};
+// A step's pair searches (before the solve, after it, after each of the two
+// time-of-impact passes) and their words: moved proxies, overlapping pairs,
+// new pairs, workgroups done, and the bounds of the AABB centres (keys).
+constexpr int kFindSlots = 4;
+enum : int {
+    kFindMoved = 0, kFindHits, kFindFresh, kFindDone, kFindLoX, kFindLoY, kFindHiX, kFindHiY, kFindWords
 };
 // Indices into BigState::metrics.
 enum : int { kBigMinSeparation = 0, kBigMetrics = 4 };
@@ -42,11 +52,17 @@ struct BigState {
     int* visit;   // P-1
     float4* naabb;  // 2P-1
     float4* bounds;
-    // Candidate pairs.
     int* pcount;   // P + 1
     int2* pairs;   // pairCap
-    int* paccept;  // pairCap
-    std::uint64_t* hash;  // hashMask + 1
+    // The step's pair search.
+    std::uint64_t* hash;         // hashMask + 1: set of existing contact keys
+    int* moved;                  // P: moved proxies
+    unsigned long long* fresh;   // pairCap: new pairs
+    int* find;                   // kFindSlots * kFindWords
+    // Per workgroup range of 256 contacts: kept or touching contacts, and
+    // touching contacts per colour.
+    int* blockSum;
+    int* blockHist;
     // Colouring and solve order.
     int* list;
     int* list2;

@@ -34,6 +34,7 @@ extern "C" hipError_t prx_launch_step(const prx::DeviceState* d, const prx::Step
                                       hipStream_t stream);
 extern "C" hipError_t prx_big_launch_step(const prx::DeviceState* d, const prx::BigState* g,
                                           const prx::StepParams* c, hipStream_t s);
+extern "C" hipError_t prx_big_prepare(int nbodies);
 extern "C" hipError_t prx_big_launch_pairs(const prx::DeviceState* d, const prx::BigState* g, hipStream_t s);
 extern "C" int prx_lbvh_pairs_noalloc_impl(const float* aabbs, const std::int32_t* bodies, const std::uint8_t* moved,
                                            int n, std::int32_t* pairs, int cap, int* count, void* stream,
@@ -3167,12 +3168,10 @@ std::size_t NextPow2(std::size_t v) {
     return p;
 }
 
-int AllocBig(DeviceArena& a, prx::BigState& g, int P, int B, int cap) {
+// Working arrays of the linear BVH over P proxies.
+int AllocLbvh(DeviceArena& a, prx::BigState& g, int P) {
     g.P = std::max(P, 1);
-    g.B = std::max(B, 1);
-    g.cap = std::max(cap, 1);
     g.pairCap = std::max(16 * g.P, 1024);
-    g.hashMask = int(NextPow2(std::size_t(2 * g.cap))) - 1;
     const std::size_t n = std::size_t(g.P), nodes = 2 * n;
     PRX_HIP(a.alloc(g.morton, n));
     PRX_HIP(a.alloc(g.morton2, n));
@@ -3187,8 +3186,26 @@ int AllocBig(DeviceArena& a, prx::BigState& g, int P, int B, int cap) {
     PRX_HIP(a.alloc(g.bounds, 1));
     PRX_HIP(a.alloc(g.pcount, n + 1));
     PRX_HIP(a.alloc(g.pairs, std::size_t(g.pairCap)));
-    PRX_HIP(a.alloc(g.paccept, std::size_t(g.pairCap)));
-    PRX_HIP(a.alloc(g.hash, std::size_t(g.hashMask) + 1));
+    PRX_HIP(a.alloc(g.counters, std::size_t(prx::kBigCounters)));
+    PRX_HIP(hipMemset(g.counters, 0, sizeof(int) * prx::kBigCounters));
+    return PRX_OK;
+}
+
+// State of the large-world step (P proxies, B bodies, contact capacity cap).
+int AllocBig(DeviceArena& a, prx::BigState& g, int P, int B, int cap) {
+    g.P = std::max(P, 1);
+    g.B = std::max(B, 1);
+    g.cap = std::max(cap, 1);
+    g.pairCap = std::max(16 * g.P, 1024);
+    g.hashMask = int(NextPow2(std::size_t(2 * g.cap))) - 1;
+    const std::size_t hash = std::size_t(g.hashMask) + 1, blocks = std::size_t(g.cap) / 256 + 1;
+    PRX_HIP(a.alloc(g.hash, hash));
+    PRX_HIP(hipMemset(g.hash, 0, sizeof(std::uint64_t) * hash));
+    PRX_HIP(a.alloc(g.moved, std::size_t(g.P)));
+    PRX_HIP(a.alloc(g.fresh, std::size_t(g.pairCap)));
+    PRX_HIP(a.alloc(g.find, std::size_t(prx::kFindSlots * prx::kFindWords)));
+    PRX_HIP(a.alloc(g.blockSum, blocks));
+    PRX_HIP(a.alloc(g.blockHist, blocks * (prx::kBigMaxColors + 1)));
     PRX_HIP(a.alloc(g.list, std::size_t(g.cap)));
     PRX_HIP(a.alloc(g.list2, std::size_t(g.cap)));
     PRX_HIP(a.alloc(g.color, std::size_t(g.cap)));
@@ -3196,7 +3213,6 @@ int AllocBig(DeviceArena& a, prx::BigState& g, int P, int B, int cap) {
     PRX_HIP(hipMemset(g.claim, 0xff, sizeof(unsigned long long) * std::size_t(g.B) * prx::kBigMaxColors));
     PRX_HIP(a.alloc(g.used, std::size_t(g.B)));
     PRX_HIP(a.alloc(g.tent, std::size_t(g.cap)));
-    PRX_HIP(a.alloc(g.win, std::size_t(g.cap)));
     PRX_HIP(a.alloc(g.colorStart, std::size_t(prx::kBigMaxColors + 2)));
     PRX_HIP(a.alloc(g.toiKey, std::size_t(g.B)));
     PRX_HIP(hipMemset(g.toiKey, 0xff, sizeof(unsigned long long) * std::size_t(g.B)));
@@ -3204,7 +3220,9 @@ int AllocBig(DeviceArena& a, prx::BigState& g, int P, int B, int cap) {
     PRX_HIP(a.alloc(g.sweep, std::size_t(prx::kBigSweepSlots)));
     PRX_HIP(a.alloc(g.counters, std::size_t(prx::kBigCounters)));
     PRX_HIP(a.alloc(g.metrics, std::size_t(prx::kBigMetrics)));
-    PRX_HIP(hipMemset(g.counters, 0, sizeof(int) * prx::kBigCounters));
+    int counters[prx::kBigCounters] = {};
+    counters[prx::kBigFirstGone] = 0x7fffffff;
+    PRX_HIP(hipMemcpy(g.counters, counters, sizeof(counters), hipMemcpyHostToDevice));
     PRX_HIP(hipMemset(g.metrics, 0, sizeof(float) * prx::kBigMetrics));
     return PRX_OK;
 }
@@ -3248,6 +3266,10 @@ int prx_big_create(prx_world* w, prx_big** out) {
     if (int st = AllocBig(big->arena, big->g, int(b->totP), int(b->totB), int(b->totC))) {
         prx_batch_destroy(b);
         return st;
+    }
+    if (const hipError_t e = prx_big_prepare(big->g.B); e != hipSuccess) {
+        prx_batch_destroy(b);
+        return Fail(PRX_E_DEVICE, std::string("LDS limit: ") + hipGetErrorString(e));
     }
     *out = big.release();
     return PRX_OK;
@@ -3344,7 +3366,7 @@ int prx_lbvh_pairs(const float* aabbs, const std::int32_t* bodies, const std::ui
     PRX_HIP(a.alloc(d.paabb, std::size_t(n)));
     PRX_HIP(a.alloc(d.pbody, std::size_t(n)));
     PRX_HIP(a.alloc(d.pflags, std::size_t(n)));
-    if (int st = AllocBig(a, g, n, 1, 1)) return st;
+    if (int st = AllocLbvh(a, g, n)) return st;
     prx::WorldHeader h{};
     h.nproxies = n;
     h.nbodies = 0;

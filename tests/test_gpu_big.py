@@ -268,3 +268,27 @@ def test_big_world_20k_against_reference_measures(toi):
         ke_tol = 0.01 if s < 600 else (0.03 if toi else 0.15)
         assert abs(got["kinetic_energy"] - r["kinetic_energy"]) <= ke_tol * r["kinetic_energy"]
         assert abs(got["total_mass"] - r["total_mass"]) <= 1e-6 * r["total_mass"]
+
+
+@pytest.mark.parametrize("bodies,toi", [(12, False), (300, True), (900, True)])
+def test_big_solve_forms_agree(bodies, toi):
+    """The one-workgroup solve (few bodies) and the grid's launches (many) give
+    the same bits: bodies without shapes added to the world move it to the
+    second form and change nothing else."""
+    conf = pa.StepConf(do_toi=1 if toi else 0)
+    states = []
+    for extra in (0, 4200):
+        w = pa.World.scene("drop", [bodies, 10, 40, 5])
+        for _ in range(extra):
+            w.create_body(pa.BodyConf())
+        big = pa.BigWorld(w)
+        big.step(conf, 150)
+        big.sync()
+        states.append(dumpfmt.read_state(dumpfmt.Reader(w.state_record())))
+    small, grid = states
+    n = small["bodies"].shape[0]
+    assert (small["ct"][:, 0] & 0xff).any() and len(small["cu"]) > bodies // 2
+    for k in ("bodies", "bflags"):
+        assert np.array_equal(small[k].view(np.uint32), grid[k][:n].view(np.uint32)), k
+    for k in ("cu", "ct", "cf", "paabb"):
+        assert np.array_equal(small[k].view(np.uint32), grid[k].view(np.uint32)), k
