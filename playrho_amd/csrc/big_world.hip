@@ -859,18 +859,22 @@ __global__ __launch_bounds__(kGrid) void k_big_touch_list(DeviceState d, BigStat
     if (moves(d, bd.y)) atomicMin(&g.claim[bd.y * prx::kBigMaxColors], key);
 }
 
-// Claims and used masks are changed by atomics of other workgroups' threads
-// and, in the last rounds, read back in the same launch: agent-scope loads.
+// Claims and used masks are changed by atomics; a round that runs in the same
+// launch as the one before (kSame) reads them with agent-scope loads.
+template <bool kSame>
 __device__ __forceinline__ unsigned long long seen64(const void* p) {
-    return __hip_atomic_load(static_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (kSame)
+        return __hip_atomic_load(static_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else return *static_cast<const unsigned long long*>(p);
 }
 
+template <bool kSame>
 __device__ __forceinline__ void col_propose(const DeviceState& d, const BigState& g, int round, int e) {
     const int2 bd = d.c_body[g.list[e]];
     const bool ma = moves(d, bd.x), mb = moves(d, bd.y);
     std::uint64_t mask = 0ull;
-    if (ma) mask |= seen64(g.used + bd.x);
-    if (mb) mask |= seen64(g.used + bd.y);
+    if (ma) mask |= seen64<kSame>(g.used + bd.x);
+    if (mb) mask |= seen64<kSame>(g.used + bd.y);
     const unsigned long long freeCols = ~mask & ((1ull << prx::kBigMaxColors) - 1ull);
     const int col = freeCols ? (__ffsll(freeCols) - 1) : -1;
     g.tent[e] = col;
@@ -882,14 +886,15 @@ __device__ __forceinline__ void col_propose(const DeviceState& d, const BigState
 
 // Whether contact e won its claims (and took its colour); ncol grows to the
 // colours in use.
+template <bool kSame>
 __device__ __forceinline__ bool col_commit(const DeviceState& d, const BigState& g, int round, int e, int& ncol) {
     const int col = g.tent[e];
     if (col < 0) return false;
     const int2 bd = d.c_body[g.list[e]];
     const bool ma = moves(d, bd.x), mb = moves(d, bd.y);
     const unsigned long long key = claim_key(g, round, e);
-    if (ma && seen64(&g.claim[bd.x * prx::kBigMaxColors + col]) != key) return false;
-    if (mb && seen64(&g.claim[bd.y * prx::kBigMaxColors + col]) != key) return false;
+    if (ma && seen64<kSame>(&g.claim[bd.x * prx::kBigMaxColors + col]) != key) return false;
+    if (mb && seen64<kSame>(&g.claim[bd.y * prx::kBigMaxColors + col]) != key) return false;
     g.color[e] = col;
     const unsigned long long bit = 1ull << col;
     if (ma) atomicOr(reinterpret_cast<unsigned long long*>(g.used + bd.x), bit);
@@ -909,7 +914,7 @@ __global__ __launch_bounds__(kGrid) void k_col_propose(DeviceState d, BigState g
     if (done) return;
     const int m = g.counters[prx::kBigTouching];
     for (int e = int(blockIdx.x * blockDim.x + threadIdx.x); e < m; e += int(gridDim.x * blockDim.x))
-        if (g.color[e] < 0) col_propose(d, g, round, e);
+        if (g.color[e] < 0) col_propose<false>(d, g, round, e);
 }
 
 // keepWork: the contacts left go to the work list (list2) of k_col_rest.
@@ -918,7 +923,7 @@ __global__ __launch_bounds__(kGrid) void k_col_commit(DeviceState d, BigState g,
     const int m = g.counters[prx::kBigTouching];
     int left = 0, ncol = 0;
     for (int e = int(blockIdx.x * blockDim.x + threadIdx.x); e < m; e += int(gridDim.x * blockDim.x)) {
-        if (g.color[e] >= 0 || col_commit(d, g, round, e, ncol)) continue;
+        if (g.color[e] >= 0 || col_commit<false>(d, g, round, e, ncol)) continue;
         ++left;
         if (keepWork) g.list2[atomicAdd(&g.counters[prx::kBigWork], 1)] = e;
     }
@@ -935,10 +940,12 @@ __global__ __launch_bounds__(kGrid) void k_col_commit(DeviceState d, BigState g,
 }
 
 // The rounds from `first` on, by one workgroup over the contacts the grid's
-// rounds left (a few per cent after kGridRounds): a round here costs a
-// workgroup barrier instead of two launches (7.5 us a round before, 80
-// launches a step whether or not contacts were left).
-constexpr int kGridRounds = 4;
+// rounds left: a round here costs two workgroup barriers instead of two
+// launches.  The lowest list position wins a claim, so a round colours a tenth
+// to a half of what is left: of 49,000 touching contacts 22,000 are left after
+// 4 rounds and 1,000 after 8, of which the rest take 6 to 8 rounds more.  With
+// 4 grid rounds this kernel took 340 us.
+constexpr int kGridRounds = 8;
 __global__ __launch_bounds__(kBlock) void k_col_rest(DeviceState d, BigState g, int first) {
     __shared__ int s_left, s_ncol;
     const int n = g.counters[prx::kBigWork];
@@ -948,14 +955,14 @@ __global__ __launch_bounds__(kBlock) void k_col_rest(DeviceState d, BigState g, 
         if (threadIdx.x == 0) s_left = s_ncol = 0;
         for (int k = int(threadIdx.x); k < n; k += kBlock) {
             const int e = g.list2[k];
-            if (g.color[e] < 0) col_propose(d, g, round, e);
+            if (g.color[e] < 0) col_propose<true>(d, g, round, e);
         }
         __threadfence();
         __syncthreads();
         int left = 0, ncol = 0;
         for (int k = int(threadIdx.x); k < n; k += kBlock) {
             const int e = g.list2[k];
-            if (g.color[e] < 0 && !col_commit(d, g, round, e, ncol)) ++left;
+            if (g.color[e] < 0 && !col_commit<true>(d, g, round, e, ncol)) ++left;
         }
         if (left) atomicAdd(&s_left, left);
         if (ncol) atomicMax(&s_ncol, ncol);
@@ -972,24 +979,43 @@ __global__ __launch_bounds__(kBlock) void k_col_rest(DeviceState d, BigState g, 
     if (threadIdx.x == 0) g.counters[prx::kBigRounds] = round;
 }
 
-constexpr int kBuckets = prx::kBigMaxColors + 1;  // the colours, then the serial bucket
+// The colour order: within a colour the contacts with two manifold points come
+// first, so that a wavefront's updates take one path of the velocity solve
+// (block or sequential) and of the position solve; the order within a colour
+// does not change a result.  Two buckets per colour, then the serial bucket
+// (list order).
+constexpr int kColourBuckets = 2 * prx::kBigMaxColors;
+constexpr int kBuckets = kColourBuckets + 1;
+__device__ __forceinline__ int colour_bucket(const DeviceState& d, const BigState& g, int e) {
+    const int col = g.color[e];
+    if (col < 0) return kColourBuckets;
+    return 2 * col + (((d.m_hdr[g.list[e]].x >> 8) & 0xffu) == 2u ? 0 : 1);
+}
 constexpr int kTailContacts = 2048;
 
-// Colour counts of each workgroup's range of the touching list; contacts left
-// uncoloured go to a last bucket solved by one thread in list order.
-__global__ __launch_bounds__(kGrid) void k_big_buckets(BigState g) {
+// Bucket counts of each workgroup's range of the touching list.
+__global__ __launch_bounds__(kGrid) void k_big_buckets(DeviceState d, BigState g) {
     __shared__ int s_cnt[kBuckets];
     const int m = g.counters[prx::kBigTouching];
     const int blk = int(blockIdx.x), e = blk * kGrid + int(threadIdx.x);
     if (blk * kGrid >= m) return;
     if (threadIdx.x < kBuckets) s_cnt[threadIdx.x] = 0;
     __syncthreads();
-    if (e < m) {
-        if (g.color[e] < 0) g.color[e] = prx::kBigMaxColors;
-        atomicAdd(&s_cnt[g.color[e]], 1);
-    }
+    if (e < m) atomicAdd(&s_cnt[colour_bucket(d, g, e)], 1);
     __syncthreads();
     if (threadIdx.x < kBuckets) g.blockHist[blk * kBuckets + int(threadIdx.x)] = s_cnt[threadIdx.x];
+}
+
+// The wave's lanes holding the same bucket.
+__device__ __forceinline__ unsigned long long bucket_peers(bool valid, int bucket) {
+    unsigned long long peers = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+        const bool bit = (bucket >> b) & 1;
+        const unsigned long long mm = __ballot(bit);
+        peers &= bit ? mm : ~mm;
+    }
+    return peers;
 }
 
 // The velocity and position constraint record of contact gi at place e of
@@ -1034,14 +1060,8 @@ __global__ __launch_bounds__(kGrid) void k_big_records(DeviceState d, BigState g
         if (k / kBuckets < blk) atomicAdd(&s_before[col], cnt);
     }
     const bool valid = e < m;
-    const int col = valid ? g.color[e] : 0;
-    unsigned long long peers = __ballot(valid);
-#pragma unroll
-    for (int b = 0; b < 5; ++b) {
-        const bool bit = (col >> b) & 1;
-        const unsigned long long mm = __ballot(bit);
-        peers &= bit ? mm : ~mm;
-    }
+    const int col = valid ? colour_bucket(d, g, e) : 0;
+    const unsigned long long peers = bucket_peers(valid, col);
     const int rank = __popcll(peers & lanes_below(lane));
     if (valid && rank == 0) s_wave[wave][col] = __popcll(peers);
     __syncthreads();
@@ -1055,12 +1075,14 @@ __global__ __launch_bounds__(kGrid) void k_big_records(DeviceState d, BigState g
     }
     __syncthreads();
     if (blk == 0) {
-        if (threadIdx.x <= kBuckets) g.colorStart[threadIdx.x] = s_start[threadIdx.x];
-        // The sweeps' last launch takes every colour from the first whose
-        // successors hold few contacts in all (k_big_sweep).
+        // colorStart: the colours' starts, the serial bucket's, the end.
+        if (threadIdx.x <= prx::kBigMaxColors) g.colorStart[threadIdx.x] = s_start[2 * threadIdx.x];
         if (threadIdx.x == 0) {
-            int k = kBuckets - 1;
-            while (k > 0 && m - s_start[k - 1] <= kTailContacts) --k;
+            g.colorStart[prx::kBigMaxColors + 1] = m;
+            // The sweeps' last launch takes every colour from the first whose
+            // successors hold few contacts in all (k_big_sweep).
+            int k = prx::kBigMaxColors;
+            while (k > 0 && m - s_start[2 * (k - 1)] <= kTailContacts) --k;
             g.counters[prx::kBigTail] = k;
         }
     }
@@ -1081,37 +1103,53 @@ __global__ __launch_bounds__(kGrid) void k_big_records(DeviceState d, BigState g
 // kTailContacts contacts in all, and the grid's launches of later colours
 // return at once.  A launch for each of the 16 colours and the serial bucket
 // spent 2.5 us on every empty one.
-constexpr int kGridColours = 6;
+constexpr int kGridColours = 7;
 
-// The sweeps' work on the constraint of place e; the body state in bs.
+// The sweeps' work on a constraint: its record (float4 kRec of them, read
+// ahead by the one-workgroup sweeps) and the update, with the body state in bs.
 struct WarmSweep {
     static constexpr bool kMin = false;
+    static constexpr int kRec = prx::kVcStride;
+    static __device__ __forceinline__ const float4* rec(const DeviceState& d, int e) {
+        return d.s_vc + std::size_t(e) * prx::kVcStride;
+    }
     template <bool kLds>
-    static __device__ __forceinline__ float one(const DeviceState& d, const StepParams&, const Bodies<kLds>& bs, int e) {
+    static __device__ __forceinline__ float one(const DeviceState&, const StepParams&, const Bodies<kLds>& bs,
+                                                const float4 (&r)[kRec], int) {
         BodyC A, B;
-        const Vc vc = load_vc(d.s_vc + std::size_t(e) * prx::kVcStride, A, B);
+        const Vc vc = load_vc(r, A, B);
         warm_start_one(vc, A, B, bs);  // WarmStartVelocities, AabbTreeWorld.cpp:264-274
         return 0.0f;
     }
 };
 struct VelocitySweep {
     static constexpr bool kMin = false;
+    static constexpr int kRec = prx::kVcStride;
+    static __device__ __forceinline__ const float4* rec(const DeviceState& d, int e) {
+        return d.s_vc + std::size_t(e) * prx::kVcStride;
+    }
     template <bool kLds>
-    static __device__ __forceinline__ float one(const DeviceState& d, const StepParams&, const Bodies<kLds>& bs, int e) {
-        float4* rec = d.s_vc + std::size_t(e) * prx::kVcStride;
+    static __device__ __forceinline__ float one(const DeviceState& d, const StepParams&, const Bodies<kLds>& bs,
+                                                const float4 (&r)[kRec], int e) {
+        float4* out = d.s_vc + std::size_t(e) * prx::kVcStride;
         BodyC A, B;
-        Vc vc = load_vc(rec, A, B);
+        Vc vc = load_vc(r, A, B);
         const float mi = solve_velocity_one(vc, A, B, bs);  // SolveVelocityConstraintsViaGS
-        rec[4] = float4{vc.p[0].ni, vc.p[0].ti, vc.p[0].nm, vc.p[0].tm};
-        rec[7] = float4{vc.p[1].ni, vc.p[1].ti, vc.p[1].nm, vc.p[1].tm};
+        out[4] = float4{vc.p[0].ni, vc.p[0].ti, vc.p[0].nm, vc.p[0].tm};
+        out[7] = float4{vc.p[1].ni, vc.p[1].ti, vc.p[1].nm, vc.p[1].tm};
         return mi;
     }
 };
 struct PositionSweep {
     static constexpr bool kMin = true;
+    static constexpr int kRec = prx::kPcStride;
+    static __device__ __forceinline__ const float4* rec(const DeviceState& d, int e) {
+        return d.s_pc + std::size_t(e) * prx::kPcStride;
+    }
     template <bool kLds>
-    static __device__ __forceinline__ float one(const DeviceState& d, const StepParams& c, const Bodies<kLds>& bs, int e) {
-        const Pc pc = load_pc(d.s_pc + std::size_t(e) * prx::kPcStride);
+    static __device__ __forceinline__ float one(const DeviceState&, const StepParams& c, const Bodies<kLds>& bs,
+                                                const float4 (&r)[kRec], int) {
+        const Pc pc = load_pc(r);
         float4 pa = bs.pos(pc.bA);
         float4 pb = bs.pos(pc.bB);
         const float sep = solve_pc(pc.m, pc.totalRadius, pc.A, pc.B, pa, pb, c);  // SolvePositionConstraintsViaGS
@@ -1120,6 +1158,12 @@ struct PositionSweep {
         return sep;
     }
 };
+template <class Sweep>
+__device__ __forceinline__ void sweep_load(const DeviceState& d, int e, float4 (&r)[Sweep::kRec]) {
+    const float4* src = Sweep::rec(d, e);
+#pragma unroll
+    for (int f = 0; f < Sweep::kRec; ++f) r[f] = src[f];
+}
 
 // Velocity iteration `it` stops the sweeps if an earlier iteration's largest
 // impulse change was at most regMinMomentum (the early exit of
@@ -1169,8 +1213,48 @@ __global__ __launch_bounds__(kGrid) void k_big_sweep(DeviceState d, BigState g, 
     float v = Sweep::kMin ? __builtin_inff() : 0.0f;
     const int e1 = g.colorStart[k + 1];
     for (int e = g.colorStart[k] + int(blockIdx.x * blockDim.x + threadIdx.x); e < e1; e += int(gridDim.x * blockDim.x))
-        v = sweep_more<Sweep>(v, Sweep::one(d, c, bs, e));
+    {
+        float4 rec[Sweep::kRec];
+        sweep_load<Sweep>(d, e, rec);
+        v = sweep_more<Sweep>(v, Sweep::one(d, c, bs, rec, e));
+    }
     sweep_report<Sweep>(g, it, v);
+}
+
+// A sweep by one workgroup over colours [k0, k1), a barrier between colours,
+// then the serial bucket in list order by one thread; returns the thread's
+// extreme.  start: the colours' first places and, at kBigMaxColors and after
+// it, the serial bucket's and the end.  A constraint always falls to the same
+// thread, which reads the next one's record (of this colour or the next)
+// while it solves the present one.
+template <class Sweep, bool kLds>
+__device__ __forceinline__ float sweep_colours(const DeviceState& d, const StepParams& c, const Bodies<kLds>& bs,
+                                               const int* start, int k0, int k1) {
+    float v = Sweep::kMin ? __builtin_inff() : 0.0f;
+    const int tid = int(threadIdx.x);
+    float4 cur[Sweep::kRec], next[Sweep::kRec];
+    if (k0 < k1 && start[k0] + tid < start[k0 + 1]) sweep_load<Sweep>(d, start[k0] + tid, cur);
+    for (int k = k0; k < k1; ++k) {
+        const int e1 = start[k + 1];
+        const int ahead = (k + 1 < k1 && e1 + tid < start[k + 2]) ? e1 + tid : -1;
+        int e = start[k] + tid;
+        if (e >= e1 && ahead >= 0) sweep_load<Sweep>(d, ahead, cur);
+        while (e < e1) {
+            const int after = e + kSmallBlock < e1 ? e + kSmallBlock : ahead;
+            if (after >= 0) sweep_load<Sweep>(d, after, next);
+            v = sweep_more<Sweep>(v, Sweep::one(d, c, bs, cur, e));
+#pragma unroll
+            for (int f = 0; f < Sweep::kRec; ++f) cur[f] = next[f];
+            e += kSmallBlock;
+        }
+        __syncthreads();
+    }
+    if (tid == 0)
+        for (int e = start[prx::kBigMaxColors]; e < start[prx::kBigMaxColors + 1]; ++e) {
+            sweep_load<Sweep>(d, e, cur);
+            v = sweep_more<Sweep>(v, Sweep::one(d, c, bs, cur, e));
+        }
+    return v;
 }
 
 // Iteration `it` over the other colours (one workgroup) and, in list order,
@@ -1179,18 +1263,11 @@ template <class Sweep>
 __global__ __launch_bounds__(kSmallBlock) void k_big_sweep_rest(DeviceState d, BigState g, StepParams c, int it) {
     if (!sweep_runs<Sweep>(g, c, it)) return;
     const Bodies<false> bs{d.s_bc_pos, d.s_bc_vel, d.hdr[0].nbodies};
-    float v = Sweep::kMin ? __builtin_inff() : 0.0f;
-    const int last = g.counters[prx::kBigColors];
-    for (int k = min(g.counters[prx::kBigTail], kGridColours); k < last; ++k) {
-        const int e1 = g.colorStart[k + 1];
-        for (int e = g.colorStart[k] + int(threadIdx.x); e < e1; e += kSmallBlock)
-            v = sweep_more<Sweep>(v, Sweep::one(d, c, bs, e));
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        for (int e = g.colorStart[prx::kBigMaxColors]; e < g.colorStart[prx::kBigMaxColors + 1]; ++e)
-            v = sweep_more<Sweep>(v, Sweep::one(d, c, bs, e));
-    sweep_report<Sweep>(g, it, v);
+    __shared__ int s_start[prx::kBigMaxColors + 2];
+    if (threadIdx.x < prx::kBigMaxColors + 2) s_start[threadIdx.x] = g.colorStart[threadIdx.x];
+    __syncthreads();
+    const int first = min(g.counters[prx::kBigTail], kGridColours);
+    sweep_report<Sweep>(g, it, sweep_colours<Sweep>(d, c, bs, s_start, first, g.counters[prx::kBigColors]));
 }
 
 // IntegratePositions (AabbTreeWorld.cpp:176-188).
@@ -1218,7 +1295,7 @@ __global__ __launch_bounds__(kGrid) void k_big_integrate(DeviceState d, StepPara
 // there is a workgroup barrier where the grid's form has a launch.  Same
 // colours, order and arithmetic as the grid's form.
 __global__ __launch_bounds__(kSmallBlock) void k_big_solve_small(DeviceState d, BigState g, StepParams c) {
-    __shared__ int s_cnt[kBuckets + 1];
+    __shared__ int s_cnt[kBuckets], s_start[prx::kBigMaxColors + 2];
     __shared__ int s_wave[kSmallBlock / kWave][kBuckets];
     __shared__ int s_left, s_ncol;
     __shared__ int s_ext;
@@ -1239,12 +1316,12 @@ __global__ __launch_bounds__(kSmallBlock) void k_big_solve_small(DeviceState d, 
         }
         if (round > 0)
             for (int e = tid; e < m; e += kSmallBlock)
-                if (g.color[e] < 0) col_propose(d, g, round, e);
+                if (g.color[e] < 0) col_propose<true>(d, g, round, e);
         __threadfence();
         __syncthreads();
         int left = 0, ncol = 0;
         for (int e = tid; e < m; e += kSmallBlock)
-            if (g.color[e] < 0 && !col_commit(d, g, round, e, ncol)) ++left;
+            if (g.color[e] < 0 && !col_commit<true>(d, g, round, e, ncol)) ++left;
         if (left) atomicAdd(&s_left, left);
         if (ncol) atomicMax(&s_ncol, ncol);
         __threadfence();
@@ -1256,22 +1333,19 @@ __global__ __launch_bounds__(kSmallBlock) void k_big_solve_small(DeviceState d, 
         if (rest == 0) break;
     }
     // Colour order.
-    if (tid <= kBuckets) s_cnt[tid] = 0;
+    if (tid < kBuckets) s_cnt[tid] = 0;
     __syncthreads();
-    for (int e = tid; e < m; e += kSmallBlock) {
-        if (g.color[e] < 0) g.color[e] = prx::kBigMaxColors;
-        atomicAdd(&s_cnt[g.color[e]], 1);
-    }
+    for (int e = tid; e < m; e += kSmallBlock) atomicAdd(&s_cnt[colour_bucket(d, g, e)], 1);
     __syncthreads();
     if (tid == 0) {
         int run = 0;
         for (int k = 0; k < kBuckets; ++k) {
             const int n = s_cnt[k];
             s_cnt[k] = run;
-            g.colorStart[k] = run;
+            if ((k & 1) == 0) s_start[k >> 1] = run;
             run += n;
         }
-        g.colorStart[kBuckets] = run;
+        s_start[prx::kBigMaxColors + 1] = run;
         g.counters[prx::kBigColors] = colors;
     }
     __syncthreads();
@@ -1280,14 +1354,8 @@ __global__ __launch_bounds__(kSmallBlock) void k_big_solve_small(DeviceState d, 
         __syncthreads();
         const int e = base + tid;
         const bool valid = e < m;
-        const int col = valid ? g.color[e] : 0;
-        unsigned long long peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 5; ++b) {
-            const bool bit = (col >> b) & 1;
-            const unsigned long long mm = __ballot(bit);
-            peers &= bit ? mm : ~mm;
-        }
+        const int col = valid ? colour_bucket(d, g, e) : 0;
+        const unsigned long long peers = bucket_peers(valid, col);
         const int rank = __popcll(peers & lanes_below(lane));
         if (valid && rank == 0) s_wave[wave][col] = __popcll(peers);
         __syncthreads();
@@ -1303,18 +1371,10 @@ __global__ __launch_bounds__(kSmallBlock) void k_big_solve_small(DeviceState d, 
             for (int w = 0; w < kSmallBlock / kWave; ++w) s_cnt[tid] += s_wave[w][tid];
         __syncthreads();
     }
-    // After the walk s_cnt[k] is colour k's end.  One sweep; returns its extreme.
+    // One sweep; returns its extreme.
     auto sweep = [&](auto kind) {
         using Sweep = decltype(kind);
-        float v = Sweep::kMin ? __builtin_inff() : 0.0f;
-        for (int k = 0; k < colors; ++k) {
-            const int e1 = s_cnt[k];
-            for (int e = (k ? s_cnt[k - 1] : 0) + tid; e < e1; e += kSmallBlock)
-                v = sweep_more<Sweep>(v, Sweep::one(d, c, bs, e));
-            __syncthreads();
-        }
-        if (tid == 0)
-            for (int e = s_cnt[kBuckets - 2]; e < s_cnt[kBuckets - 1]; ++e) v = sweep_more<Sweep>(v, Sweep::one(d, c, bs, e));
+        float v = sweep_colours<Sweep>(d, c, bs, s_start, 0, colors);
         for (int off = kWave / 2; off > 0; off >>= 1) v = sweep_more<Sweep>(v, __shfl_xor(v, off));
         if (tid == 0) s_ext = Sweep::kMin ? 0x7f800000 : 0;
         __syncthreads();
@@ -1601,7 +1661,7 @@ extern "C" hipError_t prx_big_launch_step(const prx::DeviceState* dp, const prx:
                 hipLaunchKernelGGL(k_col_commit, dim3(colBlocks), block, 0, s, d, g, r, r == kGridRounds - 1 ? 1 : 0);
             }
             hipLaunchKernelGGL(k_col_rest, dim3(1), dim3(kBlock), 0, s, d, g, kGridRounds);
-            hipLaunchKernelGGL(k_big_buckets, perContact, block, 0, s, g);
+            hipLaunchKernelGGL(k_big_buckets, perContact, block, 0, s, d, g);
             hipLaunchKernelGGL(k_big_records, perContact, block, 0, s, d, g, *c);
             if (c->warmStart) SweepLaunches<WarmSweep>(d, g, *c, 0, s);
             for (int it = 0; it < int(c->velIters); ++it) SweepLaunches<VelocitySweep>(d, g, *c, it, s);

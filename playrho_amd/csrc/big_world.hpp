@@ -60,7 +60,7 @@ struct BigState {
     unsigned long long* fresh;   // pairCap: new pairs
     int* find;                   // kFindSlots * kFindWords
     // Per workgroup range of 256 contacts: kept or touching contacts, and
-    // touching contacts per colour.
+    // touching contacts per bucket of the colour order (2 kBigMaxColors + 1).
     int* blockSum;
     int* blockHist;
     // Colouring and solve order.

@@ -3205,7 +3205,7 @@ int AllocBig(DeviceArena& a, prx::BigState& g, int P, int B, int cap) {
     PRX_HIP(a.alloc(g.fresh, std::size_t(g.pairCap)));
     PRX_HIP(a.alloc(g.find, std::size_t(prx::kFindSlots * prx::kFindWords)));
     PRX_HIP(a.alloc(g.blockSum, blocks));
-    PRX_HIP(a.alloc(g.blockHist, blocks * (prx::kBigMaxColors + 1)));
+    PRX_HIP(a.alloc(g.blockHist, blocks * (2 * prx::kBigMaxColors + 1)));
     PRX_HIP(a.alloc(g.list, std::size_t(g.cap)));
     PRX_HIP(a.alloc(g.list2, std::size_t(g.cap)));
     PRX_HIP(a.alloc(g.color, std::size_t(g.cap)));
