@@ -569,8 +569,8 @@ class World:
 
     def bodies(self):
         n = self.body_count
-        out = np.zeros((n, 10), dtype=np.float32)
-        flags = np.zeros(n, dtype=np.uint32)
+        out = np.empty((n, 10), dtype=np.float32)
+        flags = np.empty(n, dtype=np.uint32)
         _check(lib().prx_world_get_bodies(self.h, out.ctypes.data, flags.ctypes.data))
         return out, flags
 

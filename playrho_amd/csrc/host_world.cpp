@@ -40,6 +40,9 @@ extern "C" int prx_lbvh_pairs_noalloc_impl(const float* aabbs, const std::int32_
                                            int n, std::int32_t* pairs, int cap, int* count, void* stream,
                                            const char** err);
 extern "C" hipError_t prx_big_launch_metrics(const prx::DeviceState* d, const prx::BigState* g, hipStream_t s);
+extern "C" hipError_t prx_launch_body_view(const prx::DeviceState* d, float* rows, std::uint32_t* flags, int n,
+                                           hipStream_t stream);
+extern "C" hipError_t prx_launch_report(const prx::DeviceState* d, std::uint32_t* out, hipStream_t stream);
 extern "C" hipError_t prx_launch_step_tape(const prx::DeviceState* d, const prx::StepParams* c, int count,
                                            hipStream_t stream);
 extern "C" hipError_t prx_launch_adjoint_step(const prx::DeviceState* d, const prx::Tape* t, const prx::AdjState* a,
@@ -404,7 +407,16 @@ struct prx_batch {
     int lds_bytes = 16 * 1024;
     int lds_min = 16 * 1024;
     std::vector<void*> snapshot;  // state before a recorded step (listener record growth)
+    // Written by kernels into pinned memory (each followed by a stream
+    // synchronisation before it is read): the body rows of
+    // prx_world_get_bodies for every world, then their flags; and the worlds'
+    // status bits combined, then the first world's header.
+    float* view = nullptr;
+    bool view_valid = false;  // view holds the present device state
+    std::uint32_t* report = nullptr;
     ~prx_batch() {
+        if (view) (void)hipHostFree(view);
+        if (report) (void)hipHostFree(report);
         if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
         if (graph) (void)hipGraphDestroy(graph);
         if (ev0) (void)hipEventDestroy(ev0);
@@ -434,6 +446,43 @@ int DownloadBatch(prx_batch* b);
 // Brings a world's host mirror up to date (device -> host).
 int Refresh(prx_world* w) {
     if (w->owner && w->host_stale) return DownloadBatch(w->owner);
+    return PRX_OK;
+}
+
+// The body rows of a batch's worlds from the device, in pinned memory.  A
+// caller that reads the bodies after stepping needs 44 bytes a body; the
+// whole state is some 1,200 (most of it contact slots), and copying it, into
+// fresh pageable arrays, cost 128 ms for 4096 pile worlds.
+constexpr std::size_t kViewFloats = 10;
+int LaunchView(prx_batch* b) {
+    if (!b->view) {
+        void* p = nullptr;
+        PRX_HIP(hipHostMalloc(&p, std::max<std::size_t>(b->totB, 1) * (kViewFloats + 1) * sizeof(float), 0));
+        b->view = static_cast<float*>(p);
+    }
+    PRX_HIP(prx_launch_body_view(&b->d, b->view, reinterpret_cast<std::uint32_t*>(b->view + kViewFloats * b->totB),
+                                 int(b->totB), b->stream));
+    return PRX_OK;
+}
+
+// The world's body rows and flags when the device holds its newer state
+// (null rows: the host mirror is up to date).
+struct BodyView {
+    const float* rows = nullptr;
+    const std::uint32_t* flags = nullptr;
+};
+int ViewBodies(prx_world* w, BodyView& out) {
+    out = BodyView{};
+    prx_batch* b = w->owner;
+    if (!b || !w->host_stale) return PRX_OK;
+    if (!b->view_valid) {
+        if (int st = LaunchView(b)) return st;
+        PRX_HIP(hipStreamSynchronize(b->stream));
+        b->view_valid = true;
+    }
+    const std::size_t off = std::size_t(b->hdr[std::size_t(w->index_in_owner)].body_off);
+    out.rows = b->view + kViewFloats * off;
+    out.flags = reinterpret_cast<const std::uint32_t*>(b->view + kViewFloats * b->totB) + off;
     return PRX_OK;
 }
 
@@ -1584,12 +1633,27 @@ int CreateBatch(prx_world* const* worlds, int n, const prx_batch_conf* conf, prx
     return PRX_OK;
 }
 
-int CheckStatus(prx_batch* b) {
+// Waits for the batch's stream and checks the worlds' status words, which a
+// kernel combines into the report (the headers are read only where one is
+// set); the report's header copy is the first world's.  withView: the body
+// rows come along.
+int CheckStatus(prx_batch* b, bool withView = false) {
     // Status words are checked after each synchronising call.  A lost
     // listener call or a TOI phase cut short affects the steps since the last
     // check only: those bits are reported once, then cleared, so the worlds
     // step on.  Contact and scratch overflows leave a world's contact set
     // incomplete and stay set.
+    if (!b->report) {
+        void* p = nullptr;
+        PRX_HIP(hipHostMalloc(&p, sizeof(std::uint32_t) + sizeof(prx::WorldHeader), 0));
+        b->report = static_cast<std::uint32_t*>(p);
+    }
+    PRX_HIP(prx_launch_report(&b->d, b->report, b->stream));
+    if (withView)
+        if (int st = LaunchView(b)) return st;
+    PRX_HIP(hipStreamSynchronize(b->stream));
+    if (withView) b->view_valid = true;
+    if (*b->report == 0u) return PRX_OK;
     std::vector<prx::WorldHeader> hdr(b->worlds.size());
     PRX_HIP(hipMemcpy(hdr.data(), b->d.hdr, hdr.size() * sizeof(prx::WorldHeader), hipMemcpyDeviceToHost));
     constexpr std::uint32_t kRecoverable = prx::kStatusEventOverflow | prx::kStatusToiLimit;
@@ -1650,6 +1714,7 @@ int StepBatch(prx_batch* b, const prx_step_conf* conf, int nsteps) {
     b->last_launches = nsteps;
     for (prx_world* w : b->worlds)
         if (w) w->host_stale = true;
+    b->view_valid = false;
     return PRX_OK;
 }
 
@@ -1736,10 +1801,12 @@ std::vector<std::pair<void*, std::size_t>> DynamicArrays(prx_batch* b);
 // it, with that world's record grown to what the step needed; the calls
 // delivered are then the complete list.
 int StepRecorded(prx_batch* b, const prx_step_conf* conf) {
+    // A world stepped by itself is usually read after each step: up to this
+    // many bodies the rows are written along with the step's report (2 us).
+    constexpr std::size_t kEagerViewBodies = 4096;
     if (b->totE == 0) {
         if (int st = StepBatch(b, conf, 1)) return st;
-        PRX_HIP(hipStreamSynchronize(b->stream));
-        return CheckStatus(b);
+        return CheckStatus(b, b->totB <= kEagerViewBodies);
     }
     std::vector<std::pair<void*, std::size_t>> arrays = DynamicArrays(b);
     arrays.pop_back();  // the previous step's calls (the last entry) need no copy
@@ -2441,7 +2508,7 @@ int prx_step(prx_world* w, const prx_step_conf* conf, prx_step_stats* stats) {
     if (int st = DeliverEvents(w->solo)) return st;
     if (stats) {
         prx::WorldHeader h;
-        PRX_HIP(hipMemcpy(&h, w->solo->d.hdr, sizeof(h), hipMemcpyDeviceToHost));
+        std::memcpy(&h, w->solo->report + 1, sizeof(h));  // of the check that ended the step
         *stats = StatsOf(h);
     }
     return PRX_OK;
@@ -2449,7 +2516,14 @@ int prx_step(prx_world* w, const prx_step_conf* conf, prx_step_stats* stats) {
 
 int prx_world_get_bodies(prx_world* w, float* out, std::uint32_t* flags) {
     if (int st = CheckWorld(w)) return st;
-    if (int st = Refresh(w)) return st;
+    BodyView view;
+    if (int st = ViewBodies(w, view)) return st;
+    if (view.rows) {
+        const std::size_t n = w->bodies.size();
+        if (out) std::memcpy(out, view.rows, n * kViewFloats * sizeof(float));
+        if (flags) std::memcpy(flags, view.flags, n * sizeof(std::uint32_t));
+        return PRX_OK;
+    }
     for (std::size_t i = 0; i < w->bodies.size(); ++i) {
         const HostBody& b = w->bodies[i];
         if (out) {
@@ -2473,10 +2547,12 @@ int prx_world_get_bodies(prx_world* w, float* out, std::uint32_t* flags) {
 int prx_world_get_transformation(prx_world* w, std::uint32_t body, float out[4]) {
     if (int st = CheckWorld(w)) return st;
     if (int st = CheckBody(w, body)) return st;
-    if (int st = Refresh(w)) return st;
+    BodyView view;
+    if (int st = ViewBodies(w, view)) return st;
     const HostBody& b = w->bodies[body];
-    const V2 q = UnitFromAngle(b.pos1[2]);
-    const V2 p = V2{b.pos1[0], b.pos1[1]} - Rotate(b.lc, q);
+    const float* pos1 = view.rows ? view.rows + kViewFloats * body + 3 : b.pos1;
+    const V2 q = UnitFromAngle(pos1[2]);
+    const V2 p = V2{pos1[0], pos1[1]} - Rotate(b.lc, q);
     out[0] = p.x;
     out[1] = p.y;
     out[2] = q.x;
@@ -3011,7 +3087,6 @@ int prx_batch_step(prx_batch* b, const prx_step_conf* conf, int nsteps) {
 
 int prx_batch_sync(prx_batch* b) {
     if (!b) return Fail(PRX_E_INVALID_ARGUMENT, "null batch");
-    PRX_HIP(hipStreamSynchronize(b->stream));
     return CheckStatus(b);
 }
 
@@ -3315,12 +3390,12 @@ int prx_big_step(prx_big* big, const prx_step_conf* conf, int nsteps) {
     PRX_HIP(hipEventRecord(b->ev1, b->stream));
     b->last_launches = nsteps;
     big->world->host_stale = true;
+    b->view_valid = false;
     return PRX_OK;
 }
 
 int prx_big_sync(prx_big* big) {
     if (!big) return Fail(PRX_E_INVALID_ARGUMENT, "null argument");
-    PRX_HIP(hipStreamSynchronize(big->batch->stream));
     return CheckStatus(big->batch);
 }
 
@@ -3473,7 +3548,7 @@ int AdjointForward(prx_adjoint* adj, const prx::StepParams& p) {
         const hipError_t le = prx_launch_step(&b->d, &p, 0, nw, st);
         if (le != hipSuccess) return Fail(PRX_E_DEVICE, std::string("launch: ") + hipGetErrorString(le));
     }
-    PRX_HIP(hipStreamSynchronize(st));
+    b->view_valid = false;
     if (int e = CheckStatus(b)) return e;
     adj->forwarded = true;
     return PRX_OK;
@@ -3539,6 +3614,7 @@ int AdjointBackward(prx_adjoint* adj, const prx::StepParams& p, const std::vecto
     if (int e = AdjointCopy(adj, 0, false)) return e;
     PRX_HIP(hipStreamSynchronize(st));
     for (prx_world* w : b->worlds) w->host_stale = true;
+    b->view_valid = false;
     if (status) return Fail(PRX_E_UNSUPPORTED, "a contact the adjoint does not model (two-point manifold or face B)");
     return PRX_OK;
 }

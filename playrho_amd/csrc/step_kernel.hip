@@ -66,6 +66,54 @@ extern "C" hipError_t prx_launch_step_tape(const prx::DeviceState* d, const prx:
     return hipGetLastError();
 }
 
+namespace prxd {
+
+// Body rows of prx_world_get_bodies (both sweep positions, velocity,
+// under-active time) and flags, written straight into pinned host memory.  A
+// thread per row word keeps the stores coalesced (the link is the bound: 22 MB
+// for 500,000 bodies); the loads hit a line each of ten threads shares.
+__global__ __launch_bounds__(256) void k_body_view(DeviceState d, float* rows, std::uint32_t* flags, int n) {
+    for (int i = int(blockIdx.x * blockDim.x + threadIdx.x); i < 11 * n; i += int(gridDim.x * blockDim.x)) {
+        if (i >= 10 * n) {
+            flags[i - 10 * n] = d.bflags[i - 10 * n] & 0x7fu;
+            continue;
+        }
+        const int b = i / 10, f = i - 10 * b;
+        const float4* src = f < 3 ? d.pos0 : (f < 6 ? d.pos1 : d.vel);
+        rows[i] = reinterpret_cast<const float*>(src + b)[f < 6 ? f % 3 : f - 6];
+    }
+}
+
+// The worlds' status bits combined and the first world's header, into pinned
+// host memory (one workgroup).
+__global__ __launch_bounds__(1024) void k_report(DeviceState d, std::uint32_t* out) {
+    __shared__ std::uint32_t s_or;
+    if (threadIdx.x == 0) s_or = 0u;
+    __syncthreads();
+    std::uint32_t v = 0u;
+    for (int w = int(threadIdx.x); w < d.nworlds; w += int(blockDim.x)) v |= std::uint32_t(d.hdr[w].status);
+    if (v) atomicOr(&s_or, v);
+    __syncthreads();
+    if (threadIdx.x == 0) out[0] = s_or;
+    constexpr unsigned kWords = sizeof(prx::WorldHeader) / 4;
+    if (threadIdx.x < kWords) out[1 + threadIdx.x] = reinterpret_cast<const std::uint32_t*>(d.hdr)[threadIdx.x];
+}
+
+}  // namespace prxd
+
+extern "C" hipError_t prx_launch_body_view(const prx::DeviceState* d, float* rows, std::uint32_t* flags, int n,
+                                           hipStream_t stream) {
+    if (n <= 0) return hipSuccess;
+    const unsigned blocks = unsigned((std::size_t(n) * 11 + 255) / 256);
+    hipLaunchKernelGGL(prxd::k_body_view, dim3(blocks < 4096u ? blocks : 4096u), dim3(256), 0, stream, *d, rows, flags, n);
+    return hipGetLastError();
+}
+
+extern "C" hipError_t prx_launch_report(const prx::DeviceState* d, std::uint32_t* out, hipStream_t stream) {
+    hipLaunchKernelGGL(prxd::k_report, dim3(1), dim3(d->nworlds < 256 ? 256u : 1024u), 0, stream, *d, out);
+    return hipGetLastError();
+}
+
 // Diagnostic: evaluates the device sine/cosine (UnitVec::Get) on n angles.
 namespace prxd {
 __global__ void k_sincos(const float* in, float* out, int n) {
