@@ -41,6 +41,127 @@ __device__ __forceinline__ void add_body(float4* p, V2 v, float w) {
     *p = a;
 }
 
+// ---------------------------------------------------------------------------
+// Reverse rounds.  A step's solver updates are reversed in the opposite of
+// their recorded order, but only updates that share a moving body depend on
+// one another.  An update's level is one more than the last level that touched
+// either of its bodies (bodies with zero inverse mass and inertia order
+// nothing); the updates of a level touch distinct moving bodies, so they are
+// reversed together, levels from the last to the first, and every sum is
+// formed in the order the serial walk forms it.  The plan covers all of a
+// world's islands at once; an update takes part in the iterations its island
+// ran.
+
+// Levels of items 0..n-1 in recorded order (bodies(k): the moving bodies of
+// item k, -1 for none), then rounds of at most `width` items of one level:
+// round r is order[start[r]..start[r + 1]).  last: a table of nb ints; lvl: n
+// ints of scratch.  Run by one wavefront.  period: the most rounds that any
+// body's items span; iterations started that many rounds apart still reach
+// every body in order, so they can be reversed side by side.
+struct RoundPlan {
+    int rounds, period;
+};
+template <class F>
+__device__ __forceinline__ RoundPlan plan_rounds(int n, int nb, int width, int lane, F bodies, int* last, int* lvl, int* order,
+                                           int* start) {
+    auto fence = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); };
+    for (int b = lane; b < nb; b += kWave) last[b] = 0;
+    fence();
+    int levels = 0;
+    for (int base = 0; base < n; base += kWave) {
+        int2 ab{-1, -1};
+        if (base + lane < n) ab = bodies(base + lane);
+        const int cnt = (n - base < kWave) ? n - base : kWave;
+        int mine = 0;
+        for (int j = 0; j < cnt; ++j) {
+            const int aj = __builtin_amdgcn_readlane(ab.x, j), bj = __builtin_amdgcn_readlane(ab.y, j);
+            const int la = (aj >= 0) ? last[aj] : 0, lb = (bj >= 0) ? last[bj] : 0;
+            const int l = ((la > lb) ? la : lb) + 1;
+            if (lane == 0) {
+                if (aj >= 0) last[aj] = l;
+                if (bj >= 0) last[bj] = l;
+            }
+            fence();
+            if (lane == j) mine = l - 1;
+            levels = (l > levels) ? l : levels;
+        }
+        if (base + lane < n) lvl[base + lane] = mine;
+    }
+    fence();
+    // Items by level, then by recorded order: one level after another.  The
+    // round of an item replaces its level.
+    int rounds = 0, at = 0;
+    if (lane == 0) start[0] = 0;
+    for (int l = 0; l < levels; ++l) {
+        const int first = at;
+        for (int base = 0; base < n; base += kWave) {
+            const bool in = base + lane < n && lvl[base + lane] == l;
+            const unsigned long long m = __ballot(in);
+            if (in) {
+                const int pos = at + __popcll(m & lanes_below(lane));
+                order[pos] = base + lane;
+                lvl[base + lane] = -1 - (rounds + (pos - first) / width);
+            }
+            at += __popcll(m);
+        }
+        for (int k = first; k < at; k += width) {
+            ++rounds;
+            if (lane == 0) start[rounds] = (k + width < at) ? k + width : at;
+        }
+    }
+    fence();
+    for (int b = lane; b < nb; b += kWave) last[b] = rounds;
+    fence();
+    for (int k = lane; k < n; k += kWave) {
+        const int2 ab = bodies(k);
+        if (ab.x >= 0) atomicMin(&last[ab.x], -1 - lvl[k]);
+        if (ab.y >= 0) atomicMin(&last[ab.y], -1 - lvl[k]);
+    }
+    fence();
+    int period = 1;
+    for (int k = lane; k < n; k += kWave) {
+        const int2 ab = bodies(k);
+        const int r = -1 - lvl[k];
+        if (ab.x >= 0) period = max(period, r - last[ab.x] + 1);
+        if (ab.y >= 0) period = max(period, r - last[ab.y] + 1);
+    }
+    for (int o = 32; o > 0; o >>= 1) period = max(period, __shfl_xor(period, o));
+    fence();
+    return RoundPlan{rounds, __builtin_amdgcn_readfirstlane(period)};
+}
+
+// Iterations of the slots' islands, velocity | position << 16.
+__device__ __forceinline__ void slot_iterations(const int4* isl, int nisl, int tid, int threads, int* iters) {
+    for (int is = tid; is < nisl; is += threads) {
+        const int4 rng = isl[is];
+        for (int e = rng.x; e < rng.y; ++e) iters[e] = rng.z | (rng.w << 16);
+    }
+}
+__device__ __forceinline__ int max_iterations(const int4* isl, int nisl, int lane, bool position) {
+    int m = 0;
+    for (int is = lane; is < nisl; is += kWave) m = max(m, position ? isl[is].w : isl[is].z);
+    for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
+    return __builtin_amdgcn_readfirstlane(m);
+}
+
+// Ints of plan scratch per contact slot or joint of a world (AdjState::plan).
+static_assert(prx::kAdjPlanInts >= 8, "two plans of levels, order and starts, and the iterations");
+
+// Adds a wavefront's counts to the run's counters: one atomic for each, not
+// one for each update (half a million additions to one address a launch took
+// most of its time).
+__device__ __forceinline__ void add_diag(float* diag, int k, int v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if ((threadIdx.x & (kWave - 1)) == 0 && v) atomicAdd(diag + k, float(v));
+}
+
+// One wavefront per world, one lane per update of a round.  kLds: the body
+// adjoints and the round plan in LDS (36 bytes a body and 12 a contact slot),
+// else in global memory.  A round's tape records are read while the round
+// before is reversed.  Bound by the latency of one round after another.  1024
+// billiards worlds of 64 disks: 0.85 -> 0.21 ms a step against one lane per
+// island, the adjoints in global memory and an atomic for each update counted.
+template <bool kLds>
 __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjState a, StepParams c) {
     const int w = int(blockIdx.x);
     const int lane = int(threadIdx.x);
@@ -48,113 +169,180 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
     const int bo = H.body_off, co = H.contact_off, nb = H.nbodies, cap = H.contact_cap;
     const int nisl = t.nisl[w];
     const int4* isl = t.isl + bo + w;
-    const int nslots = nisl > 0 ? isl[nisl - 1].y : 0;
+    const int n = nisl > 0 ? isl[nisl - 1].y : 0;
+    float4* const X = kLds ? g_smem : a.xbar + bo;
+    float4* const V = kLds ? g_smem + nb : a.vbar + bo;
+    int* const plan = a.plan + std::size_t(co + H.joint_off) * prx::kAdjPlanInts;
+    int* const last = kLds ? reinterpret_cast<int*>(g_smem + 2 * nb) : d.s_stack + 2 * bo;
+    int* const order = kLds ? reinterpret_cast<int*>(g_smem + 2 * nb) + nb : plan;
+    int* const start = kLds ? order + cap : plan + cap;
+    int* const iters = kLds ? start + cap + 1 : plan + 2 * cap + 1;
+    int* const lvl = plan + 4 * cap;
+    auto vcrec = [&](int e) { return t.vc + (std::size_t(co) + std::size_t(e)) * prx::kTapeVc; };
+    if constexpr (kLds) {
+        for (int b = lane; b < nb; b += kWave) {
+            X[b] = a.xbar[bo + b];
+            V[b] = a.vbar[bo + b];
+        }
+    }
     // Impulse adjoints carried in from the next step, by contact id: the
     // step's final impulses warm-started the next step where the manifold
     // update after the solve carried them (by ContactFeature, else from the
     // nearest point; the tape's carry map says which).  The next step wrote
     // nothing for contacts it did not solve or that started afresh.
-    for (int e = lane; e < nslots; e += kWave) {
-        const float4* vc = t.vc + (std::size_t(co) + e) * prx::kTapeVc;
+    int unmodelled = 0;
+    for (int e = lane; e < n; e += kWave) {
+        const float4* vc = vcrec(e);
         const std::uint32_t id = __float_as_uint(vc[10].y);
         const float4 lb = a.lambar[co + int(id)];
         const std::uint32_t cm = t.cmap[co + int(id)];
         const bool carried = ((cm >> 8) & 0xfu) >= 1u && (cm & 0xfu) == 0u;
         a.lamtmp[co + e] = carried ? float2{lb.x, lb.y} : float2{0.0f, 0.0f};
+        float4* cb = a.cbar + (std::size_t(co) + e) * 3;
+        cb[0] = float4{0, 0, 0, 0};
+        cb[1] = float4{0, 0, 0, 0};
+        cb[2] = float4{0, 0, 0, 0};
     }
     __syncthreads();
     for (int i = lane; i < cap; i += kWave) a.lambar[co + i] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+    slot_iterations(isl, nisl, lane, kWave, iters);
+    const RoundPlan rp = plan_rounds(n, nb, kWave, lane, [&](int e) {
+        const float4* vc = vcrec(e);
+        const float4 ms = vc[8];
+        return int2{(ms.x != 0.0f || ms.y != 0.0f) ? __float_as_int(vc[2].w) : -1,
+                    (ms.z != 0.0f || ms.w != 0.0f) ? __float_as_int(vc[5].z) : -1};
+    }, last, lvl, order, start);
+    const int rounds = rp.rounds;
     __syncthreads();
+    // Slot of the lane in round r of iteration `it` (-1: past the first pass),
+    // -1 for none.
+    auto slot_at = [&](int it, int r, bool position) {
+        if (it < 0) return -1;
+        const int pos = start[r] + lane;
+        if (pos >= start[r + 1]) return -1;
+        const int e = order[pos];
+        return it < (position ? iters[e] >> 16 : iters[e] & 0xffff) ? e : -1;
+    };
 
-    // Position solver, reversed (per island, iterations and slots in reverse).
-    for (int is = lane; is < nisl; is += kWave) {
-        const int4 rng = isl[is];
-        for (int it = rng.w - 1; it >= 0; --it) {
-            for (int e = rng.y - 1; e >= rng.x; --e) {
-                const std::size_t slot = std::size_t(co) + e;
-                const float4* vc = t.vc + slot * prx::kTapeVc;
-                const std::uint32_t type = __float_as_uint(vc[10].z) & 0xffu;
-                const std::uint32_t npts = __float_as_uint(vc[10].z) >> 8;
-                if (npts != 1u || (type != 1u && type != 2u)) {
-                    *a.status = 1;
-                    continue;
-                }
-                const int bA = __float_as_int(vc[2].w), bB = __float_as_int(vc[5].z);
-                const float4 ms = vc[8];
-                const float4* g = t.ngs + (slot * std::size_t(t.itP) + it) * 2;
+    // Position solver, reversed.
+    int posUpdates = 0;
+    {
+        struct Rec {
+            float4 v0, v2, v5, v8, v9, v10, g0, g1;
+        };
+        auto fetch = [&](int e, int it, Rec& r) {
+            if (e < 0) return;
+            const float4* vc = vcrec(e);
+            const float4* g = t.ngs + ((std::size_t(co) + e) * std::size_t(t.itP) + it) * 2;
+            r = Rec{vc[0], vc[2], vc[5], vc[8], vc[9], vc[10], g[0], g[1]};
+        };
+        int it = rounds > 0 ? max_iterations(isl, nisl, lane, true) - 1 : -1, r = rounds - 1;
+        Rec cur{}, next{};
+        int e = slot_at(it, r, true);
+        fetch(e, it, cur);
+        while (it >= 0) {
+            // The round before: the last one of the iteration before.
+            if (--r < 0) {
+                r = rounds - 1;
+                --it;
+            }
+            const int en = slot_at(it, r, true);
+            fetch(en, it, next);
+            if (e >= 0) {
+                const std::uint32_t type = __float_as_uint(cur.v10.z) & 0xffu;
+                const std::uint32_t npts = __float_as_uint(cur.v10.z) >> 8;
+                const int bA = __float_as_int(cur.v2.w), bB = __float_as_int(cur.v5.z);
+                const float4 ms = cur.v8;
                 // Circle centres: a dynamic disk's is its position (disks at
                 // the body origin); a static body's point does not move.
                 const bool dynA = ms.x != 0.0f || ms.y != 0.0f;
-                const V2 pA = dynA ? v2(g[0]) : V2{vc[9].x, vc[9].y};
-                const V2 pB = v2(g[1]);
-                float4* xa = a.xbar + bo + bA;
-                float4* xb = a.xbar + bo + bB;
-                const V2 xbA = v2(*xa), xbB = v2(*xb);
-                atomicAdd(a.diag + 2, 1.0f);
-                const float s = g[0].w;  // separation the forward update used
-                const float inner = c.regResolutionRate * (s + c.linearSlop);
-                const float Cc = -clamp_std(inner, -c.maxLinearCorrection, 0.0f);
-                const bool active = !(inner < -c.maxLinearCorrection) && !(0.0f < inner);
+                const V2 pA = dynA ? v2(cur.g0) : V2{cur.v9.x, cur.v9.y};
+                const V2 pB = v2(cur.g1);
                 const float K = ms.x + ms.z;
-                if (!(K > 0.0f)) continue;
-                const V2 gP = mul(ms.z, xbB) - mul(ms.x, xbA);
-                if (type == 1u) {
-                    const V2 dd = pB - pA;
-                    const float L = __builtin_sqrtf(magsq(dd));
-                    if (!(L > 0.0f)) continue;
-                    const V2 n{dd.x / L, dd.y / L};
-                    const float Cbar = dot(gP, n) / K;
-                    const V2 nbar = mul(gP, Cc / K);
-                    const float sbar = active ? -c.regResolutionRate * Cbar : 0.0f;
-                    const float nn = dot(n, nbar);
-                    const V2 dbar = mul(nbar - mul(n, nn), 1.0f / L) + mul(n, sbar);
-                    if (ms.x != 0.0f || ms.y != 0.0f) add_body(xa, -dbar, 0.0f);
-                    add_body(xb, dbar, 0.0f);
-                } else {
-                    // Face A: A is the polygon (static: its plane and normal
-                    // are fixed), B the disk whose centre is the clip point.
-                    const V2 n = v2(vc[0]);
-                    const float Cbar = dot(gP, n) / K;
-                    const float sbar = active ? -c.regResolutionRate * Cbar : 0.0f;
-                    add_body(xb, mul(n, sbar), 0.0f);
+                if (npts != 1u || (type != 1u && type != 2u)) unmodelled = 1;
+                else ++posUpdates;
+                if (npts == 1u && (type == 1u || type == 2u) && K > 0.0f) {
+                    const V2 xbA = dynA ? v2(X[bA]) : V2{0.0f, 0.0f}, xbB = v2(X[bB]);
+                    const float s = cur.g0.w;  // separation the forward update used
+                    const float inner = c.regResolutionRate * (s + c.linearSlop);
+                    const float Cc = -clamp_std(inner, -c.maxLinearCorrection, 0.0f);
+                    const bool active = !(inner < -c.maxLinearCorrection) && !(0.0f < inner);
+                    const V2 gP = mul(ms.z, xbB) - mul(ms.x, xbA);
+                    if (type == 1u) {
+                        const V2 dd = pB - pA;
+                        const float L = __builtin_sqrtf(magsq(dd));
+                        if (L > 0.0f) {
+                            const V2 nn2{dd.x / L, dd.y / L};
+                            const float Cbar = dot(gP, nn2) / K;
+                            const V2 nbar = mul(gP, Cc / K);
+                            const float sbar = active ? -c.regResolutionRate * Cbar : 0.0f;
+                            const float nn = dot(nn2, nbar);
+                            const V2 dbar = mul(nbar - mul(nn2, nn), 1.0f / L) + mul(nn2, sbar);
+                            if (dynA) add_body(X + bA, -dbar, 0.0f);
+                            if (ms.z != 0.0f || ms.w != 0.0f) add_body(X + bB, dbar, 0.0f);
+                        }
+                    } else {
+                        // Face A: A is the polygon (static: its plane and normal
+                        // are fixed), B the disk whose centre is the clip point.
+                        const V2 nrm = v2(cur.v0);
+                        const float Cbar = dot(gP, nrm) / K;
+                        const float sbar = active ? -c.regResolutionRate * Cbar : 0.0f;
+                        if (ms.z != 0.0f || ms.w != 0.0f) add_body(X + bB, mul(nrm, sbar), 0.0f);
+                    }
                 }
             }
+            __syncthreads();
+            cur = next;
+            e = en;
         }
     }
-    __syncthreads();
     // Position integration, reversed: x1 = x0 + h v.
     for (int b = lane; b < nb; b += kWave) {
         if (!t.inisl[bo + b]) continue;
-        const float4 xb = a.xbar[bo + b];
-        add_body(a.vbar + bo + b, V2{c.dt * xb.x, c.dt * xb.y}, c.dt * xb.z);
+        const float4 xb = X[b];
+        add_body(V + b, V2{c.dt * xb.x, c.dt * xb.y}, c.dt * xb.z);
     }
     __syncthreads();
-    // Gauss-Seidel sweeps, warm start and constraint creation, reversed.
-    for (int is = lane; is < nisl; is += kWave) {
-        const int4 rng = isl[is];
-        for (int e = rng.x; e < rng.y; ++e) {
-            float4* cb = a.cbar + (std::size_t(co) + e) * 3;
-            cb[0] = float4{0, 0, 0, 0};
-            cb[1] = float4{0, 0, 0, 0};
-            cb[2] = float4{0, 0, 0, 0};
-        }
-        for (int it = rng.z - 1; it >= 0; --it) {
-            for (int e = rng.y - 1; e >= rng.x; --e) {
+    // Gauss-Seidel sweeps, reversed.
+    int velUpdates = 0;
+    {
+        struct Rec {
+            float4 v0, v2, v3, v4, v5, v8, v10, g0, g1;
+        };
+        auto fetch = [&](int e, int it, Rec& r) {
+            if (e < 0) return;
+            const float4* vc = vcrec(e);
+            const float4* g = t.gs + ((std::size_t(co) + e) * std::size_t(t.itV) + it) * 3;
+            r = Rec{vc[0], vc[2], vc[3], vc[4], vc[5], vc[8], vc[10], g[0], g[1]};
+        };
+        int it = rounds > 0 ? max_iterations(isl, nisl, lane, false) - 1 : -1, r = rounds - 1;
+        Rec cur{}, next{};
+        int e = slot_at(it, r, false);
+        fetch(e, it, cur);
+        while (it >= 0) {
+            // The round before: the last one of the iteration before.
+            if (--r < 0) {
+                r = rounds - 1;
+                --it;
+            }
+            const int en = slot_at(it, r, false);
+            fetch(en, it, next);
+            if (e >= 0 && (__float_as_uint(cur.v10.z) >> 8) == 1u) {
+                ++velUpdates;
                 const std::size_t slot = std::size_t(co) + e;
-                const float4* vc = t.vc + slot * prx::kTapeVc;
-                if ((__float_as_uint(vc[10].z) >> 8) != 1u) continue;
-                const V2 n = v2(vc[0]);
-                const V2 tg = fwdperp(n);
-                const float f = vc[0].z, ts = vc[0].w;
-                const V2 rA{vc[3].x, vc[3].y}, rB{vc[3].z, vc[3].w};
-                const float nm = vc[4].z, tm = vc[4].w, bias = vc[5].x;
-                const float4 ms = vc[8];
-                const float mA = ms.x, iA = ms.y, mB = ms.z, iB = ms.w;
-                const int bA = __float_as_int(vc[2].w), bB = __float_as_int(vc[5].z);
-                const float4* g = t.gs + (slot * std::size_t(t.itV) + it) * 3;
-                const V2 vA{g[0].x, g[0].y}, vB{g[1].x, g[1].y};
-                const float wA = g[0].z, wB = g[1].z, ltOld = g[0].w, lnOld = g[1].w;
-                atomicAdd(a.diag + 3, 1.0f);
+                // Sums over the iterations (read late, off the chain through the bodies).
+                const float2 lb0 = a.lamtmp[slot];  // (normal, tangent)
+                const float4 c0 = a.cbar[slot * 3 + 0], c1 = a.cbar[slot * 3 + 1], c2 = a.cbar[slot * 3 + 2];
+                const V2 nrm = v2(cur.v0);
+                const V2 tg = fwdperp(nrm);
+                const float f = cur.v0.z, ts = cur.v0.w;
+                const V2 rA{cur.v3.x, cur.v3.y}, rB{cur.v3.z, cur.v3.w};
+                const float nm = cur.v4.z, tm = cur.v4.w, bias = cur.v5.x;
+                const float mA = cur.v8.x, iA = cur.v8.y, mB = cur.v8.z, iB = cur.v8.w;
+                const int bA = __float_as_int(cur.v2.w), bB = __float_as_int(cur.v5.z);
+                const bool movA = mA != 0.0f || iA != 0.0f, movB = mB != 0.0f || iB != 0.0f;
+                const V2 vA{cur.g0.x, cur.g0.y}, vB{cur.g1.x, cur.g1.y};
+                const float wA = cur.g0.z, wB = cur.g1.z, ltOld = cur.g0.w, lnOld = cur.g1.w;
                 // Forward recomputation of this update.
                 const V2 cl0 = (vB + mul(revperp(rB), wB)) - (vA + mul(revperp(rA), wA));
                 const float vt = dot(cl0, tg);
@@ -167,25 +355,26 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
                 const V2 vA1 = vA - mul(mA, PT), vB1 = vB + mul(mB, PT);
                 const float wA1 = wA - iA * cross(rA, PT), wB1 = wB + iB * cross(rB, PT);
                 const V2 cl1 = (vB1 + mul(revperp(rB), wB1)) - (vA1 + mul(revperp(rA), wA1));
-                const float vn = dot(cl1, n);
+                const float vn = dot(cl1, nrm);
                 const float rawN = lnOld + nm * (bias - vn);
                 const float lnNew = (rawN < 0.0f) ? 0.0f : rawN;
                 const float incN = lnNew - lnOld;
-                // Adjoints of the outputs.
-                float4 va4 = a.vbar[bo + bA], vb4 = a.vbar[bo + bB];
+                // Adjoints of the outputs (a body that does not move has none
+                // that reaches another).
+                const float4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+                const float4 va4 = movA ? V[bA] : zero, vb4 = movB ? V[bB] : zero;
                 V2 vbA = v2(va4), vbB = v2(vb4);
                 float wbA = va4.z, wbB = vb4.z;
-                float2 lb = a.lamtmp[slot];  // (normal, tangent)
-                float4 c0 = a.cbar[slot * 3 + 0], c1 = a.cbar[slot * 3 + 1], c2 = a.cbar[slot * 3 + 2];
+                float2 lb = lb0;
                 V2 nbar{c0.x, c0.y}, rAbar{c0.z, c0.w}, rBbar{c1.x, c1.y}, tbar{c1.z, c1.w};
                 float nmbar = c2.x, tmbar = c2.y, biasbar = c2.z, fbar = c2.w;
                 // Normal update.
                 {
                     const V2 gv = mul(mB, vbB) - mul(mA, vbA);
-                    const float ginc = dot(gv, n) - iA * wbA * cross(rA, n) + iB * wbB * cross(rB, n);
+                    const float ginc = dot(gv, nrm) - iA * wbA * cross(rA, nrm) + iB * wbB * cross(rB, nrm);
                     nbar = nbar + mul(gv, incN) + mul(revperp(rA), -iA * wbA * incN) + mul(revperp(rB), iB * wbB * incN);
-                    rAbar = rAbar + mul(perp_grad(n), -iA * wbA * incN);
-                    rBbar = rBbar + mul(perp_grad(n), iB * wbB * incN);
+                    rAbar = rAbar + mul(perp_grad(nrm), -iA * wbA * incN);
+                    rBbar = rBbar + mul(perp_grad(nrm), iB * wbB * incN);
                     const float lnTot = lb.x + ginc;
                     float lnOldBar = -ginc;
                     const float rawBar = (rawN < 0.0f) ? 0.0f : lnTot;
@@ -193,7 +382,7 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
                     nmbar += rawBar * (bias - vn);
                     biasbar += rawBar * nm;
                     const float vnbar = -rawBar * nm;
-                    const V2 cbv = mul(n, vnbar);
+                    const V2 cbv = mul(nrm, vnbar);
                     nbar = nbar + mul(cl1, vnbar);
                     vbB = vbB + cbv;
                     wbB += cross(rB, cbv);
@@ -231,84 +420,92 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
                     rAbar = rAbar - mul(perp_grad(cbv), wA);
                     lb.y = ltOldBar;
                 }
-                if (mA != 0.0f || iA != 0.0f) a.vbar[bo + bA] = float4{vbA.x, vbA.y, wbA, va4.w};
-                a.vbar[bo + bB] = float4{vbB.x, vbB.y, wbB, vb4.w};
+                if (movA) V[bA] = float4{vbA.x, vbA.y, wbA, va4.w};
+                if (movB) V[bB] = float4{vbB.x, vbB.y, wbB, vb4.w};
                 a.lamtmp[slot] = lb;
                 a.cbar[slot * 3 + 0] = float4{nbar.x, nbar.y, rAbar.x, rAbar.y};
                 a.cbar[slot * 3 + 1] = float4{rBbar.x, rBbar.y, tbar.x, tbar.y};
                 a.cbar[slot * 3 + 2] = float4{nmbar, tmbar, biasbar, fbar};
             }
+            __syncthreads();
+            cur = next;
+            e = en;
         }
-        // Warm start, per slot.  Its deltas do not depend on velocities, so
-        // the velocity adjoints here are those after every slot's warm start
-        // and before any creation-time term below is added: constraint
-        // creation (the restitution bias reads the velocities) precedes the
-        // whole island's warm start in the forward step.
-        for (int e = rng.x; e < rng.y; ++e) {
-            const std::size_t slot = std::size_t(co) + e;
-            const float4* vc = t.vc + slot * prx::kTapeVc;
-            if ((__float_as_uint(vc[10].z) >> 8) != 1u) continue;
-            const V2 n = v2(vc[0]);
-            const V2 tg = fwdperp(n);
-            const V2 rA{vc[3].x, vc[3].y}, rB{vc[3].z, vc[3].w};
-            const float lnInit = vc[4].x, ltInit = vc[4].y;
-            const float4 ms = vc[8];
-            const float mA = ms.x, iA = ms.y, mB = ms.z, iB = ms.w;
-            const int bA = __float_as_int(vc[2].w), bB = __float_as_int(vc[5].z);
-            float2 lb = a.lamtmp[slot];
-            if (c.warmStart) {
-                const float4 va4 = a.vbar[bo + bA], vb4 = a.vbar[bo + bB];
-                const V2 vbA = v2(va4), vbB = v2(vb4);
-                const float wbA = va4.z, wbB = vb4.z;
-                const float4 c0 = a.cbar[slot * 3 + 0], c1 = a.cbar[slot * 3 + 1];
-                V2 nbar{c0.x, c0.y}, rAbar{c0.z, c0.w}, rBbar{c1.x, c1.y}, tbar{c1.z, c1.w};
-                const V2 P = mul(lnInit, n) + mul(ltInit, tg);
-                const V2 Pbar = mul(mB, vbB) - mul(mA, vbA) + mul(revperp(rA), -iA * wbA) + mul(revperp(rB), iB * wbB);
-                rAbar = rAbar + mul(perp_grad(P), -iA * wbA);
-                rBbar = rBbar + mul(perp_grad(P), iB * wbB);
-                lb.x += dot(Pbar, n);
-                lb.y += dot(Pbar, tg);
-                nbar = nbar + mul(Pbar, lnInit);
-                tbar = tbar + mul(Pbar, ltInit);
-                a.cbar[slot * 3 + 0] = float4{nbar.x, nbar.y, rAbar.x, rAbar.y};
-                a.cbar[slot * 3 + 1] = float4{rBbar.x, rBbar.y, tbar.x, tbar.y};
-            }
-            // Impulses as carried from the previous step (dtRatio scaling is
-            // part of the record: warm start uses them as stored); nothing
-            // for a contact created before this step's solve.
-            const std::uint32_t id = __float_as_uint(vc[10].y);
-            const bool fresh = (t.cmap[co + int(id)] & prx::kCarryFresh) != 0u;
-            a.lambar[co + int(id)] = fresh ? float4{0.0f, 0.0f, 0.0f, 0.0f} : float4{lb.x, lb.y, lnInit, ltInit};
+    }
+    // Warm start, per slot.  Its deltas do not depend on velocities, so
+    // the velocity adjoints here are those after every slot's warm start
+    // and before any creation-time term below is added: constraint
+    // creation (the restitution bias reads the velocities) precedes the
+    // whole island's warm start in the forward step.
+    for (int e = lane; e < n; e += kWave) {
+        const std::size_t slot = std::size_t(co) + e;
+        const float4* vc = vcrec(e);
+        if ((__float_as_uint(vc[10].z) >> 8) != 1u) continue;
+        const V2 nrm = v2(vc[0]);
+        const V2 tg = fwdperp(nrm);
+        const V2 rA{vc[3].x, vc[3].y}, rB{vc[3].z, vc[3].w};
+        const float lnInit = vc[4].x, ltInit = vc[4].y;
+        const float4 ms = vc[8];
+        const float mA = ms.x, iA = ms.y, mB = ms.z, iB = ms.w;
+        const int bA = __float_as_int(vc[2].w), bB = __float_as_int(vc[5].z);
+        float2 lb = a.lamtmp[slot];
+        if (c.warmStart) {
+            const float4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+            const float4 va4 = (mA != 0.0f || iA != 0.0f) ? V[bA] : zero;
+            const float4 vb4 = (mB != 0.0f || iB != 0.0f) ? V[bB] : zero;
+            const V2 vbA = v2(va4), vbB = v2(vb4);
+            const float wbA = va4.z, wbB = vb4.z;
+            const float4 c0 = a.cbar[slot * 3 + 0], c1 = a.cbar[slot * 3 + 1];
+            V2 nbar{c0.x, c0.y}, rAbar{c0.z, c0.w}, rBbar{c1.x, c1.y}, tbar{c1.z, c1.w};
+            const V2 P = mul(lnInit, nrm) + mul(ltInit, tg);
+            const V2 Pbar = mul(mB, vbB) - mul(mA, vbA) + mul(revperp(rA), -iA * wbA) + mul(revperp(rB), iB * wbB);
+            rAbar = rAbar + mul(perp_grad(P), -iA * wbA);
+            rBbar = rBbar + mul(perp_grad(P), iB * wbB);
+            lb.x += dot(Pbar, nrm);
+            lb.y += dot(Pbar, tg);
+            nbar = nbar + mul(Pbar, lnInit);
+            tbar = tbar + mul(Pbar, ltInit);
+            a.cbar[slot * 3 + 0] = float4{nbar.x, nbar.y, rAbar.x, rAbar.y};
+            a.cbar[slot * 3 + 1] = float4{rBbar.x, rBbar.y, tbar.x, tbar.y};
         }
-        // Constraint creation, per slot.
-        for (int e = rng.x; e < rng.y; ++e) {
+        // Impulses as carried from the previous step (dtRatio scaling is
+        // part of the record: warm start uses them as stored); nothing
+        // for a contact created before this step's solve.
+        const std::uint32_t id = __float_as_uint(vc[10].y);
+        const bool fresh = (t.cmap[co + int(id)] & prx::kCarryFresh) != 0u;
+        a.lambar[co + int(id)] = fresh ? float4{0.0f, 0.0f, 0.0f, 0.0f} : float4{lb.x, lb.y, lnInit, ltInit};
+    }
+    __syncthreads();
+    // Constraint creation, round by round (its terms add to the bodies').
+    int slots = 0, biased = 0;
+    for (int r = 0; r < rounds; ++r) {
+        const int pos = start[r] + lane;
+        const int e = pos < start[r + 1] ? order[pos] : -1;
+        if (e >= 0 && (__float_as_uint(vcrec(e)[10].z) >> 8) == 1u) {
             const std::size_t slot = std::size_t(co) + e;
-            const float4* vc = t.vc + slot * prx::kTapeVc;
-            if ((__float_as_uint(vc[10].z) >> 8) != 1u) continue;
+            const float4* vc = vcrec(e);
             const std::uint32_t type = __float_as_uint(vc[10].z) & 0xffu;
-            const V2 n = v2(vc[0]);
-            const V2 tg = fwdperp(n);
+            const V2 nrm = v2(vc[0]);
+            const V2 tg = fwdperp(nrm);
             const V2 rA{vc[3].x, vc[3].y}, rB{vc[3].z, vc[3].w};
             const float nm = vc[4].z, tm = vc[4].w;
             const float4 ms = vc[8];
             const float mA = ms.x, iA = ms.y, mB = ms.z, iB = ms.w;
             const int bA = __float_as_int(vc[2].w), bB = __float_as_int(vc[5].z);
-            const float4 va4 = a.vbar[bo + bA], vb4 = a.vbar[bo + bB];
-            V2 vbA = v2(va4), vbB = v2(vb4);
-            float wbA = va4.z, wbB = vb4.z;
+            const bool movA = mA != 0.0f || iA != 0.0f, movB = mB != 0.0f || iB != 0.0f;
             const float4 c0 = a.cbar[slot * 3 + 0], c1 = a.cbar[slot * 3 + 1], c2 = a.cbar[slot * 3 + 2];
             V2 nbar{c0.x, c0.y}, rAbar{c0.z, c0.w}, rBbar{c1.x, c1.y}, tbar{c1.z, c1.w};
             const float nmbar = c2.x, tmbar = c2.y, biasbar = c2.z, fbarC = c2.w;
             // Effective masses (VelocityConstraint.cpp:136-185).
             {
-                const float cnA = cross(rA, n), cnB = cross(rB, n);
+                const float cnA = cross(rA, nrm), cnB = cross(rB, nrm);
                 const float K = mA + mB + iA * cnA * cnA + iB * cnB * cnB;
                 if (K > 0.0f) {
                     const float Kbar = -nmbar * nm * nm;
                     const float gA = 2.0f * iA * cnA * Kbar, gB = 2.0f * iB * cnB * Kbar;
-                    rAbar = rAbar + mul(perp_grad(n), gA);
+                    rAbar = rAbar + mul(perp_grad(nrm), gA);
                     nbar = nbar + mul(revperp(rA), gA);
-                    rBbar = rBbar + mul(perp_grad(n), gB);
+                    rBbar = rBbar + mul(perp_grad(nrm), gB);
                     nbar = nbar + mul(revperp(rB), gB);
                 }
                 const float ctA = cross(rA, tg), ctB = cross(rB, tg);
@@ -326,19 +523,21 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
             const float vn0 = vc[10].x;
             const float rest = vc[5].w;
             const float4 vA0 = vc[12], vB0 = vc[13];
-            atomicAdd(a.diag + 0, 1.0f);
+            V2 dvA{0.0f, 0.0f}, dvB{0.0f, 0.0f};
+            float dwA = 0.0f, dwB = 0.0f;
+            ++slots;
             if (vn0 < -c.velocityThreshold) {
-                atomicAdd(a.diag + 1, 1.0f);
+                ++biased;
                 const float ebarC = -vn0 * biasbar;
                 const float vn0bar = -rest * biasbar;
                 const V2 cl0 = (V2{vB0.x, vB0.y} + mul(revperp(rB), vB0.z)) - (V2{vA0.x, vA0.y} + mul(revperp(rA), vA0.z));
-                const V2 cbv = mul(n, vn0bar);
+                const V2 cbv = mul(nrm, vn0bar);
                 nbar = nbar + mul(cl0, vn0bar);
-                vbB = vbB + cbv;
-                wbB += cross(rB, cbv);
+                dvB = cbv;
+                dwB = cross(rB, cbv);
                 rBbar = rBbar + mul(perp_grad(cbv), vB0.z);
-                vbA = vbA - cbv;
-                wbA -= cross(rA, cbv);
+                dvA = -cbv;
+                dwA = -cross(rA, cbv);
                 rAbar = rAbar - mul(perp_grad(cbv), vA0.z);
                 // Restitution = max(eA, eB), ties to B (Contact.hpp:66-69).
                 const int sA = __float_as_int(vc[11].y), sB = __float_as_int(vc[11].z);
@@ -355,49 +554,55 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
                     atomicAdd(a.fbar + sB, fbarC * fA / (2.0f * fm));
                 }
             }
-            if (mA != 0.0f || iA != 0.0f) a.vbar[bo + bA] = float4{vbA.x, vbA.y, wbA, va4.w};
-            a.vbar[bo + bB] = float4{vbB.x, vbB.y, wbB, vb4.w};
+            if (movA) add_body(V + bA, dvA, dwA);
+            if (movB) add_body(V + bB, dvB, dwB);
             // Geometry (WorldManifold.cpp:37-130): tangent from the normal,
             // then the normal and points from the positions.
             nbar.x += -tbar.y;
             nbar.y += tbar.x;
-            const float4 pos = vc[9];
+            const float4 pos4 = vc[9];
             const float rAd = vc[10].w, rBd = vc[11].x;
             if (type == 1u) {
-                const V2 dd = V2{pos.z - pos.x, pos.w - pos.y};
+                const V2 dd = V2{pos4.z - pos4.x, pos4.w - pos4.y};
                 const float L = __builtin_sqrtf(magsq(dd));
                 if (L > 0.0f) {
                     const float k = 0.5f * (rAd - rBd);
                     V2 dbar = mul(rAbar - rBbar, 0.5f);
                     const V2 ntot = nbar + mul(rAbar + rBbar, k);
-                    const float nn = dot(n, ntot);
-                    dbar = dbar + mul(ntot - mul(n, nn), 1.0f / L);
-                    if (mA != 0.0f || iA != 0.0f) add_body(a.xbar + bo + bA, -dbar, 0.0f);
-                    add_body(a.xbar + bo + bB, dbar, 0.0f);
+                    const float nn = dot(nrm, ntot);
+                    dbar = dbar + mul(ntot - mul(nrm, nn), 1.0f / L);
+                    if (movA) add_body(X + bA, -dbar, 0.0f);
+                    if (movB) add_body(X + bB, dbar, 0.0f);
                 }
             } else if (type == 2u) {
                 // relB = ((rA - dd) - rB) / 2 n with dd = dot(cB - plane, n);
                 // the normal and plane belong to the static body.
-                const float ddbar = -0.5f * dot(rBbar, n);
-                add_body(a.xbar + bo + bB, mul(n, ddbar), 0.0f);
+                const float ddbar = -0.5f * dot(rBbar, nrm);
+                if (movB) add_body(X + bB, mul(nrm, ddbar), 0.0f);
             }
         }
+        __syncthreads();
     }
-    __syncthreads();
     // Velocity integration, reversed (damping factors; caps not active).
     for (int b = lane; b < nb; b += kWave) {
-        if (!t.inisl[bo + b]) continue;
         const int gb = bo + b;
-        if (!(d.bflags[gb] & prx::kAccelerable)) continue;
-        const float2 dm = d.damp[gb];
-        const float fl = 1.0f / (1.0f + c.dt * dm.x);
-        const float fa = 1.0f / (1.0f + c.dt * dm.y);
-        float4 v = a.vbar[gb];
-        v.x *= fl;
-        v.y *= fl;
-        v.z *= fa;
+        float4 v = V[b];
+        if (t.inisl[gb] && (d.bflags[gb] & prx::kAccelerable)) {
+            const float2 dm = d.damp[gb];
+            const float fl = 1.0f / (1.0f + c.dt * dm.x);
+            const float fa = 1.0f / (1.0f + c.dt * dm.y);
+            v.x *= fl;
+            v.y *= fl;
+            v.z *= fa;
+        }
         a.vbar[gb] = v;
+        if constexpr (kLds) a.xbar[gb] = X[b];
     }
+    if (unmodelled) *a.status = 1;
+    add_diag(a.diag, 0, slots);
+    add_diag(a.diag, 1, biased);
+    add_diag(a.diag, 2, posUpdates);
+    add_diag(a.diag, 3, velUpdates);
 }
 
 // ---------------------------------------------------------------------------
@@ -925,15 +1130,27 @@ __global__ __launch_bounds__(64) void k_adjoint_general(DeviceState d, Tape t, A
 
 }  // namespace prxd
 
+namespace {
+// The body adjoints and round plans are kept in LDS where the largest world's
+// fit the default limit.
+constexpr std::size_t kAdjLdsLimit = 60 * 1024;
+}  // namespace
+
 extern "C" hipError_t prx_launch_adjoint_general(const prx::DeviceState* d, const prx::Tape* t,
                                                  const prx::AdjState* a, const prx::StepParams* c, int nworlds,
-                                                 hipStream_t s) {
+                                                 int maxBodies, int maxSlots, hipStream_t s) {
+    (void)maxBodies;
+    (void)maxSlots;
     hipLaunchKernelGGL(prxd::k_adjoint_general, dim3(unsigned(nworlds)), dim3(64), 0, s, *d, *t, *a, *c);
     return hipGetLastError();
 }
 
 extern "C" hipError_t prx_launch_adjoint_step(const prx::DeviceState* d, const prx::Tape* t, const prx::AdjState* a,
-                                              const prx::StepParams* c, int nworlds, hipStream_t s) {
-    hipLaunchKernelGGL(prxd::k_adjoint_step, dim3(unsigned(nworlds)), dim3(64), 0, s, *d, *t, *a, *c);
+                                              const prx::StepParams* c, int nworlds, int maxBodies, int maxSlots,
+                                              hipStream_t s) {
+    const std::size_t lds = std::size_t(maxBodies) * 36 + std::size_t(maxSlots) * 12 + 4;
+    const dim3 grid{unsigned(nworlds)}, block(64);
+    if (lds <= kAdjLdsLimit) hipLaunchKernelGGL(prxd::k_adjoint_step<true>, grid, block, lds, s, *d, *t, *a, *c);
+    else hipLaunchKernelGGL(prxd::k_adjoint_step<false>, grid, block, 0, s, *d, *t, *a, *c);
     return hipGetLastError();
 }

@@ -46,10 +46,11 @@ extern "C" hipError_t prx_launch_report(const prx::DeviceState* d, std::uint32_t
 extern "C" hipError_t prx_launch_step_tape(const prx::DeviceState* d, const prx::StepParams* c, int count,
                                            hipStream_t stream);
 extern "C" hipError_t prx_launch_adjoint_step(const prx::DeviceState* d, const prx::Tape* t, const prx::AdjState* a,
-                                              const prx::StepParams* c, int nworlds, hipStream_t s);
+                                              const prx::StepParams* c, int nworlds, int maxBodies, int maxSlots,
+                                              hipStream_t s);
 extern "C" hipError_t prx_launch_adjoint_general(const prx::DeviceState* d, const prx::Tape* t,
                                                  const prx::AdjState* a, const prx::StepParams* c, int nworlds,
-                                                 hipStream_t s);
+                                                 int maxBodies, int maxSlots, hipStream_t s);
 
 namespace {
 
@@ -3501,6 +3502,7 @@ std::vector<std::pair<void*, std::size_t>> DynamicArrays(prx_batch* b) {
 struct prx_adjoint {
     prx_batch* b = nullptr;
     int K = 0, S = 0, nseg = 0, itV = 0, itP = 0;
+    int maxBodies = 0, maxSlots = 0;  // of a world: bodies, contact slots and joints
     bool general = false;  // joints, polygons or off-centre disks: the general reverse kernel
     DeviceArena arena;
     std::vector<prx::Tape> tapes;
@@ -3536,9 +3538,12 @@ int AdjointCopy(prx_adjoint* adj, int k, bool save) {
 }
 
 // K steps from the batch's state with a checkpoint every S steps; the batch
-// is left at the final state.
-int AdjointForward(prx_adjoint* adj, const prx::StepParams& p) {
+// is left at the final state.  These steps record nothing, so large islands
+// are swept by the whole wave as in any batch (same bits).
+int AdjointForward(prx_adjoint* adj, const prx::StepParams& recorded) {
     prx_batch* b = adj->b;
+    prx::StepParams p = recorded;
+    p.coopMin = b->conf.coop_min_contacts;
     const int nw = int(b->worlds.size());
     hipStream_t st = b->stream;
     PRX_HIP(hipEventRecord(b->ev0, st));
@@ -3588,8 +3593,10 @@ int AdjointBackward(prx_adjoint* adj, const prx::StepParams& p, const std::vecto
         }
         for (int s = n - 1; s >= 0; --s) {
             const hipError_t le =
-                adj->general ? prx_launch_adjoint_general(&b->d, &adj->tapes[std::size_t(s)], &adj->a, &p, nw, st)
-                             : prx_launch_adjoint_step(&b->d, &adj->tapes[std::size_t(s)], &adj->a, &p, nw, st);
+                adj->general ? prx_launch_adjoint_general(&b->d, &adj->tapes[std::size_t(s)], &adj->a, &p, nw,
+                                                          adj->maxBodies, adj->maxSlots, st)
+                             : prx_launch_adjoint_step(&b->d, &adj->tapes[std::size_t(s)], &adj->a, &p, nw,
+                                                       adj->maxBodies, adj->maxSlots, st);
             if (le != hipSuccess) return Fail(PRX_E_DEVICE, std::string("launch: ") + hipGetErrorString(le));
         }
     }
@@ -3683,6 +3690,11 @@ int prx_adjoint_create(prx_batch* b, int nsteps, int every, const prx_step_conf*
     PRX_HIP(A.alloc(adj->a.jlam, J));
     PRX_HIP(A.alloc(adj->a.jcarry, J));
     PRX_HIP(A.alloc(adj->a.tbar, J));
+    PRX_HIP(A.alloc(adj->a.plan, (C + J) * std::size_t(prx::kAdjPlanInts)));
+    for (const auto& h : b->hdr) {
+        adj->maxBodies = std::max<int>(adj->maxBodies, h.nbodies);
+        adj->maxSlots = std::max<int>(adj->maxSlots, h.contact_cap + h.njoints);
+    }
     const auto arrays = DynamicArrays(b);
     adj->ckpt.resize(std::size_t(adj->nseg));
     for (auto& ck : adj->ckpt) {

@@ -154,7 +154,9 @@ struct AdjState {
     float4* jlam;   // per joint slot: adjoint of the running impulses (x, y, z, motor)
     float4* jcarry; // per joint: adjoint of the impulses the later step started from
     float* tbar;    // per joint: d loss / d maximum motor torque
+    int* plan;      // reverse rounds: kAdjPlanInts per contact slot and joint (segment contact_off + joint_off)
 };
+constexpr int kAdjPlanInts = 8;
 constexpr int kAdjFields = 32;
 constexpr int kAdjJointFields = 16;
 

@@ -1,0 +1,49 @@
+"""The reverse kernels keep a batch's body adjoints and round plans in LDS
+where its largest world's fit, else in global memory: a world's gradients are
+the same to the bit in either form, and do not depend on its neighbours."""
+import numpy as np
+import pytest
+
+import playrho_amd as pa
+from tests import dumpfmt
+
+pytestmark = pytest.mark.gpu
+
+# Disks (the disk kernel); polygons, joints and both (the general kernel).
+CASES = [
+    ("billiards", [1, 0]),
+    ("pile", [1, 0, 8, 8]),
+    ("pile", [2, 0, 48, 48]),
+    ("chain", [3, 0, 8, 12, 2]),
+    ("chain", [3, 1, 1, 0, 2]),
+]
+
+
+def _desc(scene, params, extra=0):
+    w = pa.World.scene(scene, params)
+    for _ in range(extra):
+        w.create_body(pa.BodyConf())
+    return w.save_desc()
+
+
+def _targets(desc, seed):
+    n = len(dumpfmt.read_description(dumpfmt.Reader(desc))[1])
+    return np.random.default_rng(seed).uniform(-5, 10, (n, 2)).astype(np.float32)
+
+
+@pytest.mark.parametrize("scene,params", CASES)
+def test_global_form_equals_lds_form(scene, params):
+    conf = pa.StepConf(do_toi=0)
+    steps = 20
+    # The neighbour's 36 bytes a body exceed the 60 KiB kept in LDS.
+    descs = [_desc(scene, params), _desc(scene, params, 60 * 1024 // 36 + 1)]
+    targets = [_targets(d, k) for k, d in enumerate(descs)]
+    one = pa.Adjoint(pa.Batch([pa.World.from_desc(descs[0])], use_graph=False), steps, 8, conf).run(targets[0])
+    both = pa.Adjoint(pa.Batch([pa.World.from_desc(d) for d in descs], use_graph=False), steps, 8, conf)
+    both = both.run(np.concatenate(targets))
+    assert both["loss"][0] == one["loss"][0]
+    assert np.any(one["grad_velocity"] != 0.0)
+    assert np.array_equal(both["grad_velocity"][:len(targets[0])], one["grad_velocity"])
+    if "grad_motor_torque" in one:
+        nj = len(one["grad_motor_torque"])
+        assert np.array_equal(both["grad_motor_torque"][:nj], one["grad_motor_torque"])
