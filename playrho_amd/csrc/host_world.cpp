@@ -1251,10 +1251,11 @@ int BuildBatch(prx_batch* b) {
     }
     int maxNb = 0;
     for (const prx_world* w : b->worlds) maxNb = std::max<int>(maxNb, int(w->bodies.size()));
-    // Body constraint state (32 B per body) plus the record stage; worlds whose
-    // bodies do not fit keep them in global scratch.
+    // Body constraint state (32 B per body), two words per island (at most one
+    // island per body) and the record stage; worlds whose bodies do not fit
+    // keep them in global scratch.
     const int stageBytes = prx::kStageFloat4 * 16;
-    b->lds_min = std::min<int>(64 * 1024, std::max<int>(1024 + stageBytes, ((maxNb * 32 + stageBytes + 255) / 256) * 256));
+    b->lds_min = std::min<int>(64 * 1024, std::max<int>(1024 + stageBytes, ((maxNb * 40 + stageBytes + 255) / 256) * 256));
     b->totB = B;
     b->totP = P;
     b->totS = S;
@@ -1312,8 +1313,8 @@ int BuildBatch(prx_batch* b) {
     PRX_HIP(a.alloc(d.s_bc_vel, B));
     PRX_HIP(a.alloc(d.s_vc, C * std::size_t(prx::kVcStride)));
     PRX_HIP(a.alloc(d.s_pc, C * std::size_t(prx::kPcStride)));
-    PRX_HIP(a.alloc(d.s_vc2, C * std::size_t(prx::kVcStride)));
-    PRX_HIP(a.alloc(d.s_pc2, C * std::size_t(prx::kPcStride)));
+    PRX_HIP(a.alloc(d.s_vc2, C * std::size_t(prx::kQuadVc)));
+    PRX_HIP(a.alloc(d.s_pc2, C * std::size_t(prx::kQuadPc)));
     PRX_HIP(a.alloc(d.s_lvl, C * std::size_t(prx::kLevelInts)));
     PRX_HIP(a.alloc(d.j_body, J));
     PRX_HIP(a.alloc(d.j_anchor, J));

@@ -290,6 +290,8 @@ constexpr int kEvWordsPerSlot = 48;
 
 constexpr int kVcStride = 9;
 constexpr int kPcStride = 5;
+constexpr int kQuadVc = 10;  // float4 of a velocity record of the level form
+constexpr int kQuadPc = 7;   // and of a position record
 enum : std::uint32_t { kJointLimit = 1u, kJointMotor = 2u, kJointCollideConnected = 4u };
 // Pi as the float build's Real (RealConstants.hpp:57).
 constexpr float kPiF = 3.14159265358979323846f;

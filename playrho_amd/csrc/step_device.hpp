@@ -3739,559 +3739,620 @@ __device__ __forceinline__ PosResult island_position_wave(const DeviceState& d, 
 }
 
 // ---------------------------------------------------------------------------
-// Paired-lane forms of the contact updates for the level form: lane 2j
-// (side 0) computes update j's body-A terms and lane 2j + 1 (side 1) its
-// body-B terms, exchanging what the other body contributes through a DPP
-// swap within the pair; terms of both bodies (relative velocity, impulses,
-// block-solver cases, position-solver manifolds) are computed by both lanes
-// from the same values.  Body A's changes are the negated body-B form
-// (a - b*c = a + (-1)*(b*c) exactly), so both lanes run one instruction
-// stream and every result equals the single-lane form bit for bit.
-__device__ __forceinline__ float pair_swap(float v) {
-    // quad_perm [1, 0, 3, 2]: each lane reads its pair partner.
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
-}
-__device__ __forceinline__ V2 pair_swap(V2 v) { return V2{pair_swap(v.x), pair_swap(v.y)}; }
-
-// GetContactRelVelocity (d2/Math.cpp:73-103) from the pair's two halves.
-__device__ __forceinline__ V2 pair_rel_vel(V2 v, float w, V2 rel, int side) {
-    const V2 u = v + mul(revperp(rel), w / 1.0f);
-    const V2 o = pair_swap(u);
-    const V2 uA = side ? o : u;
-    const V2 uB = side ? u : o;
-    return uB - uA;
-}
-
-struct PairBody {
-    float m, i, sgn;  // inverse mass, inverse rotational inertia, -1 for body A
-};
-
-__device__ __forceinline__ void pair_apply(V2& v, float& w, const PairBody& b, V2 P, float L) {
-    const V2 mp = mul(b.m, P);
-    v = V2{v.x + b.sgn * mp.x, v.y + b.sgn * mp.y};
-    w = w + b.sgn * (b.i * L);
-}
-
-__device__ __forceinline__ float solve_dir_pair(Vc& vc, bool tangent, const PairBody& me, int side, V2& v, float& w) {
-    float maxInc = 0.0f;
-    const V2 dir = tangent ? fwdperp(vc.normal) : vc.normal;
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-        const int k = 1 - kk;  // point 1 first, then point 0
-        if (k >= int(vc.n)) continue;
-        VcPoint& p = vc.p[k];
-        const V2 rel = side ? p.relB : p.relA;
-        const V2 closing = pair_rel_vel(v, w, rel, side);
-        float oldI, newI;
-        if (tangent) {
-            const float dirVel = vc.tangentSpeed - dot(closing, dir);
-            const float lambda = p.tm * dirVel;
-            const float maxI = vc.friction * p.ni;
-            oldI = p.ti;
-            newI = clamp_std(oldI + lambda, -maxI, maxI);
-        } else {
-            const float dirVel = dot(closing, dir);
-            const float lambda = p.nm * (p.bias - dirVel);
-            oldI = p.ni;
-            newI = fmax_std(oldI + lambda, 0.0f);
-        }
-        const float inc = newI - oldI;
-        const V2 P = mul(inc, dir);
-        pair_apply(v, w, me, P, cross(rel, P) / 1.0f);
-        maxInc = fmax_std(maxInc, __builtin_fabsf(inc));
-        if (tangent) p.ti = oldI + inc;
-        else p.ni = oldI + inc;
-    }
-    return maxInc;
-}
-
-__device__ __forceinline__ float block_solve_pair(Vc& vc, const PairBody& me, int side, V2& v, float& w) {
-    const V2 normal = vc.normal;
-    const V2 rel0 = side ? vc.p[0].relB : vc.p[0].relA;
-    const V2 rel1 = side ? vc.p[1].relB : vc.p[1].relA;
-    V2 bp;
-    {
-        const V2 dv0 = pair_rel_vel(v, w, rel0, side);
-        const V2 dv1 = pair_rel_vel(v, w, rel1, side);
-        const float vn0 = dot(dv0, normal);
-        const float vn1 = dot(dv1, normal);
-        const V2 b{vn0 - vc.p[0].bias, vn1 - vc.p[1].bias};
-        float t0 = 0.0f;
-        t0 += vc.K00 * vc.p[0].ni;
-        t0 += vc.K01 * vc.p[1].ni;
-        float t1 = 0.0f;
-        t1 += vc.K01 * vc.p[0].ni;
-        t1 += vc.K11 * vc.p[1].ni;
-        bp = V2{b.x - t0, b.y - t1};
-    }
-    float x0 = 0.0f;
-    x0 += vc.M00 * bp.x;
-    x0 += vc.M01 * bp.y;
-    float x1 = 0.0f;
-    x1 += vc.M01 * bp.x;
-    x1 += vc.M11 * bp.y;
-    const float c1n0 = -x0, c1n1 = -x1;
-    const bool ok1 = c1n0 >= 0.0f && c1n1 >= 0.0f;
-    const float c2n0 = -vc.p[0].nm * bp.x;
-    const float vn2 = vc.K01 * c2n0 + bp.y;
-    const bool ok2 = c2n0 >= 0.0f && vn2 >= 0.0f;
-    const float c3n1 = -vc.p[1].nm * bp.y;
-    const float vn1 = vc.K01 * c3n1 + bp.x;
-    const bool ok3 = c3n1 >= 0.0f && vn1 >= 0.0f;
-    const bool ok4 = bp.x >= 0.0f && bp.y >= 0.0f;
-    const float n0 = ok1 ? c1n0 : (ok2 ? c2n0 : 0.0f);
-    const float n1 = ok1 ? c1n1 : (ok2 ? 0.0f : (ok3 ? c3n1 : 0.0f));
-    const bool ok = ok1 || ok2 || ok3 || ok4;
-    const float d0 = n0 - vc.p[0].ni;
-    const float d1 = n1 - vc.p[1].ni;
-    const V2 P0 = mul(d0, normal);
-    const V2 P1 = mul(d1, normal);
-    const V2 P = P0 + P1;
-    const float L = (cross(rel0, P0) + cross(rel1, P1)) / 1.0f;
-    V2 nv = v;
-    float nw = w;
-    pair_apply(nv, nw, me, P, L);
-    v = ok ? nv : v;
-    w = ok ? nw : w;
-    vc.p[0].ni = ok ? n0 : vc.p[0].ni;
-    vc.p[1].ni = ok ? n1 : vc.p[1].ni;
-    return ok ? fmax_std(__builtin_fabsf(n0), __builtin_fabsf(n1)) : 0.0f;
-}
-
-template <bool kLds>
-__device__ __forceinline__ float solve_velocity_pair(Vc& vc, const BodyC& A, const BodyC& B, const Bodies<kLds>& bs,
-                                                     int side) {
-    const int b = side ? vc.bB : vc.bA;
-    const PairBody me{side ? B.invMass : A.invMass, side ? B.invRotI : A.invRotI, side ? 1.0f : -1.0f};
-    const float4 vel = bs.vel(b);
-    V2 v{vel.x, vel.y};
-    float w = vel.z;
-    float mi = 0.0f;
-    mi = fmax_std(mi, solve_dir_pair(vc, true, me, side, v, w));
-    float nrm;
-    if (vc.n == 1 || (vc.K00 == 0.0f && vc.K11 == 0.0f && vc.K01 == 0.0f)) nrm = solve_dir_pair(vc, false, me, side, v, w);
-    else nrm = block_solve_pair(vc, me, side, v, w);
-    mi = fmax_std(mi, nrm);
-    bs.set_vel(b, float4{v.x, v.y, w, vel.w});
-    return mi;
-}
-
-template <bool kLds>
-__device__ __forceinline__ void warm_start_pair(const Vc& vc, const BodyC& A, const BodyC& B, const Bodies<kLds>& bs,
-                                                int side) {
-    const int b = side ? vc.bB : vc.bA;
-    const PairBody me{side ? B.invMass : A.invMass, side ? B.invRotI : A.invRotI, side ? 1.0f : -1.0f};
-    const V2 tangent = fwdperp(vc.normal);
-    V2 dl{0, 0};
-    float da = 0.0f;
-#pragma unroll
-    for (std::uint32_t j = 0; j < 2; ++j) {
-        if (j >= vc.n) continue;
-        const VcPoint& p = vc.p[j];
-        const V2 P = mul(p.ni, vc.normal) + mul(p.ti, tangent);
-        pair_apply(dl, da, me, P, cross(side ? p.relB : p.relA, P) / 1.0f);
-    }
-    float4 vel = bs.vel(b);
-    vel.x = vel.x + dl.x;
-    vel.y = vel.y + dl.y;
-    vel.z = vel.z + da;
-    bs.set_vel(b, vel);
-}
-
-// GaussSeidel::SolvePositionConstraint (ContactSolver.cpp:494-643) in the
-// paired form of solve_pc: each lane computes its own body's transformation
-// (the sine and cosine of its angle) and position change.
-__device__ __forceinline__ float solve_pc_pair(const Manifold& m, float totalRadius, const BodyC& A, const BodyC& B,
-                                               float4& pos, int side, const StepParams& c) {
-    const float invMassTotal = A.invMass + B.invMass;
-    const BodyC& me = side ? B : A;
-    const float sgn = side ? 1.0f : -1.0f;
-    auto xfs = [&](V2 pl, float pa, Xf& xfA, Xf& xfB) {
-        const Xf mine = get_xf(pl.x, pl.y, pa, me.lc);
-        const Xf other{pair_swap(mine.p), pair_swap(mine.q)};
-        xfA = side ? other : mine;
-        xfB = side ? mine : other;
-    };
-    struct Sol {
-        V2 dl;
-        float da, sep;
-    };
-    auto solve = [&](const PSM& psm, V2 p) {
-        const float separation = psm.sep - totalRadius;
-        const V2 r = psm.point - p;
-        const float cr = cross(r, psm.normal) / 1.0f;
-        const float co = pair_swap(cr);
-        const float crA = side ? co : cr;
-        const float crB = side ? cr : co;
-        const float K = invMassTotal + A.invRotI * (crA * crA) + B.invRotI * (crB * crB);
-        const float C = -clamp_std(c.regResolutionRate * (separation + c.linearSlop), -c.maxLinearCorrection, 0.0f);
-        const V2 P = divs(mul(psm.normal, C), K);
-        const float L = cross(r, P) / 1.0f;
-        const V2 mp = mul(me.invMass, P);
-        return Sol{V2{sgn * mp.x, sgn * mp.y}, sgn * (me.invRotI * L), separation};
-    };
-    const V2 op{pos.x, pos.y};
-    const float oa = pos.z;
-    Xf xfA, xfB;
-    xfs(op, oa, xfA, xfB);
-    const PSM psm0 = get_psm(m, 0, xfA, xfB);
-    const PSM psm1 = get_psm(m, 1, xfA, xfB);
-    const bool two = m.n == 2;
-    const bool eq = two && almost_equal(psm0.sep, psm1.sep);
-    const bool lt = two && !eq && psm0.sep < psm1.sep;
-    const bool gt = two && !eq && psm1.sep < psm0.sep;
-    if (!(m.n == 1 || eq || lt || gt)) return __builtin_inff();
-    const Sol s0 = solve(gt ? psm1 : psm0, op);
-    V2 p = op + s0.dl;
-    float a = oa + s0.da;
-    const float minSep = two ? s0.sep : 0.0f + s0.sep;
-    if (two) {
-        Xf nA, nB;
-        xfs(p, a, nA, nB);
-        const PSM next = get_psm(m, gt ? 0u : 1u, nA, nB);
-        const Sol s1 = solve(eq ? psm1 : next, eq ? op : p);
-        p = p + s1.dl;
-        a = a + s1.da;
-    }
-    pos.x = p.x;
-    pos.y = p.y;
-    pos.z = a;
-    return minSep;
-}
-
-// ---------------------------------------------------------------------------
 // Level form of the wave-wide sweeps, for islands without joints in worlds of
 // at most kLevelMaxBodies bodies.  The Gauss-Seidel order is kept exactly: an
 // update's level is one more than the last level that touched either of its
 // bodies (bodies with zero inverse mass and inertia are never changed by an
 // update, so they order nothing), and the updates of one level touch
 // distinct bodies.  The wave runs each level's updates in parallel, level
-// after level, two lanes to an update (each lane computes its own body's
-// terms, the pair exchanging partial results), with the inputs the serial
-// sweep gives them; warm-start
+// after level, with the inputs the serial sweep gives them; warm-start
 // deltas reach each body in the same order, and the early exits reduce the
-// same maxima and minima.  The plan (levels, level order, rounds of at most
-// one wave) is built once per step and serves the warm start, the velocity
-// iterations and the position iterations; the records are copied into level
-// order so that a round reads consecutive records.
+// same maxima and minima.  One plan serves all the islands of a world at once
+// (they share no moving body): it is built once per step and serves the warm
+// start, the velocity iterations and the position iterations.  It sorts the
+// updates by level into rounds of at most kLevelRound updates of one level;
+// the records are copied into that order so that a round reads consecutive
+// records.  Islands of fewer than kLevelMinConstraints contacts stay on a
+// lane each: they would widen the first levels and cost more rounds than the
+// lanes they free.
+//
+// An iteration need not wait for the whole of the one before: an update of
+// iteration i + 1 needs only its two bodies' updates of iteration i.  With
+// every iteration started `period` rounds after the one before, where the
+// period is the most rounds any body's updates of one iteration span, each
+// body still sees its updates in order.  Pile islands of 100 to 530 contacts
+// have 62 to 243 levels (at most 9 updates wide) and periods of 25 to 207, so
+// two iterations run side by side, each on half of the wave (kLevelGroups),
+// and eight iterations take rounds + 7 periods instead of 8 rounds: 1.1 to
+// 2.1 times fewer.
 constexpr int kLevelMaxBodies = prx::kStageFloat4 * 4;
-constexpr int kLevelMinConstraints = 8;
-// Updates per round: two lanes serve one update (one lane per body).
-constexpr int kLevelRound = kWave / 2;
+constexpr int kLevelMinConstraints = 4;
+constexpr int kLevelGroups = 2;
+// Updates per round: four lanes serve one update.
+constexpr int kLevelRound = kWave / 4 / kLevelGroups;
 
 struct LevelPlan {
-    int n, rounds;
-    const int2* rb;    // per round: first and end position in level order
-    const int* order;  // level position -> island position
+    int n, rounds, period;
+    const int2* rb;    // per round: first position in level order, updates
+    const int* order;  // level position -> island-order slot
 };
 
-__device__ __forceinline__ int* level_ints(const DeviceState& d, const WorldCtx& x, int c0) {
-    return d.s_lvl + (std::size_t(x.co) + std::size_t(c0)) * prx::kLevelInts;
-}
-__device__ __forceinline__ int2* level_rounds(int* L, int n) { return reinterpret_cast<int2*>(L + ((3 * n + 3) & ~1)); }
+// Plan scratch of a world (kLevelInts ints per contact slot).
+struct LevelScratch {
+    int *lvl, *order, *sel, *island, *start;
+    int2* rb;
+    __device__ __forceinline__ LevelScratch(const DeviceState& d, const WorldCtx& x) {
+        int* L = d.s_lvl + std::size_t(x.co) * prx::kLevelInts;
+        const int cap = x.cap;
+        lvl = L;
+        order = L + cap;
+        sel = L + 2 * cap;
+        island = L + 3 * cap;
+        rb = reinterpret_cast<int2*>(L + 4 * cap);
+        start = L + 6 * cap;  // levels + 1
+    }
+};
 
-// Builds the plan of island [c0, c1) (n >= kLevelMinConstraints); the
-// record stage serves as the per-body last-level table.
-__device__ __forceinline__ LevelPlan level_plan(const DeviceState& d, const WorldCtx& x, float4* stage, int c0,
-                                                int c1) {
-    const int n = c1 - c0;
+// Two words per island in LDS behind the body state.  Velocity sweeps: the
+// iterations that changed an impulse (bit 31: left out of masked runs) and
+// the largest change (float bits).  Position sweeps: the smallest separation
+// of the iteration (order-preserving key) and the iteration that solved the
+// island plus one (0: none yet).
+__device__ __forceinline__ int* island_words(const WorldCtx& x) { return reinterpret_cast<int*>(g_smem + 2 * x.nb); }
+
+// Velocity record of an update in level order (kQuadVc float4), laid out for
+// the four lanes that solve it (lane 2 s + c: body A or B, component x or y):
+//   [0] [1] per lane (0..3): component c of the reverse-perpendicular arms of
+//           points 0 and 1 from body s
+//   [2] [3] per body: -+ inverse mass, -+ inverse rotational inertia (negative
+//           for A: its changes are added with the sign flipped), the LDS
+//           float index of its velocity
+//   [4]     tangent x, normal x, tangent y, normal y
+//   [5]     friction, tangent speed, tangent masses of points 0, 1
+//   [6]     biases 0, 1, normal masses 0, 1
+//   [7]     K00, K11, K01, points | island << 8
+//   [8]     M00, M11, M01, -
+//   [9]     normal and tangent impulse of point 0, of point 1
+__device__ __forceinline__ void store_quad_vc(float4* o, const Vc& vc, const BodyC& A, const BodyC& B, int nb, int island) {
+    const V2 tg = fwdperp(vc.normal);
+    auto q = [](V2 r0, V2 r1) {
+        const V2 a = revperp(r0), b = revperp(r1);
+        return float4{a.x, b.x, a.y, b.y};
+    };
+    o[0] = q(vc.p[0].relA, vc.p[1].relA);
+    o[1] = q(vc.p[0].relB, vc.p[1].relB);
+    o[2] = float4{-A.invMass, -A.invRotI, __int_as_float(4 * (nb + vc.bA)), 0.0f};
+    o[3] = float4{B.invMass, B.invRotI, __int_as_float(4 * (nb + vc.bB)), 0.0f};
+    o[4] = float4{tg.x, vc.normal.x, tg.y, vc.normal.y};
+    o[5] = float4{vc.friction, vc.tangentSpeed, vc.p[0].tm, vc.p[1].tm};
+    o[6] = float4{vc.p[0].bias, vc.p[1].bias, vc.p[0].nm, vc.p[1].nm};
+    o[7] = float4{vc.K00, vc.K11, vc.K01, __uint_as_float(vc.n | (std::uint32_t(island) << 8))};
+    o[8] = float4{vc.M00, vc.M11, vc.M01, 0.0f};
+    o[9] = float4{vc.p[0].ni, vc.p[0].ti, vc.p[1].ni, vc.p[1].ti};
+}
+
+// Position record of an update in level order (kQuadPc float4).  Its four
+// lanes (2 s + c) serve the body X holding the manifold's local point (s = 0:
+// A for circles and face A, B for face B) and the other body Y, component x
+// or y:
+//   [0] [1] per body: LDS float index of its position, -+ inverse mass, -+
+//           inverse rotational inertia (negative for A)
+//   [2] [3] X: local centre, local point, local point, local normal
+//   [4] [5] Y: local centre, manifold points 0 and 1
+//   [6]     total radius, total inverse mass, type | points << 8 | island << 16
+__device__ __forceinline__ void store_quad_pc(float4* o, const Pc& pc, int island) {
+    const bool faceB = pc.m.type == kFaceB;
+    const BodyC& X = faceB ? pc.B : pc.A;
+    const BodyC& Y = faceB ? pc.A : pc.B;
+    const float4 a{__int_as_float(4 * pc.bA), -pc.A.invMass, -pc.A.invRotI, 0.0f};
+    const float4 b{__int_as_float(4 * pc.bB), pc.B.invMass, pc.B.invRotI, 0.0f};
+    o[0] = faceB ? b : a;
+    o[1] = faceB ? a : b;
+    o[2] = float4{X.lc.x, X.lc.y, pc.m.lpt.x, pc.m.lpt.y};
+    o[3] = float4{pc.m.lpt.x, pc.m.lpt.y, pc.m.ln.x, pc.m.ln.y};
+    o[4] = float4{Y.lc.x, Y.lc.y, pc.m.p[0].lp.x, pc.m.p[0].lp.y};
+    o[5] = float4{pc.m.p[1].lp.x, pc.m.p[1].lp.y, 0.0f, 0.0f};
+    o[6] = float4{pc.totalRadius, pc.A.invMass + pc.B.invMass,
+                  __uint_as_float(pc.m.type | (pc.m.n << 8) | (std::uint32_t(island) << 16)), 0.0f};
+}
+
+// Builds the plan of the slots whose island (LevelScratch::island) is not
+// negative; the record stage serves as the per-body tables.
+__device__ __forceinline__ LevelPlan level_plan(const DeviceState& d, const WorldCtx& x, float4* stage, int nce) {
     const int lane = x.lane;
-    const float4* vbase = d.s_vc + (std::size_t(x.co) + std::size_t(c0)) * prx::kVcStride;
-    const float4* pbase = d.s_pc + (std::size_t(x.co) + std::size_t(c0)) * prx::kPcStride;
-    int* L = level_ints(d, x, c0);
-    int* lvl = L;
-    int* order = L + n;
-    int* start = L + 2 * n;  // levels + 1 entries
-    int2* rb = level_rounds(L, n);
+    const float4* vbase = d.s_vc + std::size_t(x.co) * prx::kVcStride;
+    const float4* pbase = d.s_pc + std::size_t(x.co) * prx::kPcStride;
+    const LevelScratch L(d, x);
     int* last = reinterpret_cast<int*>(stage);
     for (int b = lane; b < x.nb; b += kWave) last[b] = 0;
+    int n = 0;
+    for (int base = 0; base < nce; base += kWave) {
+        const bool in = base + lane < nce && L.island[base + lane] >= 0;
+        const unsigned long long m = __ballot(in);
+        if (in) L.sel[n + __popcll(m & lanes_below(lane))] = base + lane;
+        n += __popcll(m);
+    }
     __syncthreads();
     int levels = 0;
     for (int base = 0; base < n; base += kWave) {
         const int r = base + lane;
         int a = -1, bb = -1;
         if (r < n) {
-            const float4* v = vbase + std::size_t(r) * prx::kVcStride;
+            const float4* v = vbase + std::size_t(L.sel[r]) * prx::kVcStride;
             const float4 m = v[8];
             if (m.x != 0.0f || m.y != 0.0f) a = __float_as_int(v[2].w);
             if (m.z != 0.0f || m.w != 0.0f) bb = __float_as_int(v[5].z);
         }
         const int cnt = (n - base < kWave) ? n - base : kWave;
+        int mine = 0;
         for (int j = 0; j < cnt; ++j) {
-            const int aj = __shfl(a, j), bj = __shfl(bb, j);
+            // Uniform: every lane reads the same two words; one writes them.
+            const int aj = __builtin_amdgcn_readlane(a, j), bj = __builtin_amdgcn_readlane(bb, j);
+            const int la = (aj >= 0) ? last[aj] : 0;
+            const int lb = (bj >= 0) ? last[bj] : 0;
+            const int l = ((la > lb) ? la : lb) + 1;
             if (lane == 0) {
-                const int la = (aj >= 0) ? last[aj] : 0;
-                const int lb = (bj >= 0) ? last[bj] : 0;
-                const int l = ((la > lb) ? la : lb) + 1;
                 if (aj >= 0) last[aj] = l;
                 if (bj >= 0) last[bj] = l;
-                lvl[base + j] = l - 1;
-                levels = (l > levels) ? l : levels;
             }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (lane == j) mine = l - 1;
+            levels = (l > levels) ? l : levels;
         }
+        if (r < n) L.lvl[r] = mine;
     }
-    levels = __shfl(levels, 0);
     __syncthreads();
-    for (int k = lane; k <= levels; k += kWave) start[k] = 0;
+    for (int k = lane; k <= levels; k += kWave) L.start[k] = 0;
     __syncthreads();
-    for (int r = lane; r < n; r += kWave) atomicAdd(&start[lvl[r]], 1);
+    for (int r = lane; r < n; r += kWave) atomicAdd(&L.start[L.lvl[r]], 1);
     __syncthreads();
     {
         int carry = 0;
         for (int base = 0; base <= levels; base += kWave) {
             const int k = base + lane;
-            const int v = (k <= levels) ? start[k] : 0;
+            const int v = (k <= levels) ? L.start[k] : 0;
             const int incl = wave_incl_scan(v, lane);
-            if (k <= levels) start[k] = carry + incl - v;
+            if (k <= levels) L.start[k] = carry + incl - v;
             carry += __shfl(incl, kWave - 1);
         }
     }
     __syncthreads();
-    int* cur = reinterpret_cast<int*>(rb);
-    for (int k = lane; k < levels; k += kWave) cur[k] = start[k];
+    int* cur = reinterpret_cast<int*>(L.rb);
+    for (int k = lane; k < levels; k += kWave) cur[k] = L.start[k];
     __syncthreads();
-    for (int r = lane; r < n; r += kWave) order[atomicAdd(&cur[lvl[r]], 1)] = r;
+    for (int r = lane; r < n; r += kWave) L.order[atomicAdd(&cur[L.lvl[r]], 1)] = L.sel[r];
     __syncthreads();
     int rounds = 0;
     for (int base = 0; base < levels; base += kWave) {
         const int k = base + lane;
-        const int cnt = (k < levels) ? start[k + 1] - start[k] : 0;
+        const int cnt = (k < levels) ? L.start[k + 1] - L.start[k] : 0;
         const int nr = (cnt + kLevelRound - 1) / kLevelRound;
         const int incl = wave_incl_scan(nr, lane);
         for (int i = 0; i < nr; ++i) {
-            const int b = start[k] + i * kLevelRound;
-            const int e = (b + kLevelRound < start[k + 1]) ? b + kLevelRound : start[k + 1];
-            rb[rounds + incl - nr + i] = int2{b, e};
+            const int b = L.start[k] + i * kLevelRound;
+            const int e = (b + kLevelRound < L.start[k + 1]) ? b + kLevelRound : L.start[k + 1];
+            L.rb[rounds + incl - nr + i] = int2{b, e - b};
         }
         rounds += __shfl(incl, kWave - 1);
     }
-    float4* v2 = d.s_vc2 + (std::size_t(x.co) + std::size_t(c0)) * prx::kVcStride;
-    float4* p2 = d.s_pc2 + (std::size_t(x.co) + std::size_t(c0)) * prx::kPcStride;
-    for (int k = lane; k < n * prx::kVcStride; k += kWave) {
-        const int pos = k / prx::kVcStride, f = k - pos * prx::kVcStride;
-        v2[k] = vbase[std::size_t(order[pos]) * prx::kVcStride + f];
+    // Records in level order.
+    float4* v2 = d.s_vc2 + std::size_t(x.co) * prx::kQuadVc;
+    float4* p2 = d.s_pc2 + std::size_t(x.co) * prx::kQuadPc;
+    for (int pos = lane; pos < n; pos += kWave) {
+        const int slot = L.order[pos], is = L.island[slot];
+        BodyC A, B;
+        const Vc vc = load_vc(vbase + std::size_t(slot) * prx::kVcStride, A, B);
+        store_quad_vc(v2 + std::size_t(pos) * prx::kQuadVc, vc, A, B, x.nb, is);
+        // The moving bodies of the update (16 bits each), for the period.
+        L.lvl[pos] = ((A.invMass != 0.0f || A.invRotI != 0.0f) ? vc.bA : 0xffff) |
+                     (((B.invMass != 0.0f || B.invRotI != 0.0f) ? vc.bB : 0xffff) << 16);
+        store_quad_pc(p2 + std::size_t(pos) * prx::kQuadPc, load_pc(pbase + std::size_t(slot) * prx::kPcStride), is);
     }
-    for (int k = lane; k < n * prx::kPcStride; k += kWave) {
-        const int pos = k / prx::kPcStride, f = k - pos * prx::kPcStride;
-        p2[k] = pbase[std::size_t(order[pos]) * prx::kPcStride + f];
-    }
+    // Period: first round of each body, then the widest span of a body.
+    int* first = last;
+    for (int b = lane; b < x.nb; b += kWave) first[b] = rounds;
     __syncthreads();
-    if (lane == 0) lvl[0] = rounds;  // levels are no longer needed
-    __syncthreads();
-    return LevelPlan{n, rounds, rb, order};
-}
-
-__device__ __forceinline__ LevelPlan level_plan_of(const DeviceState& d, const WorldCtx& x, int c0, int c1) {
-    const int n = c1 - c0;
-    int* L = level_ints(d, x, c0);
-    return LevelPlan{n, L[0], level_rounds(L, n), L + n};
-}
-
-// Round bounds of a plan during its passes.  Round k covers level positions
-// [end(k - 1), end(k)) (rounds are contiguous).  The ends are staged in LDS
-// (the record stage is free while the passes run) when they fit in 16 bits
-// and in the stage, so that no round waits on a global load for its bounds;
-// otherwise they are read from the plan in global scratch.
-struct RoundEnds {
-    const unsigned short* lds;
-    const int2* rb;
-    int rounds;
-    __device__ __forceinline__ int end(int k) const { return lds ? int(lds[k]) : rb[k].y; }
-    __device__ __forceinline__ int2 round(int k) const {
-        return int2{k > 0 ? end(k - 1) : 0, end(k)};
-    }
-};
-
-__device__ __forceinline__ RoundEnds stage_round_ends(const LevelPlan& P, float4* stage, int lane) {
-    constexpr int kCap = prx::kStageFloat4 * 8;  // 16-bit ends in the stage
-    if (P.rounds > kCap || P.n > 0xffff) return RoundEnds{nullptr, P.rb, P.rounds};
-    unsigned short* e = reinterpret_cast<unsigned short*>(stage);
-    for (int k = lane; k < P.rounds; k += kWave) e[k] = static_cast<unsigned short>(P.rb[k].y);
-    __syncthreads();
-    return RoundEnds{e, P.rb, P.rounds};
-}
-
-// One pass of an island's level form.  Round k covers level positions
-// [end(k - 1), end(k)); its records are loaded while round k - 1 is solved,
-// and the end of round k + 1 is read while round k - 1 is solved, so that no
-// round waits on memory it did not ask for a round earlier.  The records are
-// read and the impulses written by buffer instructions that every lane
-// issues in every round, lanes without an update at an offset past the
-// buffer's end (no memory is touched for them): with no branch around them,
-// the waits the compiler places count exactly the operations in flight, so
-// a round's impulse stores retire while the next round runs.
-constexpr int kOutOfRange = 0x40000000;  // a buffer offset past every island's records
-
-template <int kStride, bool kLdsEnds>
-struct LevelRounds {
-    __amdgpu_buffer_rsrc_t rec;
-    const unsigned short* e16;
-    const int2* rb;
-    int n, rounds, lane;
-    __device__ __forceinline__ int end(int k) const {
-        if (k >= rounds) return n;
-        if constexpr (kLdsEnds) return int(e16[k]);
-        else return rb[k].y;
-    }
-    __device__ __forceinline__ void fetch(int start, int stop, float4 (&buf)[kStride]) const {
-        const int pos = start + (lane >> 1);
-        const int off = (pos < stop) ? pos * (kStride * 16) : kOutOfRange;
-#pragma unroll
-        for (int f = 0; f < kStride; ++f)
-            buf[f] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rec, off + 16 * f, 0, 0));
-    }
-    // Runs body(start, end, records) for every round, two rounds per trip
-    // (the two record buffers alternate without copies).
-    template <class F>
-    __device__ __forceinline__ void run(F&& body) const {
-        float4 a[kStride], b[kStride];
-        int s = 0;
-        int e = end(0);
-        fetch(0, e, a);
-        for (int k = 0; k < rounds; k += 2) {
-            const int e1 = end(k + 1);
-            fetch(e, e1, b);
-            body(s, e, a);
-            if (k + 1 >= rounds) break;
-            const int e2 = end(k + 2);
-            fetch(e1, e2, a);
-            body(e, e1, b);
-            s = e1;
-            e = e2;
+    auto bodies_of = [&](auto&& f) {
+        for (int k = lane; k < rounds; k += kWave) {
+            const int2 r = L.rb[k];
+            for (int pos = r.x; pos < r.x + r.y; ++pos) {
+                const int ab = L.lvl[pos];
+                if ((ab & 0xffff) != 0xffff) f(k, ab & 0xffff);
+                if (((ab >> 16) & 0xffff) != 0xffff) f(k, (ab >> 16) & 0xffff);
+            }
         }
-    }
-};
+    };
+    bodies_of([&](int k, int b) { atomicMin(&first[b], k); });
+    __syncthreads();
+    int period = 1;
+    bodies_of([&](int k, int b) { period = max(period, k - first[b] + 1); });
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) period = max(period, __shfl_xor(period, off));
+    // A group ends an iteration before it starts its next, and a record's
+    // impulses are stored before the next iteration reads them.
+    period = max(period, max((rounds + kLevelGroups - 1) / kLevelGroups, 2));
+    __syncthreads();
+    return LevelPlan{n, __builtin_amdgcn_readfirstlane(rounds), __builtin_amdgcn_readfirstlane(period), L.rb, L.order};
+}
+
+constexpr int kOutOfRange = 0x40000000;  // a buffer offset past every island's records
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t record_rsrc(const float4* base, int n, int stride) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float4*>(base), 0, n * stride * 16, 0x00020000);
 }
 
+// Bounds of a round (first position, updates), read by buffer loads as well
+// and two rounds ahead: a lane without a round reads past the end and gets
+// none.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rounds_rsrc(const LevelPlan& P) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<int2*>(P.rb), 0, P.rounds * int(sizeof(int2)), 0x00020000);
+}
+
 using U4 = __attribute__((ext_vector_type(4))) unsigned;
 
-template <bool kWarm, bool kLdsEnds, bool kLds>
-__device__ __forceinline__ float velocity_level_pass(const LevelRounds<prx::kVcStride, kLdsEnds>& R,
-                                                     const Bodies<kLds>& bs) {
-    float newInc = 0.0f;
-    const int side = R.lane & 1;
-    R.run([&](int s, int e, float4 (&cur)[prx::kVcStride]) {
-        const int pos = s + (R.lane >> 1);
-        const bool act = pos < e;
-        float4 o4 = cur[4], o7 = cur[7];
-        if (act) {
-            BodyC A, B;
-            Vc vc = load_vc(cur, A, B);
+// Exchanges within an update's four lanes (2 s + c).
+template <int kPerm>
+__device__ __forceinline__ float quad_move(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), kPerm, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float other_comp(float v) { return quad_move<0xB1>(v); }  // lanes 1 0 3 2
+__device__ __forceinline__ float other_body(float v) { return quad_move<0x4E>(v); }  // lanes 2 3 0 1
+__device__ __forceinline__ float from_b(float v) { return quad_move<0xEE>(v); }      // lanes 2 3 2 3
+
+// A velocity record as a lane holds it.
+struct QuadRec {
+    float2 q;    // this lane's arm components, points 0 and 1
+    float4 s;    // this body's -+ masses, velocity index
+    float2 tn;   // tangent and normal component
+    float4 f, b, k, m, i;
+};
+
+// The update's arithmetic is that of solve_dir and block_solve, operation for
+// operation and in their order, spread over four lanes: a lane holds one
+// velocity component and the spin of one body.  Products with a component
+// and its arm are formed lane by lane and summed across the two components
+// (the two orders of a two-term sum give the same bits); the relative
+// velocity and the impulses are formed on body B's lanes and the impulse
+// changes handed to body A's, whose masses carry the minus sign (a - b c and
+// a + (-b) c round alike).
+struct QuadBody {
+    float v, w;       // velocity component, spin
+    float sm, si;     // -+ inverse mass, inertia
+    __device__ __forceinline__ void apply(float P, float L) {
+        v = v + sm * P;
+        w = w + si * L;
+    }
+};
+// Normal or tangential relative velocity on body B's lanes.
+__device__ __forceinline__ float quad_closing(const QuadBody& me, float q, float dir) {
+    const float u = me.v + q * me.w;
+    const float m = (u - other_body(u)) * dir;
+    return (0.0f + m) + other_comp(m);
+}
+__device__ __forceinline__ float quad_arm(float q, float P) {
+    const float m = q * P;
+    return m + other_comp(m);
+}
+__device__ __forceinline__ void quad_tangent(QuadBody& me, const QuadRec& r, float q, float tm, float ni, float& ti,
+                                             float& maxInc) {
+    const float lambda = tm * (r.f.y - quad_closing(me, q, r.tn.x));
+    const float maxI = r.f.x * ni;
+    const float inc = from_b(clamp_std(ti + lambda, -maxI, maxI) - ti);
+    const float P = inc * r.tn.x;
+    me.apply(P, quad_arm(q, P));
+    maxInc = fmax_std(maxInc, __builtin_fabsf(inc));
+    ti = ti + inc;
+}
+__device__ __forceinline__ void quad_normal(QuadBody& me, const QuadRec& r, float q, float nm, float bias, float& ni,
+                                            float& maxInc) {
+    const float lambda = nm * (bias - quad_closing(me, q, r.tn.y));
+    const float inc = from_b(fmax_std(ni + lambda, 0.0f) - ni);
+    const float P = inc * r.tn.y;
+    me.apply(P, quad_arm(q, P));
+    maxInc = fmax_std(maxInc, __builtin_fabsf(inc));
+    ni = ni + inc;
+}
+__device__ __forceinline__ void quad_block(QuadBody& me, const QuadRec& r, int lane, float& ni0, float& ni1, float& maxInc) {
+    const float vn0 = quad_closing(me, r.q.x, r.tn.y);
+    const float vn1 = quad_closing(me, r.q.y, r.tn.y);
+    float t0 = 0.0f;
+    t0 += r.k.x * ni0;
+    t0 += r.k.z * ni1;
+    float t1 = 0.0f;
+    t1 += r.k.z * ni0;
+    t1 += r.k.y * ni1;
+    const float bx = (vn0 - r.b.x) - t0, by = (vn1 - r.b.y) - t1;
+    float x0 = 0.0f;
+    x0 += r.m.x * bx;
+    x0 += r.m.z * by;
+    float x1 = 0.0f;
+    x1 += r.m.z * bx;
+    x1 += r.m.y * by;
+    const float c1n0 = -x0, c1n1 = -x1;
+    const bool ok1 = c1n0 >= 0.0f && c1n1 >= 0.0f;
+    const float c2n0 = -r.b.z * bx;
+    const bool ok2 = c2n0 >= 0.0f && r.k.z * c2n0 + by >= 0.0f;
+    const float c3n1 = -r.b.w * by;
+    const bool ok3 = c3n1 >= 0.0f && r.k.z * c3n1 + bx >= 0.0f;
+    const bool ok4 = bx >= 0.0f && by >= 0.0f;
+    const float n0 = ok1 ? c1n0 : (ok2 ? c2n0 : 0.0f);
+    const float n1 = ok1 ? c1n1 : (ok2 ? 0.0f : (ok3 ? c3n1 : 0.0f));
+    const float d0 = from_b(n0 - ni0), d1 = from_b(n1 - ni1);
+    const float P0 = d0 * r.tn.y, P1 = d1 * r.tn.y;
+    QuadBody next = me;
+    next.apply(P0 + P1, quad_arm(r.q.x, P0) + quad_arm(r.q.y, P1));
+    // With no valid case (on body B's lanes) everything stays as it is.
+    const unsigned long long none = __ballot(!(ok1 || ok2 || ok3 || ok4));
+    if ((none >> (lane | 2)) & 1) return;
+    me = next;
+    ni0 = n0;
+    ni1 = n1;
+    maxInc = fmax_std(maxInc, fmax_std(__builtin_fabsf(n0), __builtin_fabsf(n1)));
+}
+
+// Iterations [0, iters) of the plan's velocity sweep, overlapped as its period
+// allows (one iteration: a plain pass).  Lane 32 g + 4 j + 2 s + c serves
+// update j of group g's round; group g runs iterations g, g + 2, ...  Bound by
+// the instructions of one round after another, about 2000 cycles each (no other
+// wave of the world can help): a pile of 400 bodies takes 2.2M cycles for the
+// velocity sweeps and 1.2M for the position sweeps, from 3.1M and 1.8M with
+// two lanes an update, one iteration after another.  A round's records are
+// read while the round before is solved, and its bounds one round earlier
+// still.  The records are read and the impulses written by buffer
+// instructions that every lane issues in every round, lanes without an update
+// at an offset past the buffer's end (no memory is touched for them): with no
+// branch around them, and one address space for the bounds, the waits the
+// compiler places count exactly the operations in flight.  Islands marked in
+// their words are left out of a masked run.
+enum LevelPass { kPassWarm, kPassWarmMasked, kPassIterations, kPassMasked };
+template <LevelPass kPass>
+__device__ __forceinline__ void velocity_level_run(const __amdgpu_buffer_rsrc_t rec, const LevelPlan& P, int iters,
+                                                   int* words, int lane) {
+    const __amdgpu_buffer_rsrc_t table = rounds_rsrc(P);
+    constexpr bool kWarm = kPass == kPassWarm || kPass == kPassWarmMasked;
+    constexpr bool kMasked = kPass == kPassMasked || kPass == kPassWarmMasked;
+    float* const lds = reinterpret_cast<float*>(g_smem);
+    const int group = lane >> 5, j = (lane >> 2) & (kLevelRound - 1), quad = lane & 3, comp = lane & 1;
+    constexpr int kStep = prx::kQuadVc * 16;
+    const int rounds = P.rounds, period = P.period;
+    int r = -group * period, it = group;  // the group's round and iteration at the tick read ahead
+    struct At {
+        int2 b;
+        int it, off;
+    };
+    auto bounds = [&](At& a) {
+        const bool on = r >= 0 && it < iters;
+        a.b = __builtin_bit_cast(int2, __builtin_amdgcn_raw_buffer_load_b64(table, on ? r * 8 : kOutOfRange, 0, 0));
+        a.it = it;
+        if (++r == kLevelGroups * period) {
+            r = 0;
+            it += kLevelGroups;
+        }
+    };
+    auto f2 = [&](int off) {
+        return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rec, off, 0, 0));
+    };
+    auto f4 = [&](int off) {
+        return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rec, off, 0, 0));
+    };
+    auto fetch = [&](At& a, QuadRec& q) {
+        const int off = a.off = j < a.b.y ? (a.b.x + j) * kStep : kOutOfRange;
+        q.q = f2(off + 8 * quad);
+        q.s = f4(off + 32 + 8 * (quad & 2));
+        q.tn = f2(off + 64 + 8 * comp);
+        if constexpr (!kWarm) {
+            q.f = f4(off + 80);
+            q.b = f4(off + 96);
+            q.m = f4(off + 128);
+        }
+        q.k = f4(off + 112);
+        q.i = f4(off + 144);
+    };
+    auto solve = [&](const At& at, QuadRec& q) {
+        const int island = int(__float_as_uint(q.k.w) >> 8);
+        bool on = at.off != kOutOfRange;
+        if constexpr (kMasked) on = on && words[2 * island] >= 0;
+        if (on) {
+            const unsigned n = __float_as_uint(q.k.w) & 0xffu;
+            const int vi = __float_as_int(q.s.z);
+            QuadBody me{lds[vi + comp], lds[vi + 2], q.s.x, q.s.y};
             if constexpr (kWarm) {
-                warm_start_pair(vc, A, B, bs, side);
+                QuadBody dl{0.0f, 0.0f, q.s.x, q.s.y};
+                if (n > 0) {
+                    const float Pn = q.i.x * q.tn.y + q.i.y * q.tn.x;
+                    dl.apply(Pn, quad_arm(q.q.x, Pn));
+                }
+                if (n > 1) {
+                    const float Pn = q.i.z * q.tn.y + q.i.w * q.tn.x;
+                    dl.apply(Pn, quad_arm(q.q.y, Pn));
+                }
+                me.v = me.v + dl.v;
+                me.w = me.w + dl.w;
             } else {
-                const float mi = solve_velocity_pair(vc, A, B, bs, side);
-                o4 = float4{vc.p[0].ni, vc.p[0].ti, vc.p[0].nm, vc.p[0].tm};
-                o7 = float4{vc.p[1].ni, vc.p[1].ti, vc.p[1].nm, vc.p[1].tm};
-                newInc = fmax_std(newInc, mi);
+                float inc = 0.0f;
+                if (n > 1) quad_tangent(me, q, q.q.y, q.f.w, q.i.z, q.i.w, inc);
+                if (n > 0) quad_tangent(me, q, q.q.x, q.f.z, q.i.x, q.i.y, inc);
+                if (n == 1 || (q.k.x == 0.0f && q.k.y == 0.0f && q.k.z == 0.0f)) {
+                    if (n > 1) quad_normal(me, q, q.q.y, q.b.w, q.b.y, q.i.z, inc);
+                    if (n > 0) quad_normal(me, q, q.q.x, q.b.z, q.b.x, q.i.x, inc);
+                } else {
+                    quad_block(me, q, lane, q.i.x, q.i.z, inc);
+                }
+                if (quad == 2 && inc > 0.0f) {
+                    atomicOr(&words[2 * island], 1 << at.it);
+                    atomicMax(&words[2 * island + 1], __float_as_int(inc));
+                }
             }
+            lds[vi + comp] = me.v;
+            lds[vi + 2] = me.w;
         }
         if constexpr (!kWarm) {
-            // The pair's lanes hold the same impulses: the body-A lane stores.
-            const int off = (act && side == 0) ? pos * (prx::kVcStride * 16) : kOutOfRange;
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, o4), R.rec, off + 64, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, o7), R.rec, off + 112, 0, 0);
+            // Body B's first lane holds the impulses and stores them.
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, q.i), rec,
+                                                   (on && quad == 2 ? at.off : kOutOfRange) + 144, 0, 0);
         }
-        __syncthreads();
-    });
-    return newInc;
-}
-
-// Warm start and velocity sweeps of one island in level form.
-template <bool kLdsEnds, bool kLds>
-__device__ __forceinline__ VelResult island_velocity_level_run(const DeviceState& d, const WorldCtx& x,
-                                                               const Bodies<kLds>& bs, const LevelPlan& P,
-                                                               int rounds, const unsigned short* e16, int c0,
-                                                               const StepParams& c) {
-    VelResult res{0.0f, int(c.velIters)};
-    float4* vbase = d.s_vc + (std::size_t(x.co) + std::size_t(c0)) * prx::kVcStride;
-    float4* v2 = d.s_vc2 + (std::size_t(x.co) + std::size_t(c0)) * prx::kVcStride;
-    const LevelRounds<prx::kVcStride, kLdsEnds> R{record_rsrc(v2, P.n, prx::kVcStride), e16, P.rb, P.n, rounds,
-                                                  x.lane};
-    if (c.warmStart) velocity_level_pass<true, kLdsEnds, kLds>(R, bs);
-    for (int it = 0; it < int(c.velIters); ++it) {
-        float newInc = velocity_level_pass<false, kLdsEnds, kLds>(R, bs);
-#pragma unroll
-        for (int off = kWave / 2; off > 0; off >>= 1) newInc = fmax_std(newInc, __shfl_xor(newInc, off));
-        res.maxInc = fmax_std(res.maxInc, newInc);
-        if (newInc <= c.regMinMomentum) {
-            res.iters = it + 1;
-            break;
-        }
+        // The wave's LDS operations run in order: nothing to wait for.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    const int ticks = rounds + (iters - 1) * period;
+    QuadRec a, b;
+    At atA, atB, atC;
+    bounds(atA);
+    bounds(atB);
+    fetch(atA, a);
+    // Two rounds a trip, the two record buffers alternating without copies (a
+    // last round past the end serves no lane).  s_waitcnt vmcnt(0) (expcnt and
+    // lgkmcnt at their maxima) before the first: with loads in flight on
+    // entry, or on a way out of the middle, the compiler waits for them at the
+    // head of every trip.
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    for (int t = 0; t < ticks; t += 2) {
+        bounds(atC);
+        fetch(atB, b);
+        solve(atA, a);
+        bounds(atA);
+        fetch(atC, a);
+        solve(atB, b);
+        atB = atA;
+        atA = atC;
     }
-    // The passes' stores complete before other lanes read the records back:
+    // The run's stores complete before other lanes read the records back:
     // s_waitcnt vmcnt(0) (expcnt and lgkmcnt at their maxima).
     __builtin_amdgcn_s_waitcnt(0x0F70);
-    for (int pos = x.lane; pos < P.n; pos += kWave) {
-        float4* dst = vbase + std::size_t(P.order[pos]) * prx::kVcStride;
-        const float4* src = v2 + std::size_t(pos) * prx::kVcStride;
-        dst[4] = src[4];
-        dst[7] = src[7];
-    }
-    __syncthreads();
-    return res;
 }
 
-template <bool kLds>
-__device__ __forceinline__ VelResult island_velocity_level(const DeviceState& d, const WorldCtx& x,
-                                                           const Bodies<kLds>& bs, const LevelPlan& P, int c0,
-                                                           const StepParams& c, float4* stage) {
-    const RoundEnds R = stage_round_ends(P, stage, x.lane);
-    const int rounds = __builtin_amdgcn_readfirstlane(P.rounds);
-    if (R.lds) return island_velocity_level_run<true, kLds>(d, x, bs, P, rounds, R.lds, c0, c);
-    return island_velocity_level_run<false, kLds>(d, x, bs, P, rounds, nullptr, c0, c);
+// A position record as a lane holds it: this body, its points, the common part.
+struct QuadPos {
+    float4 b, u, v, k;
+};
+
+// almost_equal in closed form: at most four steps to the neighbouring float
+// lie between the two (+0 and -0 are one place), and neither is a NaN.
+__device__ __forceinline__ bool almost_equal_steps(float a, float b) {
+    const int x = __float_as_int(a), y = __float_as_int(b);
+    const int kx = x >= 0 ? x : int(0x80000000u) - x, ky = y >= 0 ? y : int(0x80000000u) - y;
+    return unsigned(kx - ky + 4) <= 8u && !__builtin_isunordered(a, b);
 }
 
-// Position sweeps of one island in level form; returns whether solved.
-template <bool kLdsEnds, bool kLds>
-__device__ __forceinline__ PosResult island_position_level_run(const DeviceState& d, const WorldCtx& x,
-                                                               const Bodies<kLds>& bs, const LevelPlan& P,
-                                                               int rounds, const unsigned short* e16, int c0,
-                                                               const StepParams& c) {
-    const float4* p2 = d.s_pc2 + (std::size_t(x.co) + std::size_t(c0)) * prx::kPcStride;
-    const LevelRounds<prx::kPcStride, kLdsEnds> R{record_rsrc(p2, P.n, prx::kPcStride), e16, P.rb, P.n, rounds,
-                                                  x.lane};
-    PosResult res{__builtin_inff(), 0};
-    for (std::uint32_t it = 0; it < c.posIters; ++it) {
-        float minSep = __builtin_inff();
-        const int side = x.lane & 1;
-        R.run([&](int s, int e, float4 (&cur)[prx::kPcStride]) {
-            if (s + (x.lane >> 1) < e) {
-                const Pc pc = load_pc(cur);
-                const int mine = side ? pc.bB : pc.bA;
-                float4 p = bs.pos(mine);
-                const float sep = solve_pc_pair(pc.m, pc.totalRadius, pc.A, pc.B, p, side, c);
-                bs.set_pos(mine, p);
-                minSep = fmin_std(minSep, sep);
+// GaussSeidel::SolvePositionConstraint (ContactSolver.cpp:494-643), the
+// arithmetic of solve_pc and get_psm operation for operation: each lane
+// computes one component of its own body's transformation and point; the
+// points' difference, the separation and a circles' normal are formed on Y's
+// lanes, a face's normal on X's, and handed to the other body's.  p, a: the
+// lane's position component and angle, updated; returns the separation, or
+// infinity where nothing is solved.
+__device__ __forceinline__ float quad_position(const QuadPos& r, int quad, float& p, float& a, const StepParams& c) {
+    const bool compY = quad & 1, bodyY = quad & 2;
+    const std::uint32_t h = __float_as_uint(r.k.z);
+    const std::uint32_t type = h & 0xffu, n = (h >> 8) & 0xffu;
+    const bool faceB = type == kFaceB, circles = type == kCircles;
+    const bool isA = __float_as_int(r.b.y) < 0;  // -0 for a massless A
+    // Signed exchange for cross products: cross(r, v) = rx vy + -(ry vx).
+    auto turned = [&](float v) {
+        const float o = other_comp(v);
+        return compY ? -o : o;
+    };
+    auto cross2 = [&](float x, float vTurned) {
+        const float m = x * vTurned;
+        return m + other_comp(m);
+    };
+    struct Frame {
+        float q, qs, o;  // rotation component, the other one signed, origin
+    };
+    auto frame = [&](float pc, float ang) {
+        const V2 q = unit_from_angle(ang);
+        Frame f;
+        f.q = compY ? q.y : q.x;
+        f.qs = compY ? q.x : -q.y;
+        f.o = pc - (f.q * r.u.x + f.qs * r.u.y);
+        return f;
+    };
+    auto rotated = [](const Frame& f, float x, float y) { return f.q * x + f.qs * y; };
+    struct Psm {
+        float n, nt, pt, sep;  // normal component, turned, point, separation
+    };
+    auto face_normal = [&](const Frame& f) { return quad_move<0x44>(rotated(f, r.v.z, r.v.w)); };  // from X: lanes 0 1 0 1
+    auto psm = [&](const Frame& f, float lx, float ly, float faceN) {
+        const float at = rotated(f, lx, ly) + f.o;  // X's or Y's point
+        const float ot = other_body(at);
+        const float delta = at - ot;  // Y's lanes: Y - X
+        float nrm = faceN;
+        if (circles) {
+            const float m = delta * delta;
+            const float m2 = m + other_comp(m);
+            float u;
+            if (__builtin_isnormal(m2)) {
+                u = delta * (1.0f / __builtin_sqrtf(m2));
+            } else {
+                const float mag = hypot_f(delta, other_comp(delta));
+                u = __builtin_isnormal(mag) ? delta / mag : 0.0f;
             }
-            __syncthreads();
-        });
-#pragma unroll
-        for (int off = kWave / 2; off > 0; off >>= 1) minSep = fmin_std(minSep, __shfl_xor(minSep, off));
-        res.minSep = fmin_std(res.minSep, minSep);
-        if (minSep >= c.regMinSeparation) {
-            res.solvedAt = int(it) + 1;
-            return res;
+            nrm = from_b(u);
         }
+        const float m = delta * nrm;
+        Psm s;
+        s.sep = from_b((0.0f + m) + other_comp(m));
+        s.pt = circles ? (at + ot) * 0.5f : (bodyY ? at : ot);
+        s.n = faceB ? -nrm : nrm;
+        s.nt = turned(s.n);
+        return s;
+    };
+    struct Sol {
+        float dl, da, sep;
+    };
+    auto solve = [&](const Psm& s, float pc) {
+        const float separation = s.sep - r.k.x;
+        const float arm = s.pt - pc;
+        const float cr = cross2(arm, s.nt);
+        const float t = __builtin_fabsf(r.b.z) * (cr * cr);
+        const float to = other_body(t);
+        const float K = r.k.y + (isA ? t : to) + (isA ? to : t);
+        const float C = -clamp_std(c.regResolutionRate * (separation + c.linearSlop), -c.maxLinearCorrection, 0.0f);
+        const float P = (s.n * C) * (1.0f / K);
+        const float L = cross2(arm, turned(P));
+        return Sol{r.b.y * P, r.b.z * L, separation};
+    };
+    const float op = p, oa = a;
+    const Frame f = frame(op, oa);
+    const float fn = face_normal(f);
+    const Psm psm0 = psm(f, r.u.z, r.u.w, fn);
+    Psm psm1 = psm0;
+    const bool two = n == 2;
+    bool eq = false, lt = false, gt = false;
+    if (two) {
+        psm1 = psm(f, r.v.x, r.v.y, fn);
+        eq = almost_equal_steps(psm0.sep, psm1.sep);
+        lt = !eq && psm0.sep < psm1.sep;
+        gt = !eq && psm1.sep < psm0.sep;
     }
-    return res;
+    if (!(n == 1 || eq || lt || gt)) return __builtin_inff();
+    const Sol s0 = solve(gt ? psm1 : psm0, op);
+    p = op + s0.dl;
+    a = oa + s0.da;
+    if (two) {
+        const Frame g = frame(p, a);
+        const Psm next = psm(g, gt ? r.u.z : r.v.x, gt ? r.u.w : r.v.y, face_normal(g));
+        const Sol s1 = solve(eq ? psm1 : next, eq ? op : p);
+        p = p + s1.dl;
+        a = a + s1.da;
+        return s0.sep;
+    }
+    return 0.0f + s0.sep;
 }
 
-template <bool kLds>
-__device__ __forceinline__ PosResult island_position_level(const DeviceState& d, const WorldCtx& x, const Bodies<kLds>& bs,
-                                                      const LevelPlan& P, int c0, const StepParams& c,
-                                                      float4* stage) {
-    const RoundEnds R = stage_round_ends(P, stage, x.lane);
-    const int rounds = __builtin_amdgcn_readfirstlane(P.rounds);
-    if (R.lds) return island_position_level_run<true, kLds>(d, x, bs, P, rounds, R.lds, c0, c);
-    return island_position_level_run<false, kLds>(d, x, bs, P, rounds, nullptr, c0, c);
+// Order-preserving integer images of floats, for minima.
+__device__ __forceinline__ int float_key(float f) {
+    const int bits = __float_as_int(f);
+    return bits >= 0 ? bits : (bits ^ 0x7fffffff);
 }
+__device__ __forceinline__ float key_float(int key) { return __int_as_float(key >= 0 ? key : (key ^ 0x7fffffff)); }
 
-__device__ __forceinline__ bool level_form(const WorldCtx& x, int c0, int c1, int j0, int j1) {
-    return j0 == j1 && x.nb <= kLevelMaxBodies && (c1 - c0) >= kLevelMinConstraints;
+// The islands of a world that the level form sweeps: without joints, at least
+// kLevelMinConstraints contacts (or coopMin, if that is less; coopMin's
+// greatest value keeps every island on a lane).
+__device__ __forceinline__ bool level_island(int contacts, int joints, int coopMin) {
+    return joints == 0 && contacts >= (coopMin < kLevelMinConstraints ? coopMin : kLevelMinConstraints) &&
+           coopMin != 0x7fffffff;
 }
 
 // What the island solves add to RegStepStats (Update(RegStepStats&,
@@ -4300,6 +4361,221 @@ struct SolveSummary {
     std::uint32_t slept, solved, sumPos, sumVel;
     float minSep, maxInc;
 };
+
+// Warm start and velocity sweeps of the level islands.
+//
+// Overlapped iterations run past an island's early exit.  The exit's bound is
+// zero unless set otherwise: an island exits with the first iteration in which
+// no impulse changed (its bit in the island's word stays clear).  Such an
+// island is swept again from its starting velocities and impulses: the early
+// exit is what makes that short, so one below kLevelRedo contacts goes to its
+// lane, a larger one through plain iterations.  With a positive bound all
+// level islands take plain iterations, with a negative one none exits.
+constexpr int kLevelRedo = 32;
+template <class Level, class Add>
+__device__ __forceinline__ void velocity_levels(const DeviceState& d, const WorldCtx& x, const Bodies<true>& bs,
+                                                const IslandScratch& S, const LevelPlan& P, int nisl, Level level,
+                                                const StepParams& c, Add add) {
+    float4* v2 = d.s_vc2 + std::size_t(x.co) * prx::kQuadVc;
+    float4* vbase = d.s_vc + std::size_t(x.co) * prx::kVcStride;
+    const __amdgpu_buffer_rsrc_t rec = record_rsrc(v2, P.n, prx::kQuadVc);
+    const LevelScratch L(d, x);
+    int* const words = island_words(x);
+    constexpr int kOut = int(0x80000000u);  // left out of masked runs
+    const int iters = int(c.velIters);
+    const bool overlap = c.regMinMomentum <= 0.0f && iters <= 31;
+    for (int is = x.lane; is < nisl; is += kWave) {
+        words[2 * is] = 0;
+        words[2 * is + 1] = 0;
+    }
+    __syncthreads();
+    if (c.warmStart) velocity_level_run<kPassWarm>(rec, P, 1, words, x.lane);
+    if (overlap && iters > 0) {
+        velocity_level_run<kPassIterations>(rec, P, iters, words, x.lane);
+        __syncthreads();
+    }
+    // Islands to sweep again, on their lane or by plain iterations.
+    bool anyPlain = false, anyLane = false;
+    for (int base = 0; base < nisl; base += kWave) {
+        const int is = base + x.lane;
+        bool lane = false, plain = false;
+        if (is < nisl && level(is)) {
+            const int ran = (1 << (iters & 31)) - 1;
+            const bool exits = overlap && c.regMinMomentum == 0.0f && iters > 1 && ((words[2 * is] | (1 << (iters - 1))) & ran) != ran;
+            plain = !overlap;
+            if (exits) {
+                lane = S.istart[is + 1].y - S.istart[is].y < kLevelRedo;
+                plain = !lane;
+            } else if (overlap) {
+                add(VelResult{__int_as_float(words[2 * is + 1]), iters});
+            }
+            words[2 * is] = lane ? 1 : (plain ? 0 : kOut);
+            if (exits)
+                for (int e = S.istart[is].x; e < S.istart[is + 1].x; ++e)
+                    bs.set_vel(S.ibody[e], integrated_velocity(d, x.bo + S.ibody[e], c));
+        }
+        anyLane = anyLane || __ballot(lane) != 0;
+        anyPlain = anyPlain || __ballot(plain) != 0;
+    }
+    __syncthreads();
+    // Impulses back into island order; a lane's islands keep their own.
+    auto impulses_back = [&] {
+        for (int pos = x.lane; pos < P.n; pos += kWave) {
+            const int slot = P.order[pos];
+            if (words[2 * L.island[slot]] == 1) continue;
+            float4* dst = vbase + std::size_t(slot) * prx::kVcStride;
+            const float4 i = v2[std::size_t(pos) * prx::kQuadVc + 9];
+            dst[4].x = i.x;
+            dst[4].y = i.y;
+            dst[7].x = i.z;
+            dst[7].y = i.w;
+        }
+    };
+    if (anyPlain) {
+        if (overlap) {
+            // From the impulses the sweep started with (warm-started again).
+            for (int pos = x.lane; pos < P.n; pos += kWave) {
+                const int slot = P.order[pos];
+                if (words[2 * L.island[slot]] != 0) continue;
+                const float4* src = vbase + std::size_t(slot) * prx::kVcStride;
+                v2[std::size_t(pos) * prx::kQuadVc + 9] = float4{src[4].x, src[4].y, src[7].x, src[7].y};
+            }
+            __syncthreads();
+            if (c.warmStart) {
+                for (int is = x.lane; is < nisl; is += kWave)
+                    if (words[2 * is] == 1) words[2 * is] = kOut | 1;
+                __syncthreads();
+                velocity_level_run<kPassWarmMasked>(rec, P, 1, words, x.lane);
+            }
+        }
+        for (int is = x.lane; is < nisl; is += kWave)
+            if (words[2 * is] == 1) words[2 * is] = kOut | 1;
+        for (int it = 0; it < iters; ++it) {
+            for (int is = x.lane; is < nisl; is += kWave) words[2 * is + 1] = 0;
+            __syncthreads();
+            velocity_level_run<kPassMasked>(rec, P, 1, words, x.lane);
+            __syncthreads();
+            bool going = false;
+            for (int base = 0; base < nisl; base += kWave) {
+                const int is = base + x.lane;
+                bool on = is < nisl && level(is) && words[2 * is] >= 0;
+                if (on) {
+                    // The island's sums so far: its largest change in stat words.
+                    const float inc = __int_as_float(words[2 * is + 1]);
+                    const bool done = inc <= c.regMinMomentum || it + 1 == iters;
+                    add(VelResult{inc, done ? it + 1 : 0});
+                    words[2 * is] = done ? kOut : 0;
+                    on = !done;
+                }
+                going = going || __ballot(on) != 0;
+            }
+            __syncthreads();
+            if (!going) break;
+        }
+        for (int is = x.lane; is < nisl; is += kWave) words[2 * is] = words[2 * is] == (kOut | 1) ? 1 : words[2 * is];
+        __syncthreads();
+    }
+    impulses_back();
+    if (anyLane) {
+        for (int is = x.lane; is < nisl; is += kWave)
+            if (level(is) && words[2 * is] == 1)
+                add(island_velocity<true>(d, x, bs, S.istart[is].y, S.istart[is + 1].y, 0, 0, c));
+    }
+    __syncthreads();
+}
+
+// Position sweeps of the level islands, iteration after iteration; an island
+// solved by an iteration is left out of the later ones.
+template <class Level, class Add>
+__device__ __forceinline__ void position_levels(const DeviceState& d, const WorldCtx& x, const Bodies<true>& bs,
+                                                const IslandScratch& S, const LevelPlan& P, int nisl, Level level,
+                                                const StepParams& c, Add add) {
+    const int iters = int(c.posIters);
+    if (iters == 0) {
+        for (int is = x.lane; is < nisl; is += kWave) {
+            if (!level(is)) continue;
+            S.isl_word[is] = 0u;
+            add(PosResult{__builtin_inff(), 0}, true);
+        }
+        return;
+    }
+    const __amdgpu_buffer_rsrc_t table = rounds_rsrc(P);
+    const __amdgpu_buffer_rsrc_t rec = record_rsrc(d.s_pc2 + std::size_t(x.co) * prx::kQuadPc, P.n, prx::kQuadPc);
+    float* const lds = reinterpret_cast<float*>(g_smem);
+    int* const words = island_words(x);
+    const int j = x.lane >> 2, quad = x.lane & 3, comp = x.lane & 1;
+    constexpr int kStep = prx::kQuadPc * 16;
+    struct At {
+        int2 b;
+        int off;
+    };
+    auto bounds = [&](int k, At& a) {
+        a.b = __builtin_bit_cast(int2, __builtin_amdgcn_raw_buffer_load_b64(table, k * 8, 0, 0));
+    };
+    auto f4 = [&](int off) {
+        return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rec, off, 0, 0));
+    };
+    auto fetch = [&](At& a, QuadPos& q) {
+        const int off = a.off = j < a.b.y ? (a.b.x + j) * kStep : kOutOfRange;
+        q.b = f4(off + 8 * (quad & 2));
+        q.u = f4(off + 32 + 16 * (quad & 2));
+        q.v = f4(off + 48 + 16 * (quad & 2));
+        q.k = f4(off + 96);
+    };
+    auto solve = [&](int off, const QuadPos& q) {
+        const int island = int(__float_as_uint(q.k.z) >> 16);
+        if (off != kOutOfRange && words[2 * island + 1] == 0) {
+            const int at = __float_as_int(q.b.x);
+            float p = lds[at + comp], a = lds[at + 2];
+            const float sep = quad_position(q, quad, p, a, c);
+            lds[at + comp] = p;
+            lds[at + 2] = a;
+            if (quad == 0 && sep < __builtin_inff()) atomicMin(&words[2 * island], float_key(sep));
+        }
+        // The wave's LDS operations run in order: nothing to wait for.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    for (int is = x.lane; is < nisl; is += kWave) words[2 * is + 1] = level(is) ? 0 : 1;
+    for (int it = 0; it < iters; ++it) {
+        for (int is = x.lane; is < nisl; is += kWave) words[2 * is] = 0x7f800000;  // key of +infinity
+        __syncthreads();
+        // A round's records are read while the round before is solved, and
+        // its bounds one round earlier still.
+        QuadPos a, b;
+        At atA, atB, atC;
+        bounds(0, atA);
+        bounds(1, atB);
+        fetch(atA, a);
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // as in the velocity sweep
+        for (int k = 0; k < P.rounds; k += 2) {
+            bounds(k + 2, atC);
+            fetch(atB, b);
+            solve(atA.off, a);
+            bounds(k + 3, atA);
+            fetch(atC, a);
+            solve(atB.off, b);
+            atB = atA;
+            atA = atC;
+        }
+        __syncthreads();
+        bool going = false;
+        for (int base = 0; base < nisl; base += kWave) {
+            const int is = base + x.lane;
+            bool on = is < nisl && words[2 * is + 1] == 0;
+            if (on) {
+                const float minSep = key_float(words[2 * is]);
+                const bool solved = minSep >= c.regMinSeparation;
+                if (solved) words[2 * is + 1] = it + 1;
+                on = !solved && it + 1 < iters;
+                if (!on) S.isl_word[is] = solved ? std::uint32_t(it + 1) : 0u;
+                add(PosResult{minSep, solved ? it + 1 : 0}, !on);
+            }
+            going = going || __ballot(on) != 0;
+        }
+        __syncthreads();
+        if (!going) break;
+    }
+}
 
 template <bool kLds, bool kTape = false>
 __device__ __forceinline__ SolveSummary solve_islands(const DeviceState& d, const WorldCtx& x, int nisl,
@@ -4424,32 +4700,50 @@ __device__ __forceinline__ SolveSummary solve_islands(const DeviceState& d, cons
     }
     __syncthreads();
     T.mark(prx::kPhConstraints);
-    // Warm start and velocity sweeps: islands below coopMin contacts one lane
-    // each, larger ones by the whole wave, one after another.
+    // Warm start and velocity sweeps: the islands of the level form together;
+    // of the others, those below coopMin contacts one lane each, larger ones
+    // by the whole wave, one after another.
     float4* stage = g_smem + (int(c.ldsBytes) / 16 - prx::kStageFloat4);
     const int coopMin = (c.coopMin == 0u) ? 1 : (c.coopMin > 0x7fffffffu ? 0x7fffffff : int(c.coopMin));
     auto constraints = [&](int is) {
         return (S.istart[is + 1].y - S.istart[is].y) + (S.jstart[is + 1] - S.jstart[is]);
     };
+    // The level form needs the body state and two words per island in LDS.
+    const bool levels = kLds && !kTape && x.nb <= kLevelMaxBodies &&
+                        x.nb * 40 + prx::kStageFloat4 * 16 <= int(c.ldsBytes);
+    auto level = [&](int is) {
+        return levels && level_island(S.istart[is + 1].y - S.istart[is].y, S.jstart[is + 1] - S.jstart[is], coopMin);
+    };
+    bool anyLevel = false;
+    LevelPlan plan{0, 0, 0, nullptr, nullptr};
+    if constexpr (kLds && !kTape) {
+        const LevelScratch L(d, x);
+        for (int base = 0; base < nisl; base += kWave) {
+            const int is = base + x.lane;
+            const bool lv = is < nisl && level(is);
+            if (is < nisl)
+                for (int e = S.istart[is].y; e < S.istart[is + 1].y; ++e) L.island[e] = lv ? is : -1;
+            anyLevel = anyLevel || __ballot(lv) != 0;
+        }
+        __syncthreads();
+        if (anyLevel) {
+            plan = level_plan(d, x, stage, nce);
+            velocity_levels(d, x, bs, S, plan, nisl, level, c, addVel);
+        }
+    }
     for (int is = x.lane; is < nisl; is += kWave) {
-        if (constraints(is) < coopMin)
+        if (constraints(is) < coopMin && !level(is))
             addVel(island_velocity<kLds, kTape>(d, x, bs, S.istart[is].y, S.istart[is + 1].y, S.jstart[is],
                                                 S.jstart[is + 1], c, x.bo + x.w + is));
     }
     __syncthreads();
     for (int base = 0; base < nisl; base += kWave) {
         const int is = base + x.lane;
-        const bool big = is < nisl && constraints(is) >= coopMin;
+        const bool big = is < nisl && constraints(is) >= coopMin && !level(is);
         for (unsigned long long m = __ballot(big); m; m &= m - 1) {
             const int isl = base + __ffsll(m) - 1;
-            const int c0 = S.istart[isl].y, c1 = S.istart[isl + 1].y;
-            VelResult r;
-            if (level_form(x, c0, c1, S.jstart[isl], S.jstart[isl + 1])) {
-                const LevelPlan P = level_plan(d, x, stage, c0, c1);
-                r = island_velocity_level<kLds>(d, x, bs, P, c0, c, stage);
-            } else {
-                r = island_velocity_wave<kLds>(d, x, bs, stage, c0, c1, S.jstart[isl], S.jstart[isl + 1], c);
-            }
+            const VelResult r = island_velocity_wave<kLds>(d, x, bs, stage, S.istart[isl].y, S.istart[isl + 1].y,
+                                                           S.jstart[isl], S.jstart[isl + 1], c);
             if (x.lane == 0) addVel(r);
         }
     }
@@ -4467,8 +4761,17 @@ __device__ __forceinline__ SolveSummary solve_islands(const DeviceState& d, cons
     }
     __syncthreads();
     // Position sweeps, split like the velocity sweeps.
+    if constexpr (kLds && !kTape) {
+        // An island's smallest separation is over all its iterations; its
+        // result is counted with the last.
+        if (anyLevel)
+            position_levels(d, x, bs, S, plan, nisl, level, c, [&](const PosResult& r, bool last) {
+                if (last) addPos(r);
+                else aMin = fmin_std(aMin, r.minSep);
+            });
+    }
     for (int is = x.lane; is < nisl; is += kWave) {
-        if (constraints(is) < coopMin) {
+        if (constraints(is) < coopMin && !level(is)) {
             const PosResult r = island_position<kLds, kTape>(d, x, bs, S.istart[is].y, S.istart[is + 1].y,
                                                              S.jstart[is], S.jstart[is + 1], c, x.bo + x.w + is);
             S.isl_word[is] = std::uint32_t(r.solvedAt);
@@ -4478,15 +4781,11 @@ __device__ __forceinline__ SolveSummary solve_islands(const DeviceState& d, cons
     __syncthreads();
     for (int base = 0; base < nisl; base += kWave) {
         const int is = base + x.lane;
-        const bool big = is < nisl && constraints(is) >= coopMin;
+        const bool big = is < nisl && constraints(is) >= coopMin && !level(is);
         for (unsigned long long m = __ballot(big); m; m &= m - 1) {
             const int isl = base + __ffsll(m) - 1;
-            const int c0 = S.istart[isl].y, c1 = S.istart[isl + 1].y;
-            const PosResult r = level_form(x, c0, c1, S.jstart[isl], S.jstart[isl + 1])
-                                    ? island_position_level<kLds>(d, x, bs, level_plan_of(d, x, c0, c1), c0, c,
-                                                                  stage)
-                                    : island_position_wave<kLds>(d, x, bs, stage, c0, c1, S.jstart[isl],
-                                                                 S.jstart[isl + 1], c);
+            const PosResult r = island_position_wave<kLds>(d, x, bs, stage, S.istart[isl].y, S.istart[isl + 1].y,
+                                                           S.jstart[isl], S.jstart[isl + 1], c);
             if (x.lane == 0) {
                 S.isl_word[isl] = std::uint32_t(r.solvedAt);
                 addPos(r);

@@ -1,0 +1,55 @@
+"""The level form of the island solve (independent updates of a round side by
+side, iterations overlapped, early exits solved again) against the oracle, bit
+for bit, at the edges of its rules: islands just below and above its smallest
+size, exits on a lane and by plain iterations, bounds that forbid overlapping,
+iteration counts at the limits of the exit word."""
+import pytest
+
+import playrho_amd as pa
+from tests import dumpfmt, golden_cases, oracle_lib
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # scene, parameters, steps, conf
+    ("pile", [1, 0, 3, 3], 90, {}),
+    ("pile", [1, 1, 4, 4], 90, {}),
+    ("pile", [1, 2, 9, 9], 120, {}),
+    ("pile", [2, 0, 33, 33], 150, {}),
+    ("pile", [2, 1, 64, 64], 150, {}),
+    ("pile", [3, 0, 150, 150], 150, {}),
+    ("pyramid", [6], 90, {}),
+    ("pyramid", [12], 60, {}),
+    ("billiards", [1, 0], 60, {}),
+    ("pyramid", [8], 60, dict(reg_min_momentum=0.05)),
+    ("pile", [2, 1, 64, 64], 120, dict(reg_min_momentum=0.01)),
+    ("pile", [2, 1, 64, 64], 120, dict(reg_min_momentum=-1.0)),
+    ("pile", [2, 1, 64, 64], 90, dict(reg_velocity_iters=0)),
+    ("pile", [2, 1, 64, 64], 90, dict(reg_velocity_iters=1)),
+    ("pile", [2, 1, 64, 64], 90, dict(reg_velocity_iters=31)),
+    ("pile", [2, 1, 64, 64], 90, dict(reg_velocity_iters=32)),
+    ("pile", [2, 1, 64, 64], 90, dict(reg_position_iters=0)),
+    ("pile", [2, 1, 64, 64], 90, dict(reg_position_iters=7)),
+    ("pile", [2, 1, 64, 64], 90, dict(do_warm_start=0)),
+    ("pyramid", [8], 60, dict(do_blocksolve=0)),
+    ("terrain", [1, 0], 120, {}),
+    ("chain", [1, 0], 90, {}),
+]
+
+
+@pytest.mark.parametrize("scene,params,steps,conf", CASES)
+@pytest.mark.parametrize("coop_min", [None, 1])
+def test_level_form_matches_oracle(scene, params, steps, conf, coop_min):
+    conf = pa.StepConf(do_toi=0, **conf)
+    w = pa.World.scene(scene, params)
+    w.record_contact_events(True)
+    ow = oracle_lib.OracleWorld(w.save_desc() + dumpfmt.conf_record(conf))
+    batch = pa.Batch([w], use_graph=False, coop_min=coop_min)
+    print(scene, params, coop_min, flush=True)
+    for step in range(1, steps + 1):
+        batch.step(conf, 1)
+        batch.download()
+        got = dumpfmt.read_state(dumpfmt.Reader(w.state_record()))
+        want = ow.step(1)[0]
+        for part in golden_cases.PARTS:
+            assert dumpfmt.digest(got, (part,)) == dumpfmt.digest(want, (part,)), (step, part)
