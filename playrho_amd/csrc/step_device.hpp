@@ -18,6 +18,22 @@ using prx::WorldHeader;
 constexpr int kWave = 64;
 constexpr int kChunk = prx::kStageRecords;
 
+// Functions of their own, not inlined, hold the step's serial loops: among the
+// other phases the loops' scalars were spilled, or waits for every load put
+// into them, by changes elsewhere.  Their arguments are uniform, which a call
+// does not tell: they are read from the first lane.  (A pile of 400 bodies, the
+// velocity sweeps: 3.0M cycles inlined beside the grid's pair search, 2.1M so.)
+template <class T>
+__device__ __forceinline__ T* uniform_ptr(T* p) {
+    const unsigned long long v = reinterpret_cast<unsigned long long>(p);
+    const unsigned lo = unsigned(__builtin_amdgcn_readfirstlane(int(v))), hi = unsigned(__builtin_amdgcn_readfirstlane(int(v >> 32)));
+    return reinterpret_cast<T*>((static_cast<unsigned long long>(hi) << 32) | lo);
+}
+__device__ __forceinline__ float uniform_f(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+using LdsWord = __attribute__((address_space(3))) int;
+
 // Phase timer: lane 0 records shader-clock deltas into phase_cycles[w].
 struct PhaseTimer {
     unsigned long long* out;
@@ -496,6 +512,132 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
+// Candidate pairs by a grid in LDS: the proxies sorted by the cell of their
+// lower corner, each moved proxy (one per lane) against the entries of the cells
+// its box reaches, one below included (a proxy that spans more than two cells
+// in a direction goes to a list that everyone reads).  The cell number grows
+// with the coordinate under any rounding, so no overlap is missed; the keys are
+// sorted afterwards, so their order here is free.  Returns the number of pairs
+// (past cap: not stored), or -1 where the boxes or the LDS do not allow it.
+constexpr int kGridCells = 512;
+// From 256 rounds of 64 tests on the grid pays: its set-up costs what about
+// 80 such rounds do (150 cycles each), a chunk of 64 moved proxies another 80.
+// A pile of 400 bodies: 388k -> 217k cycles with everything that follows.
+constexpr int kGridTests = 256;
+__device__ __forceinline__ int find_pairs_grid(const DeviceState& d, const WorldCtx& x, const int* moved, int nmoved,
+                                               int ldsAvail) {
+    if (x.np * 24 + (kGridCells + 2) * 4 > ldsAvail) return -1;
+    float4* const box = g_smem;                                  // by cell
+    int2* const meta = reinterpret_cast<int2*>(box + x.np);      // proxy | moved << 31, body
+    int* const end = reinterpret_cast<int*>(meta + x.np);        // of the cells, and of the list
+    const float inf = __builtin_inff();
+    float lx = inf, ly = inf, hx = -inf, hy = -inf, ext = 0.0f;
+    for (int p = x.lane; p < x.np; p += kWave) {
+        const float4 a = d.paabb[x.po + p];
+        lx = fminf(lx, a.x);
+        ly = fminf(ly, a.y);
+        hx = fmaxf(hx, a.x);
+        hy = fmaxf(hy, a.y);
+        ext += fmaxf(a.z - a.x, a.w - a.y) + 0.0f * (a.x + a.y + a.z + a.w);  // NaN unless finite
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        lx = fminf(lx, __shfl_xor(lx, o));
+        ly = fminf(ly, __shfl_xor(ly, o));
+        hx = fmaxf(hx, __shfl_xor(hx, o));
+        hy = fmaxf(hy, __shfl_xor(hy, o));
+        ext += __shfl_xor(ext, o);
+    }
+    const float rx = hx - lx, ry = hy - ly;
+    float size = 2.0f * ext / float(x.np);
+    if (!(size > 1e-20f && size < 1e20f && rx < 1e20f && ry < 1e20f)) return -1;
+    while (!((rx / size + 1.0f) * (ry / size + 1.0f) <= float(kGridCells))) size *= 1.25f;
+    const float inv = 1.0f / size;
+    const int nx = __builtin_amdgcn_readfirstlane(min(int(rx * inv) + 1, kGridCells));
+    const int ny = __builtin_amdgcn_readfirstlane(min(int(ry * inv) + 1, kGridCells / nx));
+    auto cell_x = [&](float v) { return int(fminf(fmaxf((v - lx) * inv, 0.0f), float(nx - 1))); };
+    auto cell_y = [&](float v) { return int(fminf(fmaxf((v - ly) * inv, 0.0f), float(ny - 1))); };
+    const int ncells = nx * ny;
+    auto cell_of = [&](float4 a) {
+        const int x0 = cell_x(a.x), y0 = cell_y(a.y);
+        return (cell_x(a.z) - x0 > 1 || cell_y(a.w) - y0 > 1) ? ncells : y0 * nx + x0;
+    };
+    for (int i = x.lane; i <= ncells; i += kWave) end[i] = 0;
+    __syncthreads();
+    for (int p = x.lane; p < x.np; p += kWave) atomicAdd(&end[cell_of(d.paabb[x.po + p])], 1);
+    __syncthreads();
+    int carry = 0;
+    for (int b0 = 0; b0 <= ncells; b0 += kWave) {
+        const int i = b0 + x.lane;
+        const int v = (i <= ncells) ? end[i] : 0;
+        const int incl = wave_incl_scan(v, x.lane);
+        if (i <= ncells) end[i] = carry + incl - v;
+        carry += __shfl(incl, kWave - 1);
+    }
+    __syncthreads();
+    // The places move each cell's start to its end, the start of the next.
+    for (int p = x.lane; p < x.np; p += kWave) {
+        const float4 a = d.paabb[x.po + p];
+        const int at = atomicAdd(&end[cell_of(a)], 1);
+        box[at] = a;
+        meta[at] = int2{p | ((d.pflags[x.po + p] & prx::kProxyMoved) ? int(0x80000000u) : 0), d.pbody[x.po + p]};
+    }
+    __syncthreads();
+    auto start = [&](int i) { return i > 0 ? end[i - 1] : 0; };
+    int ncand = 0;
+    for (int mb = 0; mb < nmoved; mb += kWave) {
+        const bool on = mb + x.lane < nmoved;
+        int m = 0, mbody = -1, x0 = 0, x1 = -1, y0 = 0, y1 = -1;
+        float4 am{0, 0, 0, 0};
+        if (on) {
+            m = moved[mb + x.lane];
+            mbody = d.pbody[x.po + m];
+            am = d.paabb[x.po + m];
+            x0 = max(cell_x(am.x) - 1, 0);
+            x1 = cell_x(am.z);
+            y0 = max(cell_y(am.y) - 1, 0);
+            y1 = cell_y(am.w);
+        }
+        auto test = [&](bool in, float4 aq, int2 q) {
+            const int qi = q.x & 0x7fffffff;
+            // A pair of two moved proxies is produced once, from the smaller.
+            const bool hit = in && qi != m && !(q.x < 0 && qi < m) && q.y != mbody && overlap(am, aq);
+            const unsigned long long hm = __ballot(hit);
+            if (hm == 0) return;
+            if (hit) {
+                const int r = ncand + __popcll(hm & lanes_below(x.lane));
+                if (r < x.cap) {
+                    const int lo = qi < m ? qi : m, hi = qi < m ? m : qi;
+                    d.s_keys[x.co + r] = (std::uint32_t(lo) << 16) | std::uint32_t(hi);
+                }
+            }
+            ncand += __popcll(hm);
+        };
+        // The list, then row after row of cells (a row's cells are side by side).
+        for (int row = -1;; ++row) {
+            int e = 0, e1 = 0;
+            const bool go = on && (row < 0 || y0 + row <= y1);
+            if (row >= 0 && !__ballot(go)) break;
+            if (go) {
+                const int first = row < 0 ? ncells : (y0 + row) * nx + x0;
+                e = start(first);
+                e1 = end[row < 0 ? ncells : (y0 + row) * nx + x1];
+            }
+            while (__ballot(e < e1)) {
+                // Two entries at a time: their reads overlap.
+                const bool in0 = e < e1, in1 = e + 1 < e1;
+                const int k0 = in0 ? e : 0, k1 = in1 ? e + 1 : 0;
+                const float4 a0 = box[k0], a1 = box[k1];
+                const int2 q0 = meta[k0], q1 = meta[k1];
+                test(in0, a0, q0);
+                test(in1, a1, q1);
+                e += 2;
+            }
+        }
+    }
+    __syncthreads();
+    return ncand;
+}
+
 // ldsAvail: bytes of dynamic LDS the caller's kernel has (free during this
 // phase).  When the candidates fit, they are sorted and looked up there.
 __device__ __forceinline__ std::uint32_t phase_find_add(const DeviceState& d, const WorldCtx& x, Counters& k, const StepParams& c,
@@ -517,13 +659,17 @@ __device__ __forceinline__ std::uint32_t phase_find_add(const DeviceState& d, co
     if (nmoved == 0) return 0;
     int* moved = d.s_isl_body + x.bo + x.co;
 
-    // Candidate pairs: every proxy q (one per lane) against every moved proxy
+    // Candidate pairs, by the grid where that is shorter, else every proxy q (one per lane) against every moved proxy
     // m.  The moved proxies come in chunks of one per lane (index, body and
     // fat AABB in registers) and the wave reads them one at a time from the
     // holding lane, so the inner loop does no memory access.
-    int ncand = 0;
     bool overflow = false;
-    for (int base = 0; base < x.np; base += kWave) {
+    int ncand = -1;
+    if (nmoved * ((x.np + kWave - 1) / kWave) >= kGridTests) ncand = find_pairs_grid(d, x, moved, nmoved, ldsAvail);
+    // Past the scratch, the pairs kept are those of the plain order.
+    const bool plain = ncand < 0 || ncand > x.cap;
+    if (plain) ncand = 0;
+    for (int base = 0; plain && base < x.np; base += kWave) {
         const int q = base + x.lane;
         const bool qv = q < x.np;
         float4 qa = float4{0, 0, 0, 0};
@@ -717,24 +863,20 @@ __device__ __forceinline__ std::uint32_t phase_find_add(const DeviceState& d, co
     }
     __syncthreads();
     // Awake flags (SetAwakeFlag for speedable bodies of non-sensor contacts):
-    // idempotent, so done per new contact in a second pass without races on
-    // the flags word of a body touched by two lanes.
+    // idempotent, so done per new contact in a second pass, by atomics for a
+    // body touched by two lanes.
     int nadd = int(added);
     if (nc0 + nadd > x.cap) {
         k.status |= prx::kStatusContactOverflow;
         nadd = x.cap - nc0;
     }
     if (overflow) k.status |= prx::kStatusScratchOverflow;
-    if (x.lane == 0) {
-        for (int r = 0; r < nadd; ++r) {
-            const int gi = x.co + nc0 + r;
-            if (d.c_flags[gi] & prx::kSensor) continue;
-            const int2 bd = d.c_body[gi];
-            const std::uint32_t fa = d.bflags[x.bo + bd.x];
-            if (fa & prx::kSpeedable) d.bflags[x.bo + bd.x] = fa | prx::kAwake;
-            const std::uint32_t fb = d.bflags[x.bo + bd.y];
-            if (fb & prx::kSpeedable) d.bflags[x.bo + bd.y] = fb | prx::kAwake;
-        }
+    for (int r = x.lane; r < nadd; r += kWave) {
+        const int gi = x.co + nc0 + r;
+        if (d.c_flags[gi] & prx::kSensor) continue;
+        const int2 bd = d.c_body[gi];
+        if (d.bflags[x.bo + bd.x] & prx::kSpeedable) atomicOr(&d.bflags[x.bo + bd.x], std::uint32_t(prx::kAwake));
+        if (d.bflags[x.bo + bd.y] & prx::kSpeedable) atomicOr(&d.bflags[x.bo + bd.y], std::uint32_t(prx::kAwake));
     }
     const int consumedFree = nadd < k.nfree ? nadd : k.nfree;
     k.pool += nadd - consumedFree;
@@ -3005,6 +3147,152 @@ __device__ __forceinline__ int find_islands(const DeviceState& d, const WorldCtx
 }
 
 
+// The depth first search of the islands, body after body as the serial one goes
+// (AddToIsland, AabbTreeWorld.cpp:1339-1444), the wave looking at a body's
+// contacts (joints) side by side: what is new is listed in order by ballots,
+// and the last body reached, kept at hand, is the next one.  Bound by its
+// instructions, one body after another: a function of its own and not inlined,
+// so that its scalars stay in registers, with every value that steers it read
+// as uniform and no lane masked off where all may write the same.  400 bodies:
+// 1075 -> 750 cycles a body; a chain world of 98 bodies with its joints' lists
+// in LDS 140k -> 60k cycles in all.
+//
+// LDS words: off (nb + 1), the stack (nb; reached static bodies from its top,
+// :1386-1398), the entries contact << 16 | other body; then the bytes of the
+// bodies (0 to reach, 1 reached, 2 static, 3 static and counted for the
+// island; 8: not enabled, 16: may start an island), contacts and joints; then
+// the bodies' joint ranges and list.  The wave's LDS operations run in order,
+// so a compiler fence is enough.  Returns islands, most bodies of one.
+using LdsByte = __attribute__((address_space(3))) std::uint8_t;
+template <bool kJoints>
+__device__ __attribute__((noinline)) int2 search_islands(LdsWord* smem, int nb, int nc, int nj, int nent, int* ibody,
+                                                         int* bisland, int* icont, int2* istart, int* jstart, int* ijoint,
+                                                         int nisl) {
+    nb = __builtin_amdgcn_readfirstlane(nb);
+    nisl = __builtin_amdgcn_readfirstlane(nisl);
+    ibody = uniform_ptr(ibody);
+    bisland = uniform_ptr(bisland);
+    icont = uniform_ptr(icont);
+    istart = uniform_ptr(istart);
+    jstart = uniform_ptr(jstart);
+    ijoint = uniform_ptr(ijoint);
+    const int lane = int(threadIdx.x);
+    LdsWord* const off = smem;
+    LdsWord* const stack = off + nb + 1;
+    LdsWord* const ent = stack + nb;
+    const int marks = 4 * (2 * nb + 1 + __builtin_amdgcn_readfirstlane(nent));
+    LdsByte* const islb = (LdsByte*)smem + marks;
+    LdsByte* const islc = islb + nb;
+    LdsByte* const islj = islc + __builtin_amdgcn_readfirstlane(nc);
+    LdsWord* const jrange = smem + (marks + nb + __builtin_amdgcn_readfirstlane(nc) + __builtin_amdgcn_readfirstlane(nj) + 7) / 8 * 2;
+    LdsWord* const jlist = jrange + 2 * nb;
+    auto order = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+    auto rank = [](unsigned long long m) {  // lanes of m below this one
+        return int(__builtin_amdgcn_mbcnt_hi(unsigned(m >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(m), 0u)));
+    };
+    int nbe = nisl, nce = 0, nje = 0;
+    int maxB = nisl > 0 ? 1 : 0;
+    for (int base = 0; base < nb; base += kWave) {
+        const int mine = base + lane < nb ? base + lane : nb - 1;
+        auto seeds = [&] { return __ballot(base + lane < nb && (islb[mine] & 19) == 16); };
+        for (unsigned long long left = seeds(); left; left = seeds()) {
+            int bb = base + __builtin_ctzll(left);
+            istart[nisl] = int2{nbe, nce};
+            if constexpr (kJoints) jstart[nisl] = nje;
+            else jstart[nisl] = 0;
+            islb[bb] |= 1;
+            order();
+            const int nbe0 = nbe;
+            int nst = 0, sp = 0;
+            int e0 = __builtin_amdgcn_readfirstlane(off[bb]), e1 = __builtin_amdgcn_readfirstlane(off[bb + 1]);
+            for (;;) {
+                ibody[nbe] = bb;
+                bisland[bb] = nisl;
+                ++nbe;
+                int next = -1, next0 = 0, next1 = 0;
+                // The new bodies of the lanes, in lane order: a moving one is
+                // put on the stack, a static one is counted.
+                auto reach = [&](bool fresh, int ob, int mark, int r0, int r1) {
+                    const bool push = fresh && (mark & 3) == 0, count = fresh && (mark & 3) == 2;
+                    if (push || count) islb[ob] = std::uint8_t(mark | 1);
+                    for (unsigned long long p = __ballot(push); p;) {
+                        const int l = __builtin_ctzll(p);
+                        const int o = readlane_i(ob, l);
+                        p &= ~__ballot(push && ob == o);
+                        if (next >= 0) {
+                            stack[sp] = next;
+                            ++sp;
+                        }
+                        next = o;
+                        next0 = readlane_i(r0, l);
+                        next1 = readlane_i(r1, l);
+                    }
+                    for (unsigned long long p = __ballot(count); p;) {
+                        const int o = readlane_i(ob, __builtin_ctzll(p));
+                        p &= ~__ballot(count && ob == o);
+                        stack[nb - 1 - nst] = o;
+                        ++nst;
+                    }
+                    order();
+                };
+                for (int e = e0; e < e1; e += kWave) {
+                    const bool has = e + lane < e1;
+                    const std::uint32_t en = std::uint32_t(ent[has ? e + lane : e]);
+                    const int ci = int(en >> 16), ob = int(en & 0xffffu);
+                    const int taken = islc[ci], mark = islb[ob], r0 = off[ob], r1 = off[ob + 1];
+                    const bool fresh = has && taken == 0;
+                    const unsigned long long m = __ballot(fresh);
+                    if (fresh) {
+                        icont[nce + rank(m)] = ci;
+                        islc[ci] = 1;
+                    }
+                    nce += __popcll(m);
+                    reach(fresh, ob, mark, r0, r1);
+                }
+                if constexpr (kJoints) {
+                    // AddJointsToIsland (AabbTreeWorld.cpp:1446-1470).
+                    const int j0 = __builtin_amdgcn_readfirstlane(jrange[2 * bb]), j1 = j0 + __builtin_amdgcn_readfirstlane(jrange[2 * bb + 1]);
+                    for (int j = j0; j < j1; j += kWave) {
+                        const bool has = j + lane < j1;
+                        const int at = has ? j + lane : j;
+                        const int ji = jlist[2 * at], other = jlist[2 * at + 1];
+                        // A target joint has no other body (-1).
+                        const int ob = other >= 0 ? other : 0;
+                        const int taken = islj[ji], mark = other >= 0 ? int(islb[ob]) : 1, r0 = off[ob], r1 = off[ob + 1];
+                        bool fresh = has && taken == 0 && (mark & 8) == 0;
+                        // A joint of a body with itself is listed twice: one
+                        // lane's claim stays.
+                        if (fresh) islj[ji] = std::uint8_t(lane + 1);
+                        order();
+                        fresh = fresh && islj[ji] == lane + 1;
+                        const unsigned long long m = __ballot(fresh);
+                        if (fresh) ijoint[nje + rank(m)] = ji;
+                        nje += __popcll(m);
+                        reach(fresh, ob, mark, r0, r1);
+                    }
+                }
+                if (next < 0) {
+                    if (sp == 0) break;
+                    --sp;
+                    next = __builtin_amdgcn_readfirstlane(stack[sp]);
+                    next0 = __builtin_amdgcn_readfirstlane(off[next]);
+                    next1 = __builtin_amdgcn_readfirstlane(off[next + 1]);
+                }
+                bb = next;
+                e0 = next0;
+                e1 = next1;
+            }
+            for (int q = lane; q < nst; q += kWave) islb[stack[nb - 1 - q]] &= std::uint8_t(~1u);
+            order();
+            maxB = (nbe - nbe0 + nst > maxB) ? nbe - nbe0 + nst : maxB;
+            ++nisl;
+        }
+    }
+    istart[nisl] = int2{nbe, nce};
+    jstart[nisl] = nje;
+    return int2{nisl, maxB};
+}
+
 // Islands with everything in LDS (ldsAvail bytes): the per-body adjacency
 // (entries packed as contact index << 16 | other body, for worlds under 2^16
 // contacts and bodies), the DFS stack and the flags.  Only the lists of
@@ -3014,7 +3302,6 @@ __device__ __forceinline__ int find_islands(const DeviceState& d, const WorldCtx
 // with nothing written outside LDS, when the world does not fit.
 __device__ __forceinline__ int find_islands_lds(const DeviceState& d, const WorldCtx& x, int nc, const IslandScratch& S,
                                                 int& maxBodies, int ldsAvail) {
-    __shared__ int s_cnt[2];
     if (x.nb >= 0xffff || nc >= 0xffff) return -1;
     const int nb = x.nb;
     // off: nb + 1 ints; stack: nb ints (first the scatter cursors); entries.
@@ -3049,7 +3336,8 @@ __device__ __forceinline__ int find_islands_lds(const DeviceState& d, const Worl
     std::uint8_t* islb = reinterpret_cast<std::uint8_t*>(ent + nent);
     std::uint8_t* islc = islb + nb;
     std::uint8_t* islj = islc + nc;
-    if (4 * (2 * nb + 1 + nent) + nb + nc + x.nj > ldsAvail) return -1;
+    const int marks = 4 * (2 * nb + 1 + nent) + nb + nc + x.nj;
+    if (marks + (x.nj > 0 ? 7 + 8 * (nb + 2 * x.nj) : 0) > ldsAvail) return -1;
     for (int b = x.lane; b < nb; b += kWave) stack[b] = off[b];
     __syncthreads();
     for (int i = x.lane; i < nc; i += kWave) {
@@ -3072,11 +3360,19 @@ __device__ __forceinline__ int find_islands_lds(const DeviceState& d, const Worl
             }
             ent[j + 1] = v;
         }
-        islb[b] = listed(b) ? 0 : 2;
+        const std::uint32_t f = d.bflags[x.bo + b];
+        islb[b] = std::uint8_t(((f & prx::kSpeedable) ? 0 : 2) | ((f & prx::kEnabled) ? 0 : 8) |
+                               (((f & prx::kAwake) && (f & prx::kEnabled)) ? 16 : 0));
         S.bisland[b] = -1;
     }
     for (int i = x.lane; i < nc; i += kWave) islc[i] = 0;
     for (int i = x.lane; i < x.nj; i += kWave) islj[i] = 0;
+    // The bodies' joints behind the marks.
+    int2* const jrange = reinterpret_cast<int2*>(g_smem) + (marks + 7) / 8;
+    if (x.nj > 0) {
+        for (int b = x.lane; b < nb; b += kWave) jrange[b] = d.bjoint[x.bo + b];
+        for (int i = x.lane; i < 2 * x.nj; i += kWave) jrange[nb + i] = d.bjoint_list[2 * x.jo + i];
+    }
     __syncthreads();
     // One-body islands.
     int nsingle = 0;
@@ -3095,81 +3391,19 @@ __device__ __forceinline__ int find_islands_lds(const DeviceState& d, const Worl
             S.istart[r] = int2{r, 0};
             S.jstart[r] = 0;
             S.bisland[b] = r;
-            islb[b] = 1;
+            islb[b] |= 1;
         }
         nsingle += __popcll(m);
     }
     __syncthreads();
-    if (x.lane == 0) {
-        int nisl = nsingle, nbe = nsingle, nce = 0, nje = 0;
-        // Reached static bodies are marked 3 while counted and listed from
-        // the top of the stack array (AabbTreeWorld.cpp:1386-1398).
-        int maxB = nsingle > 0 ? 1 : 0;
-        for (int seed = 0; seed < nb; ++seed) {
-            if (islb[seed]) continue;
-            const std::uint32_t sf = d.bflags[x.bo + seed];
-            if (!((sf & prx::kAwake) && (sf & prx::kEnabled))) continue;
-            S.istart[nisl] = int2{nbe, nce};
-            S.jstart[nisl] = nje;
-            const int nbe0 = nbe;
-            int nst = 0;
-            int sp = 0;
-            stack[sp++] = seed;
-            islb[seed] = 1;
-            while (sp > 0) {
-                const int bb = stack[--sp];
-                S.ibody[nbe++] = bb;
-                S.bisland[bb] = nisl;
-                const int e1 = off[bb + 1];
-                for (int e = off[bb]; e < e1; ++e) {
-                    const std::uint32_t en = ent[e];
-                    const int ci = int(en >> 16), ob = int(en & 0xffffu);
-                    if (islc[ci]) continue;
-                    S.icont[nce++] = ci;
-                    islc[ci] = 1;
-                    if (islb[ob] == 0) {
-                        islb[ob] = 1;
-                        stack[sp++] = ob;
-                    } else if (islb[ob] == 2) {
-                        islb[ob] = 3;
-                        stack[nb - 1 - nst++] = ob;
-                    }
-                }
-                // AddJointsToIsland (AabbTreeWorld.cpp:1446-1470).
-                if (x.nj) {
-                    const int2 bj = d.bjoint[x.bo + bb];
-                    for (int k = 0; k < bj.y; ++k) {
-                        const int2 je = d.bjoint_list[2 * x.jo + bj.x + k];
-                        if (islj[je.x]) continue;
-                        // A target joint has no other body (-1).
-                        if (je.y >= 0 && !(d.bflags[x.bo + je.y] & prx::kEnabled)) continue;
-                        islj[je.x] = 1;
-                        S.ijoint[nje++] = je.x;
-                        if (je.y < 0) continue;
-                        if (islb[je.y] == 0) {
-                            islb[je.y] = 1;
-                            stack[sp++] = je.y;
-                        } else if (islb[je.y] == 2) {
-                            islb[je.y] = 3;
-                            stack[nb - 1 - nst++] = je.y;
-                        }
-                    }
-                }
-            }
-            for (int q = 0; q < nst; ++q) islb[stack[nb - 1 - q]] = 2;
-            maxB = (nbe - nbe0 + nst > maxB) ? nbe - nbe0 + nst : maxB;
-            ++nisl;
-        }
-        S.istart[nisl] = int2{nbe, nce};
-        S.jstart[nisl] = nje;
-        s_cnt[0] = nisl;
-        s_cnt[1] = maxB;
-    }
+    const int2 found = x.nj > 0
+        ? search_islands<true>((LdsWord*)reinterpret_cast<int*>(g_smem), nb, nc, x.nj, nent, S.ibody, S.bisland, S.icont,
+                               S.istart, S.jstart, S.ijoint, nsingle)
+        : search_islands<false>((LdsWord*)reinterpret_cast<int*>(g_smem), nb, nc, 0, nent, S.ibody, S.bisland, S.icont,
+                                S.istart, S.jstart, S.ijoint, nsingle);
     __syncthreads();
-    maxBodies = s_cnt[1];
-    const int n = s_cnt[0];
-    __syncthreads();
-    return n;
+    maxBodies = __builtin_amdgcn_readfirstlane(found.y);
+    return __builtin_amdgcn_readfirstlane(found.x);
 }
 
 // Position-constraint record (see the layout above).
@@ -3984,8 +4218,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t record_rsrc(const float4* base
 // Bounds of a round (first position, updates), read by buffer loads as well
 // and two rounds ahead: a lane without a round reads past the end and gets
 // none.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rounds_rsrc(const LevelPlan& P) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<int2*>(P.rb), 0, P.rounds * int(sizeof(int2)), 0x00020000);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rounds_rsrc(const int2* rb, int rounds) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<int2*>(rb), 0, rounds * int(sizeof(int2)), 0x00020000);
 }
 
 using U4 = __attribute__((ext_vector_type(4))) unsigned;
@@ -4106,15 +4340,20 @@ __device__ __forceinline__ void quad_block(QuadBody& me, const QuadRec& r, int l
 // their words are left out of a masked run.
 enum LevelPass { kPassWarm, kPassWarmMasked, kPassIterations, kPassMasked };
 template <LevelPass kPass>
-__device__ __forceinline__ void velocity_level_run(const __amdgpu_buffer_rsrc_t rec, const LevelPlan& P, int iters,
-                                                   int* words, int lane) {
-    const __amdgpu_buffer_rsrc_t table = rounds_rsrc(P);
+__device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n, const int2* rb, int rounds, int period,
+                                                             int iters, LdsWord* smem, int wordsAt) {
+    rounds = __builtin_amdgcn_readfirstlane(rounds);
+    period = __builtin_amdgcn_readfirstlane(period);
+    iters = __builtin_amdgcn_readfirstlane(iters);
+    const __amdgpu_buffer_rsrc_t table = rounds_rsrc(uniform_ptr(rb), rounds);
+    const __amdgpu_buffer_rsrc_t rec = record_rsrc(uniform_ptr(recs), __builtin_amdgcn_readfirstlane(n), prx::kQuadVc);
+    float* const lds = reinterpret_cast<float*>((int*)smem);
+    int* const words = (int*)(smem + __builtin_amdgcn_readfirstlane(wordsAt));
+    const int lane = int(threadIdx.x);
     constexpr bool kWarm = kPass == kPassWarm || kPass == kPassWarmMasked;
     constexpr bool kMasked = kPass == kPassMasked || kPass == kPassWarmMasked;
-    float* const lds = reinterpret_cast<float*>(g_smem);
     const int group = lane >> 5, j = (lane >> 2) & (kLevelRound - 1), quad = lane & 3, comp = lane & 1;
     constexpr int kStep = prx::kQuadVc * 16;
-    const int rounds = P.rounds, period = P.period;
     int r = -group * period, it = group;  // the group's round and iteration at the tick read ahead
     struct At {
         int2 b;
@@ -4221,6 +4460,10 @@ __device__ __forceinline__ void velocity_level_run(const __amdgpu_buffer_rsrc_t 
     __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
+struct PositionConf {
+    float regResolutionRate, linearSlop, maxLinearCorrection;
+};
+
 // A position record as a lane holds it: this body, its points, the common part.
 struct QuadPos {
     float4 b, u, v, k;
@@ -4241,7 +4484,7 @@ __device__ __forceinline__ bool almost_equal_steps(float a, float b) {
 // lanes, a face's normal on X's, and handed to the other body's.  p, a: the
 // lane's position component and angle, updated; returns the separation, or
 // infinity where nothing is solved.
-__device__ __forceinline__ float quad_position(const QuadPos& r, int quad, float& p, float& a, const StepParams& c) {
+__device__ __forceinline__ float quad_position(const QuadPos& r, int quad, float& p, float& a, const PositionConf& c) {
     const bool compY = quad & 1, bodyY = quad & 2;
     const std::uint32_t h = __float_as_uint(r.k.z);
     const std::uint32_t type = h & 0xffu, n = (h >> 8) & 0xffu;
@@ -4378,9 +4621,10 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
                                                 const StepParams& c, Add add) {
     float4* v2 = d.s_vc2 + std::size_t(x.co) * prx::kQuadVc;
     float4* vbase = d.s_vc + std::size_t(x.co) * prx::kVcStride;
-    const __amdgpu_buffer_rsrc_t rec = record_rsrc(v2, P.n, prx::kQuadVc);
     const LevelScratch L(d, x);
     int* const words = island_words(x);
+    LdsWord* const smem = (LdsWord*)reinterpret_cast<int*>(g_smem);
+    const int wordsAt = 8 * x.nb;
     constexpr int kOut = int(0x80000000u);  // left out of masked runs
     const int iters = int(c.velIters);
     const bool overlap = c.regMinMomentum <= 0.0f && iters <= 31;
@@ -4389,9 +4633,9 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
         words[2 * is + 1] = 0;
     }
     __syncthreads();
-    if (c.warmStart) velocity_level_run<kPassWarm>(rec, P, 1, words, x.lane);
+    if (c.warmStart) velocity_level_run<kPassWarm>(v2, P.n, P.rb, P.rounds, P.period, 1, smem, wordsAt);
     if (overlap && iters > 0) {
-        velocity_level_run<kPassIterations>(rec, P, iters, words, x.lane);
+        velocity_level_run<kPassIterations>(v2, P.n, P.rb, P.rounds, P.period, iters, smem, wordsAt);
         __syncthreads();
     }
     // Islands to sweep again, on their lane or by plain iterations.
@@ -4445,7 +4689,7 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
                 for (int is = x.lane; is < nisl; is += kWave)
                     if (words[2 * is] == 1) words[2 * is] = kOut | 1;
                 __syncthreads();
-                velocity_level_run<kPassWarmMasked>(rec, P, 1, words, x.lane);
+                velocity_level_run<kPassWarmMasked>(v2, P.n, P.rb, P.rounds, P.period, 1, smem, wordsAt);
             }
         }
         for (int is = x.lane; is < nisl; is += kWave)
@@ -4453,7 +4697,7 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
         for (int it = 0; it < iters; ++it) {
             for (int is = x.lane; is < nisl; is += kWave) words[2 * is + 1] = 0;
             __syncthreads();
-            velocity_level_run<kPassMasked>(rec, P, 1, words, x.lane);
+            velocity_level_run<kPassMasked>(v2, P.n, P.rb, P.rounds, P.period, 1, smem, wordsAt);
             __syncthreads();
             bool going = false;
             for (int base = 0; base < nisl; base += kWave) {
@@ -4484,26 +4728,16 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
     __syncthreads();
 }
 
-// Position sweeps of the level islands, iteration after iteration; an island
-// solved by an iteration is left out of the later ones.
-template <class Level, class Add>
-__device__ __forceinline__ void position_levels(const DeviceState& d, const WorldCtx& x, const Bodies<true>& bs,
-                                                const IslandScratch& S, const LevelPlan& P, int nisl, Level level,
-                                                const StepParams& c, Add add) {
-    const int iters = int(c.posIters);
-    if (iters == 0) {
-        for (int is = x.lane; is < nisl; is += kWave) {
-            if (!level(is)) continue;
-            S.isl_word[is] = 0u;
-            add(PosResult{__builtin_inff(), 0}, true);
-        }
-        return;
-    }
-    const __amdgpu_buffer_rsrc_t table = rounds_rsrc(P);
-    const __amdgpu_buffer_rsrc_t rec = record_rsrc(d.s_pc2 + std::size_t(x.co) * prx::kQuadPc, P.n, prx::kQuadPc);
-    float* const lds = reinterpret_cast<float*>(g_smem);
-    int* const words = island_words(x);
-    const int j = x.lane >> 2, quad = x.lane & 3, comp = x.lane & 1;
+// One position iteration over the plan's rounds.
+__device__ __attribute__((noinline)) void position_level_run(float4* recs, int n, const int2* rb, int rounds, LdsWord* smem,
+                                                             int wordsAt, PositionConf c) {
+    rounds = __builtin_amdgcn_readfirstlane(rounds);
+    c = PositionConf{uniform_f(c.regResolutionRate), uniform_f(c.linearSlop), uniform_f(c.maxLinearCorrection)};
+    const __amdgpu_buffer_rsrc_t table = rounds_rsrc(uniform_ptr(rb), rounds);
+    const __amdgpu_buffer_rsrc_t rec = record_rsrc(uniform_ptr(recs), __builtin_amdgcn_readfirstlane(n), prx::kQuadPc);
+    float* const lds = reinterpret_cast<float*>((int*)smem);
+    int* const words = (int*)(smem + __builtin_amdgcn_readfirstlane(wordsAt));
+    const int lane = int(threadIdx.x), j = lane >> 2, quad = lane & 3, comp = lane & 1;
     constexpr int kStep = prx::kQuadPc * 16;
     struct At {
         int2 b;
@@ -4535,28 +4769,50 @@ __device__ __forceinline__ void position_levels(const DeviceState& d, const Worl
         // The wave's LDS operations run in order: nothing to wait for.
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     };
+    // A round's records are read while the round before is solved, and
+    // its bounds one round earlier still.
+    QuadPos a, b;
+    At atA, atB, atC;
+    bounds(0, atA);
+    bounds(1, atB);
+    fetch(atA, a);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // as in the velocity sweep
+    for (int k = 0; k < rounds; k += 2) {
+        bounds(k + 2, atC);
+        fetch(atB, b);
+        solve(atA.off, a);
+        bounds(k + 3, atA);
+        fetch(atC, a);
+        solve(atB.off, b);
+        atB = atA;
+        atA = atC;
+    }
+}
+
+// Position sweeps of the level islands, iteration after iteration; an island
+// solved by an iteration is left out of the later ones.
+template <class Level, class Add>
+__device__ __forceinline__ void position_levels(const DeviceState& d, const WorldCtx& x, const Bodies<true>& bs,
+                                                const IslandScratch& S, const LevelPlan& P, int nisl, Level level,
+                                                const StepParams& c, Add add) {
+    const int iters = int(c.posIters);
+    if (iters == 0) {
+        for (int is = x.lane; is < nisl; is += kWave) {
+            if (!level(is)) continue;
+            S.isl_word[is] = 0u;
+            add(PosResult{__builtin_inff(), 0}, true);
+        }
+        return;
+    }
+    float4* const recs = d.s_pc2 + std::size_t(x.co) * prx::kQuadPc;
+    int* const words = island_words(x);
+    LdsWord* const smem = (LdsWord*)reinterpret_cast<int*>(g_smem);
     for (int is = x.lane; is < nisl; is += kWave) words[2 * is + 1] = level(is) ? 0 : 1;
     for (int it = 0; it < iters; ++it) {
         for (int is = x.lane; is < nisl; is += kWave) words[2 * is] = 0x7f800000;  // key of +infinity
         __syncthreads();
-        // A round's records are read while the round before is solved, and
-        // its bounds one round earlier still.
-        QuadPos a, b;
-        At atA, atB, atC;
-        bounds(0, atA);
-        bounds(1, atB);
-        fetch(atA, a);
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // as in the velocity sweep
-        for (int k = 0; k < P.rounds; k += 2) {
-            bounds(k + 2, atC);
-            fetch(atB, b);
-            solve(atA.off, a);
-            bounds(k + 3, atA);
-            fetch(atC, a);
-            solve(atB.off, b);
-            atB = atA;
-            atA = atC;
-        }
+        position_level_run(recs, P.n, P.rb, P.rounds, smem, 8 * x.nb,
+                           PositionConf{c.regResolutionRate, c.linearSlop, c.maxLinearCorrection});
         __syncthreads();
         bool going = false;
         for (int base = 0; base < nisl; base += kWave) {
