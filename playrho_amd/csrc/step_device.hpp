@@ -4,6 +4,8 @@
 // (step_kernel.hip) and the single-large-world kernels (big_world.hip).
 #pragma once
 
+#include <type_traits>
+
 #include <hip/hip_runtime.h>
 
 #include "layout.hpp"
@@ -1501,7 +1503,8 @@ __device__ __forceinline__ bool joint_solve_velocity(Jc& j, float4& velA, float4
 
 // SolvePosition (RevoluteJointConf.cpp:333-433).  Returns whether the joint
 // is within tolerance.
-__device__ __forceinline__ bool joint_solve_position(const float4* u, float4& posA, float4& posB, const StepParams& c) {
+template <class Conf>
+__device__ __forceinline__ bool joint_solve_position(const float4* u, float4& posA, float4& posB, const Conf& c) {
     const float4 n = u[2], ms = u[4], la = u[6], ang = u[7];
     const float angularMass = n.z;
     const std::uint32_t flags = __float_as_uint(n.w) & 0xffu, limit = __float_as_uint(n.w) >> 8;
@@ -3504,12 +3507,27 @@ __device__ __forceinline__ float solve_velocity_one(Vc& vc, const BodyC& A, cons
     return mi;
 }
 
+// The next revolute joint's record, read while the current one is solved: from
+// memory it takes as long as the solve (a chain world of 32 joints: velocity
+// 505k -> 407k cycles a step).
+template <int kFirst, int kCount>
+struct JointAhead {
+    float4 r[kCount];
+    __device__ __forceinline__ void load(const float4* jbase, int e) {
+        const float4* u = jbase + std::size_t(e) * prx::kJcStride + kFirst;
+#pragma unroll
+        for (int k = 0; k < kCount; ++k) r[k] = u[k];
+    }
+};
+
 // One pass over an island's joints in island order: the warm start of
 // InitVelocity, or SolveVelocity (returns whether every joint left its
 // bodies' velocities unchanged).
 template <bool kLds, bool kKinds>
 __device__ __forceinline__ bool joints_velocity_k(float4* jbase, int j0, int j1, const Bodies<kLds>& bs, bool warm) {
     bool ok = true;
+    JointAhead<0, 6> cur;
+    if (!kKinds && j0 < j1) cur.load(jbase, j0);
     for (int e = j0; e < j1; ++e) {
         float4* u = jbase + std::size_t(e) * prx::kJcStride;
         const std::uint32_t kind = kKinds ? jc_kind(u) : prx::kJointRevolute;
@@ -3546,7 +3564,8 @@ __device__ __forceinline__ bool joints_velocity_k(float4* jbase, int j0, int j1,
             bs.set_vel(bB, vb);
             continue;
         }
-        Jc j = load_jc_velocity(u);
+        Jc j = load_jc_velocity(kKinds ? u : cur.r);
+        if constexpr (!kKinds) cur.load(jbase, e + 1 < j1 ? e + 1 : e);
         float4 va = bs.vel(j.bA);
         float4 vb = bs.vel(j.bB);
         if (warm) {
@@ -3591,9 +3610,12 @@ template <bool kLds>
 __device__ __forceinline__ bool joints_velocity_tape(float4* jbase, int j0, int j1, const Bodies<kLds>& bs,
                                                      const prx::Tape& t, int jo, int it) {
     bool ok = true;
+    JointAhead<0, 6> cur;
+    if (j0 < j1) cur.load(jbase, j0);
     for (int e = j0; e < j1; ++e) {
         float4* u = jbase + std::size_t(e) * prx::kJcStride;
-        Jc j = load_jc_velocity(u);
+        Jc j = load_jc_velocity(cur.r);
+        cur.load(jbase, e + 1 < j1 ? e + 1 : e);
         float4 va = bs.vel(j.bA);
         float4 vb = bs.vel(j.bB);
         float4* g = t.jgs + ((std::size_t(jo) + std::size_t(e)) * std::size_t(t.itV) + std::size_t(it)) * 3;
@@ -3650,8 +3672,12 @@ template <bool kLds>
 __device__ __forceinline__ bool joints_position_tape(const float4* jbase, int j0, int j1, const Bodies<kLds>& bs,
                                                      const StepParams& c, const prx::Tape& t, int jo, int it) {
     bool ok = true;
+    JointAhead<0, 8> next, cur;
+    if (j0 < j1) next.load(jbase, j0);
     for (int e = j0; e < j1; ++e) {
-        const float4* u = jbase + std::size_t(e) * prx::kJcStride;
+        cur = next;
+        next.load(jbase, e + 1 < j1 ? e + 1 : e);
+        const float4* u = cur.r;
         const float4 mo = u[5];
         const int bA = __float_as_int(mo.z), bB = __float_as_int(mo.w);
         float4 pa = bs.pos(bA);
@@ -3984,9 +4010,9 @@ __device__ __forceinline__ PosResult island_position_wave(const DeviceState& d, 
 // same maxima and minima.  One plan serves all the islands of a world at once
 // (they share no moving body): it is built once per step and serves the warm
 // start, the velocity iterations and the position iterations.  It sorts the
-// updates by level into rounds of at most kLevelRound updates of one level;
+// updates by level into rounds of at most `width` updates of one level;
 // the records are copied into that order so that a round reads consecutive
-// records.  Islands of fewer than kLevelMinConstraints contacts stay on a
+// records.  Islands of fewer than kLevelMinConstraints updates stay on a
 // lane each: they would widen the first levels and cost more rounds than the
 // lanes they free.
 //
@@ -3996,17 +4022,22 @@ __device__ __forceinline__ PosResult island_position_wave(const DeviceState& d, 
 // period is the most rounds any body's updates of one iteration span, each
 // body still sees its updates in order.  Pile islands of 100 to 530 contacts
 // have 62 to 243 levels (at most 9 updates wide) and periods of 25 to 207, so
-// two iterations run side by side, each on half of the wave (kLevelGroups),
-// and eight iterations take rounds + 7 periods instead of 8 rounds: 1.1 to
-// 2.1 times fewer.
+// two iterations run side by side, each on half of the wave (kLevelRound), and
+// eight iterations take rounds + 7 periods instead of 8 rounds: 1.1 to 2.1
+// times fewer.  A joint chain is one update wide and each body leaves it after
+// a few rounds: worlds with joints run four iterations side by side
+// (kJointRound).  Chain worlds of 32 links with 54 to 85 contacts: periods of
+// 7 to 24 rounds, 120 to 221 rounds for the eight iterations, 170 to 224 with
+// two side by side, and 300 to 400 one after another.
 constexpr int kLevelMaxBodies = prx::kStageFloat4 * 4;
 constexpr int kLevelMinConstraints = 4;
-constexpr int kLevelGroups = 2;
 // Updates per round: four lanes serve one update.
-constexpr int kLevelRound = kWave / 4 / kLevelGroups;
+constexpr int kLevelRound = 8;
+constexpr int kJointRound = 4;
 
 struct LevelPlan {
     int n, rounds, period;
+    int width;         // most updates of a round
     const int2* rb;    // per round: first position in level order, updates
     const int* order;  // level position -> island-order slot
 };
@@ -4090,9 +4121,42 @@ __device__ __forceinline__ void store_quad_pc(float4* o, const Pc& pc, int islan
                   __uint_as_float(pc.m.type | (pc.m.n << 8) | (std::uint32_t(island) << 16)), 0.0f};
 }
 
+// Records of a revolute joint in level order, in the same places as a contact's:
+// velocity
+//   [0] [1] per lane: its body's arm
+//   [2] [3] as a contact's
+//   [5] [6] mass matrix, motor mass and speed; [7] largest motor impulse, -, -,
+//           kJointTag | flags | limit << 3 | island << 8; [9] the impulses
+// position (A is X, B is Y)
+//   [0] [1] as a contact's
+//   [2] [3] A: local anchor, reference angle, lower limit; upper limit, motor mass
+//   [4] [5] B: the same with its own anchor
+//   [6]     -, -, kJointTag | flags << 8 | limit << 11 | island << 16
+constexpr std::uint32_t kJointTag = 0x80u;
+__device__ __forceinline__ void store_quad_joint(float4* v, float4* o, const float4* u, int nb, int island) {
+    const float4 r = u[0], m = u[1], n = u[2], ms = u[4], mo = u[5], la = u[6], ang = u[7];
+    const std::uint32_t flags = __float_as_uint(n.w) & 0x7u, limit = __float_as_uint(n.w) >> 8;
+    const int bA = __float_as_int(mo.z), bB = __float_as_int(mo.w);
+    v[0] = float4{r.x, r.y, r.x, r.y};
+    v[1] = float4{r.z, r.w, r.z, r.w};
+    v[2] = float4{-ms.x, -ms.y, __int_as_float(4 * (nb + bA)), 0.0f};
+    v[3] = float4{ms.z, ms.w, __int_as_float(4 * (nb + bB)), 0.0f};
+    v[5] = m;
+    v[6] = float4{n.x, n.y, n.z, mo.x};
+    v[7] = float4{mo.y, 0.0f, 0.0f, __uint_as_float(kJointTag | flags | (limit << 3) | (std::uint32_t(island) << 8))};
+    v[9] = u[3];
+    o[0] = float4{__int_as_float(4 * bA), -ms.x, -ms.y, 0.0f};
+    o[1] = float4{__int_as_float(4 * bB), ms.z, ms.w, 0.0f};
+    o[2] = float4{la.x, la.y, ang.x, ang.y};
+    o[4] = float4{la.z, la.w, ang.x, ang.y};
+    o[3] = o[5] = float4{ang.z, n.z, 0.0f, 0.0f};
+    o[6] = float4{0.0f, 0.0f, __uint_as_float(kJointTag | (flags << 8) | (limit << 11) | (std::uint32_t(island) << 16)), 0.0f};
+}
+
 // Builds the plan of the slots whose island (LevelScratch::island) is not
-// negative; the record stage serves as the per-body tables.
-__device__ __forceinline__ LevelPlan level_plan(const DeviceState& d, const WorldCtx& x, float4* stage, int nce) {
+// negative, the joints (slots from nce on) before the contacts, as a velocity
+// iteration runs them; the record stage serves as the per-body tables.
+__device__ __forceinline__ LevelPlan level_plan(const DeviceState& d, const WorldCtx& x, float4* stage, int nce, int nje) {
     const int lane = x.lane;
     const float4* vbase = d.s_vc + std::size_t(x.co) * prx::kVcStride;
     const float4* pbase = d.s_pc + std::size_t(x.co) * prx::kPcStride;
@@ -4100,22 +4164,29 @@ __device__ __forceinline__ LevelPlan level_plan(const DeviceState& d, const Worl
     int* last = reinterpret_cast<int*>(stage);
     for (int b = lane; b < x.nb; b += kWave) last[b] = 0;
     int n = 0;
-    for (int base = 0; base < nce; base += kWave) {
-        const bool in = base + lane < nce && L.island[base + lane] >= 0;
-        const unsigned long long m = __ballot(in);
-        if (in) L.sel[n + __popcll(m & lanes_below(lane))] = base + lane;
-        n += __popcll(m);
-    }
+    auto select = [&](int from, int to) {
+        for (int base = from; base < to; base += kWave) {
+            const bool in = base + lane < to && L.island[base + lane] >= 0;
+            const unsigned long long m = __ballot(in);
+            if (in) L.sel[n + __popcll(m & lanes_below(lane))] = base + lane;
+            n += __popcll(m);
+        }
+    };
+    select(nce, nce + nje);
+    select(0, nce);
+    const float4* jbase = d.s_jc + std::size_t(x.jo) * prx::kJcStride;
     __syncthreads();
     int levels = 0;
     for (int base = 0; base < n; base += kWave) {
         const int r = base + lane;
         int a = -1, bb = -1;
         if (r < n) {
-            const float4* v = vbase + std::size_t(L.sel[r]) * prx::kVcStride;
-            const float4 m = v[8];
-            if (m.x != 0.0f || m.y != 0.0f) a = __float_as_int(v[2].w);
-            if (m.z != 0.0f || m.w != 0.0f) bb = __float_as_int(v[5].z);
+            const int slot = L.sel[r];
+            const bool joint = slot >= nce;
+            const float4* v = joint ? jbase + std::size_t(slot - nce) * prx::kJcStride : vbase + std::size_t(slot) * prx::kVcStride;
+            const float4 m = v[joint ? 4 : 8];
+            if (m.x != 0.0f || m.y != 0.0f) a = __float_as_int(joint ? v[5].z : v[2].w);
+            if (m.z != 0.0f || m.w != 0.0f) bb = __float_as_int(joint ? v[5].w : v[5].z);
         }
         const int cnt = (n - base < kWave) ? n - base : kWave;
         int mine = 0;
@@ -4156,15 +4227,16 @@ __device__ __forceinline__ LevelPlan level_plan(const DeviceState& d, const Worl
     __syncthreads();
     for (int r = lane; r < n; r += kWave) L.order[atomicAdd(&cur[L.lvl[r]], 1)] = L.sel[r];
     __syncthreads();
+    const int width = nje > 0 ? kJointRound : kLevelRound;
     int rounds = 0;
     for (int base = 0; base < levels; base += kWave) {
         const int k = base + lane;
         const int cnt = (k < levels) ? L.start[k + 1] - L.start[k] : 0;
-        const int nr = (cnt + kLevelRound - 1) / kLevelRound;
+        const int nr = (cnt + width - 1) / width;
         const int incl = wave_incl_scan(nr, lane);
         for (int i = 0; i < nr; ++i) {
-            const int b = L.start[k] + i * kLevelRound;
-            const int e = (b + kLevelRound < L.start[k + 1]) ? b + kLevelRound : L.start[k + 1];
+            const int b = L.start[k] + i * width;
+            const int e = (b + width < L.start[k + 1]) ? b + width : L.start[k + 1];
             L.rb[rounds + incl - nr + i] = int2{b, e - b};
         }
         rounds += __shfl(incl, kWave - 1);
@@ -4174,6 +4246,14 @@ __device__ __forceinline__ LevelPlan level_plan(const DeviceState& d, const Worl
     float4* p2 = d.s_pc2 + std::size_t(x.co) * prx::kQuadPc;
     for (int pos = lane; pos < n; pos += kWave) {
         const int slot = L.order[pos], is = L.island[slot];
+        if (slot >= nce) {
+            const float4* u = jbase + std::size_t(slot - nce) * prx::kJcStride;
+            const float4 ms = u[4], mo = u[5];
+            store_quad_joint(v2 + std::size_t(pos) * prx::kQuadVc, p2 + std::size_t(pos) * prx::kQuadPc, u, x.nb, is);
+            L.lvl[pos] = ((ms.x != 0.0f || ms.y != 0.0f) ? __float_as_int(mo.z) : 0xffff) |
+                         (((ms.z != 0.0f || ms.w != 0.0f) ? __float_as_int(mo.w) : 0xffff) << 16);
+            continue;
+        }
         BodyC A, B;
         const Vc vc = load_vc(vbase + std::size_t(slot) * prx::kVcStride, A, B);
         store_quad_vc(v2 + std::size_t(pos) * prx::kQuadVc, vc, A, B, x.nb, is);
@@ -4204,9 +4284,10 @@ __device__ __forceinline__ LevelPlan level_plan(const DeviceState& d, const Worl
     for (int off = kWave / 2; off > 0; off >>= 1) period = max(period, __shfl_xor(period, off));
     // A group ends an iteration before it starts its next, and a record's
     // impulses are stored before the next iteration reads them.
-    period = max(period, max((rounds + kLevelGroups - 1) / kLevelGroups, 2));
+    const int groups = kWave / 4 / width;
+    period = max(period, max((rounds + groups - 1) / groups, 2));
     __syncthreads();
-    return LevelPlan{n, __builtin_amdgcn_readfirstlane(rounds), __builtin_amdgcn_readfirstlane(period), L.rb, L.order};
+    return LevelPlan{n, __builtin_amdgcn_readfirstlane(rounds), __builtin_amdgcn_readfirstlane(period), width, L.rb, L.order};
 }
 
 constexpr int kOutOfRange = 0x40000000;  // a buffer offset past every island's records
@@ -4324,9 +4405,55 @@ __device__ __forceinline__ void quad_block(QuadBody& me, const QuadRec& r, int l
     maxInc = fmax_std(maxInc, fmax_std(__builtin_fabsf(n0), __builtin_fabsf(n1)));
 }
 
+// A revolute joint's warm start or velocity update, computed whole by each of
+// its four lanes (joint_warm_start, joint_solve_velocity): the bodies' values
+// and masses come from the quad, each lane keeps its component.  vOther: the
+// lane's body's other velocity component.
+constexpr int kJointMoved = 2;  // a masked run's mark in an island's first word
+template <bool kWarm>
+__device__ __forceinline__ bool quad_joint(QuadBody& me, QuadRec& r, int quad, float vOther, unsigned tag) {
+    const bool compY = quad & 1;
+    const float vx = compY ? vOther : me.v, vy = compY ? me.v : vOther;
+    auto a = [](float v) { return quad_move<0x44>(v); };  // from A: lanes 0 1 0 1
+    auto b = [](float v) { return from_b(v); };
+    Jc j;
+    j.rA = V2{a(r.q.x), a(r.q.y)};
+    j.rB = V2{b(r.q.x), b(r.q.y)};
+    j.A = BodyC{-a(me.sm), -a(me.si), V2{0, 0}};
+    j.B = BodyC{b(me.sm), b(me.si), V2{0, 0}};
+    j.ix = r.i.x;
+    j.iy = r.i.y;
+    j.iz = r.i.z;
+    j.motorImp = r.i.w;
+    float4 va{a(vx), a(vy), a(me.w), 0.0f}, vb{b(vx), b(vy), b(me.w), 0.0f};
+    bool same = true;
+    if constexpr (kWarm) {
+        joint_warm_start(j, va, vb);
+    } else {
+        j.exx = r.f.x;
+        j.eyx = r.f.y;
+        j.ezx = r.f.z;
+        j.eyy = r.f.w;
+        j.ezy = r.b.x;
+        j.ezz = r.b.y;
+        j.angularMass = r.b.z;
+        j.motorSpeed = r.b.w;
+        j.maxImpulse = r.k.x;
+        j.flags = tag & 0x7u;
+        j.limit = (tag >> 3) & 0x3u;
+        same = joint_solve_velocity(j, va, vb);
+        r.i = float4{j.ix, j.iy, j.iz, j.motorImp};
+    }
+    const float4 v = (quad & 2) ? vb : va;
+    me.v = compY ? v.y : v.x;
+    me.w = v.z;
+    return same;
+}
+
 // Iterations [0, iters) of the plan's velocity sweep, overlapped as its period
-// allows (one iteration: a plain pass).  Lane 32 g + 4 j + 2 s + c serves
-// update j of group g's round; group g runs iterations g, g + 2, ...  Bound by
+// allows (one iteration: a plain pass).  Lane 4 (width g + j) + 2 s + c serves
+// update j of group g's round (a group is 4 `width` lanes); group g runs iterations
+// g, g + groups, ...  Bound by
 // the instructions of one round after another, about 2000 cycles each (no other
 // wave of the world can help): a pile of 400 bodies takes 2.2M cycles for the
 // velocity sweeps and 1.2M for the position sweeps, from 3.1M and 1.8M with
@@ -4339,9 +4466,11 @@ __device__ __forceinline__ void quad_block(QuadBody& me, const QuadRec& r, int l
 // compiler places count exactly the operations in flight.  Islands marked in
 // their words are left out of a masked run.
 enum LevelPass { kPassWarm, kPassWarmMasked, kPassIterations, kPassMasked };
-template <LevelPass kPass>
+enum LevelItems { kContactItems, kJointItems, kAllItems };
+template <LevelPass kPass, LevelItems kItems>
 __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n, const int2* rb, int rounds, int period,
-                                                             int iters, LdsWord* smem, int wordsAt) {
+                                                             int width, int iters, LdsWord* smem, int wordsAt) {
+    width = __builtin_amdgcn_readfirstlane(width);
     rounds = __builtin_amdgcn_readfirstlane(rounds);
     period = __builtin_amdgcn_readfirstlane(period);
     iters = __builtin_amdgcn_readfirstlane(iters);
@@ -4352,7 +4481,9 @@ __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n
     const int lane = int(threadIdx.x);
     constexpr bool kWarm = kPass == kPassWarm || kPass == kPassWarmMasked;
     constexpr bool kMasked = kPass == kPassMasked || kPass == kPassWarmMasked;
-    const int group = lane >> 5, j = (lane >> 2) & (kLevelRound - 1), quad = lane & 3, comp = lane & 1;
+    const int shift = __builtin_ctz(unsigned(4 * width)), groups = kWave >> shift;
+    const int group = lane >> shift, j = (lane >> 2) & (width - 1), quad = lane & 3, comp = lane & 1;
+    const int turn = groups * period;
     constexpr int kStep = prx::kQuadVc * 16;
     int r = -group * period, it = group;  // the group's round and iteration at the tick read ahead
     struct At {
@@ -4363,9 +4494,9 @@ __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n
         const bool on = r >= 0 && it < iters;
         a.b = __builtin_bit_cast(int2, __builtin_amdgcn_raw_buffer_load_b64(table, on ? r * 8 : kOutOfRange, 0, 0));
         a.it = it;
-        if (++r == kLevelGroups * period) {
+        if (++r == turn) {
             r = 0;
-            it += kLevelGroups;
+            it += groups;
         }
     };
     auto f2 = [&](int off) {
@@ -4378,7 +4509,7 @@ __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n
         const int off = a.off = j < a.b.y ? (a.b.x + j) * kStep : kOutOfRange;
         q.q = f2(off + 8 * quad);
         q.s = f4(off + 32 + 8 * (quad & 2));
-        q.tn = f2(off + 64 + 8 * comp);
+        if constexpr (kItems != kJointItems) q.tn = f2(off + 64 + 8 * comp);
         if constexpr (!kWarm) {
             q.f = f4(off + 80);
             q.b = f4(off + 96);
@@ -4390,12 +4521,18 @@ __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n
     auto solve = [&](const At& at, QuadRec& q) {
         const int island = int(__float_as_uint(q.k.w) >> 8);
         bool on = at.off != kOutOfRange;
+        if constexpr (kItems != kAllItems) on = on && ((__float_as_uint(q.k.w) & kJointTag) != 0) == (kItems == kJointItems);
         if constexpr (kMasked) on = on && words[2 * island] >= 0;
         if (on) {
             const unsigned n = __float_as_uint(q.k.w) & 0xffu;
             const int vi = __float_as_int(q.s.z);
             QuadBody me{lds[vi + comp], lds[vi + 2], q.s.x, q.s.y};
-            if constexpr (kWarm) {
+            if (kItems != kContactItems && (n & kJointTag)) {
+                const bool same = quad_joint<kWarm>(me, q, quad, lds[vi + (comp ^ 1)], n);
+                if (!kWarm && quad == 2 && !same)
+                    atomicOr(&words[2 * island], kMasked ? kJointMoved : 1 << at.it);
+            } else if constexpr (kItems == kJointItems) {
+            } else if constexpr (kWarm) {
                 QuadBody dl{0.0f, 0.0f, q.s.x, q.s.y};
                 if (n > 0) {
                     const float Pn = q.i.x * q.tn.y + q.i.y * q.tn.x;
@@ -4461,7 +4598,7 @@ __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n
 }
 
 struct PositionConf {
-    float regResolutionRate, linearSlop, maxLinearCorrection;
+    float regResolutionRate, linearSlop, maxLinearCorrection, angularSlop, maxAngularCorrection;
 };
 
 // A position record as a lane holds it: this body, its points, the common part.
@@ -4583,6 +4720,30 @@ __device__ __forceinline__ float quad_position(const QuadPos& r, int quad, float
     return 0.0f + s0.sep;
 }
 
+// A revolute joint's position update (joint_solve_position), computed whole by
+// each of its four lanes; pOther: the lane's body's other component.  Returns
+// whether the joint is within its slops.
+constexpr int kJointOpen = int(0x80000000u);  // a joint is not, in an island's second word
+__device__ __forceinline__ bool quad_joint_position(const QuadPos& r, int quad, float& p, float pOther, float& ang,
+                                                    const PositionConf& c) {
+    const bool compY = quad & 1;
+    const float px = compY ? pOther : p, py = compY ? p : pOther;
+    auto a = [](float v) { return quad_move<0x44>(v); };
+    auto b = [](float v) { return from_b(v); };
+    const std::uint32_t h = __float_as_uint(r.k.z);
+    float4 u[8];
+    u[2] = float4{0.0f, 0.0f, r.v.y, __uint_as_float(((h >> 8) & 0x7u) | (((h >> 11) & 0x3u) << 8))};
+    u[4] = float4{-a(r.b.y), -a(r.b.z), b(r.b.y), b(r.b.z)};
+    u[6] = float4{a(r.u.x), a(r.u.y), b(r.u.x), b(r.u.y)};
+    u[7] = float4{r.u.z, r.u.w, r.v.x, 0.0f};
+    float4 pa{a(px), a(py), a(ang), 0.0f}, pb{b(px), b(py), b(ang), 0.0f};
+    const bool ok = joint_solve_position(u, pa, pb, c);
+    const float4 o = (quad & 2) ? pb : pa;
+    p = compY ? o.y : o.x;
+    ang = o.z;
+    return ok;
+}
+
 // Order-preserving integer images of floats, for minima.
 __device__ __forceinline__ int float_key(float f) {
     const int bits = __float_as_int(f);
@@ -4590,11 +4751,13 @@ __device__ __forceinline__ int float_key(float f) {
 }
 __device__ __forceinline__ float key_float(int key) { return __int_as_float(key >= 0 ? key : (key ^ 0x7fffffff)); }
 
-// The islands of a world that the level form sweeps: without joints, at least
-// kLevelMinConstraints contacts (or coopMin, if that is less; coopMin's
-// greatest value keeps every island on a lane).
-__device__ __forceinline__ bool level_island(int contacts, int joints, int coopMin) {
-    return joints == 0 && contacts >= (coopMin < kLevelMinConstraints ? coopMin : kLevelMinConstraints) &&
+// The islands of a world that the level form sweeps: at least
+// kLevelMinConstraints contacts and joints (or coopMin, if that is less;
+// coopMin's greatest value keeps every island on a lane), and no joints where
+// some joint of the batch is not revolute.
+__device__ __forceinline__ bool level_island(int contacts, int joints, int coopMin, bool revolute) {
+    return (joints == 0 || revolute) &&
+           contacts + joints >= (coopMin < kLevelMinConstraints ? coopMin : kLevelMinConstraints) &&
            coopMin != 0x7fffffff;
 }
 
@@ -4609,7 +4772,8 @@ struct SolveSummary {
 //
 // Overlapped iterations run past an island's early exit.  The exit's bound is
 // zero unless set otherwise: an island exits with the first iteration in which
-// no impulse changed (its bit in the island's word stays clear).  Such an
+// no impulse changed and no joint moved a body (its bit in the island's word
+// stays clear).  Such an
 // island is swept again from its starting velocities and impulses: the early
 // exit is what makes that short, so one below kLevelRedo contacts goes to its
 // lane, a larger one through plain iterations.  With a positive bound all
@@ -4617,14 +4781,24 @@ struct SolveSummary {
 constexpr int kLevelRedo = 32;
 template <class Level, class Add>
 __device__ __forceinline__ void velocity_levels(const DeviceState& d, const WorldCtx& x, const Bodies<true>& bs,
-                                                const IslandScratch& S, const LevelPlan& P, int nisl, Level level,
-                                                const StepParams& c, Add add) {
+                                                const IslandScratch& S, const LevelPlan& P, int nisl, int nce, bool joints,
+                                                Level level, const StepParams& c, Add add) {
     float4* v2 = d.s_vc2 + std::size_t(x.co) * prx::kQuadVc;
     float4* vbase = d.s_vc + std::size_t(x.co) * prx::kVcStride;
     const LevelScratch L(d, x);
     int* const words = island_words(x);
+    float4* jbase = d.s_jc + std::size_t(x.jo) * prx::kJcStride;
     LdsWord* const smem = (LdsWord*)reinterpret_cast<int*>(g_smem);
-    const int wordsAt = 8 * x.nb;
+    auto warm = [&](auto masked) {
+        constexpr LevelPass kPass = decltype(masked)::value ? kPassWarmMasked : kPassWarm;
+        velocity_level_run<kPass, kContactItems>(v2, P.n, P.rb, P.rounds, P.period, P.width, 1, smem, 8 * x.nb);
+        if (joints) velocity_level_run<kPass, kJointItems>(v2, P.n, P.rb, P.rounds, P.period, P.width, 1, smem, 8 * x.nb);
+    };
+    auto sweep = [&](auto masked, int n) {
+        constexpr LevelPass kPass = decltype(masked)::value ? kPassMasked : kPassIterations;
+        if (joints) velocity_level_run<kPass, kAllItems>(v2, P.n, P.rb, P.rounds, P.period, P.width, n, smem, 8 * x.nb);
+        else velocity_level_run<kPass, kContactItems>(v2, P.n, P.rb, P.rounds, P.period, P.width, n, smem, 8 * x.nb);
+    };
     constexpr int kOut = int(0x80000000u);  // left out of masked runs
     const int iters = int(c.velIters);
     const bool overlap = c.regMinMomentum <= 0.0f && iters <= 31;
@@ -4633,9 +4807,9 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
         words[2 * is + 1] = 0;
     }
     __syncthreads();
-    if (c.warmStart) velocity_level_run<kPassWarm>(v2, P.n, P.rb, P.rounds, P.period, 1, smem, wordsAt);
+    if (c.warmStart) warm(std::false_type{});
     if (overlap && iters > 0) {
-        velocity_level_run<kPassIterations>(v2, P.n, P.rb, P.rounds, P.period, iters, smem, wordsAt);
+        sweep(std::false_type{}, iters);
         __syncthreads();
     }
     // Islands to sweep again, on their lane or by plain iterations.
@@ -4648,7 +4822,7 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
             const bool exits = overlap && c.regMinMomentum == 0.0f && iters > 1 && ((words[2 * is] | (1 << (iters - 1))) & ran) != ran;
             plain = !overlap;
             if (exits) {
-                lane = S.istart[is + 1].y - S.istart[is].y < kLevelRedo;
+                lane = S.istart[is + 1].y - S.istart[is].y + S.jstart[is + 1] - S.jstart[is] < kLevelRedo;
                 plain = !lane;
             } else if (overlap) {
                 add(VelResult{__int_as_float(words[2 * is + 1]), iters});
@@ -4667,8 +4841,12 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
         for (int pos = x.lane; pos < P.n; pos += kWave) {
             const int slot = P.order[pos];
             if (words[2 * L.island[slot]] == 1) continue;
-            float4* dst = vbase + std::size_t(slot) * prx::kVcStride;
             const float4 i = v2[std::size_t(pos) * prx::kQuadVc + 9];
+            if (slot >= nce) {
+                jbase[std::size_t(slot - nce) * prx::kJcStride + 3] = i;
+                continue;
+            }
+            float4* dst = vbase + std::size_t(slot) * prx::kVcStride;
             dst[4].x = i.x;
             dst[4].y = i.y;
             dst[7].x = i.z;
@@ -4682,14 +4860,16 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
                 const int slot = P.order[pos];
                 if (words[2 * L.island[slot]] != 0) continue;
                 const float4* src = vbase + std::size_t(slot) * prx::kVcStride;
-                v2[std::size_t(pos) * prx::kQuadVc + 9] = float4{src[4].x, src[4].y, src[7].x, src[7].y};
+                v2[std::size_t(pos) * prx::kQuadVc + 9] =
+                    slot >= nce ? jbase[std::size_t(slot - nce) * prx::kJcStride + 3]
+                                : float4{src[4].x, src[4].y, src[7].x, src[7].y};
             }
             __syncthreads();
             if (c.warmStart) {
                 for (int is = x.lane; is < nisl; is += kWave)
                     if (words[2 * is] == 1) words[2 * is] = kOut | 1;
                 __syncthreads();
-                velocity_level_run<kPassWarmMasked>(v2, P.n, P.rb, P.rounds, P.period, 1, smem, wordsAt);
+                warm(std::true_type{});
             }
         }
         for (int is = x.lane; is < nisl; is += kWave)
@@ -4697,7 +4877,7 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
         for (int it = 0; it < iters; ++it) {
             for (int is = x.lane; is < nisl; is += kWave) words[2 * is + 1] = 0;
             __syncthreads();
-            velocity_level_run<kPassMasked>(v2, P.n, P.rb, P.rounds, P.period, 1, smem, wordsAt);
+            sweep(std::true_type{}, 1);
             __syncthreads();
             bool going = false;
             for (int base = 0; base < nisl; base += kWave) {
@@ -4706,7 +4886,7 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
                 if (on) {
                     // The island's sums so far: its largest change in stat words.
                     const float inc = __int_as_float(words[2 * is + 1]);
-                    const bool done = inc <= c.regMinMomentum || it + 1 == iters;
+                    const bool done = (inc <= c.regMinMomentum && !(words[2 * is] & kJointMoved)) || it + 1 == iters;
                     add(VelResult{inc, done ? it + 1 : 0});
                     words[2 * is] = done ? kOut : 0;
                     on = !done;
@@ -4723,16 +4903,19 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
     if (anyLane) {
         for (int is = x.lane; is < nisl; is += kWave)
             if (level(is) && words[2 * is] == 1)
-                add(island_velocity<true>(d, x, bs, S.istart[is].y, S.istart[is + 1].y, 0, 0, c));
+                add(island_velocity<true>(d, x, bs, S.istart[is].y, S.istart[is + 1].y, S.jstart[is], S.jstart[is + 1], c));
     }
     __syncthreads();
 }
 
-// One position iteration over the plan's rounds.
+// One position iteration over the plan's rounds: the contacts' or the joints'
+// updates of it (the contacts go first here).
+template <bool kJoints>
 __device__ __attribute__((noinline)) void position_level_run(float4* recs, int n, const int2* rb, int rounds, LdsWord* smem,
                                                              int wordsAt, PositionConf c) {
     rounds = __builtin_amdgcn_readfirstlane(rounds);
-    c = PositionConf{uniform_f(c.regResolutionRate), uniform_f(c.linearSlop), uniform_f(c.maxLinearCorrection)};
+    c = PositionConf{uniform_f(c.regResolutionRate), uniform_f(c.linearSlop), uniform_f(c.maxLinearCorrection),
+                     uniform_f(c.angularSlop), uniform_f(c.maxAngularCorrection)};
     const __amdgpu_buffer_rsrc_t table = rounds_rsrc(uniform_ptr(rb), rounds);
     const __amdgpu_buffer_rsrc_t rec = record_rsrc(uniform_ptr(recs), __builtin_amdgcn_readfirstlane(n), prx::kQuadPc);
     float* const lds = reinterpret_cast<float*>((int*)smem);
@@ -4758,13 +4941,19 @@ __device__ __attribute__((noinline)) void position_level_run(float4* recs, int n
     };
     auto solve = [&](int off, const QuadPos& q) {
         const int island = int(__float_as_uint(q.k.z) >> 16);
-        if (off != kOutOfRange && words[2 * island + 1] == 0) {
+        const bool joint = (__float_as_uint(q.k.z) & kJointTag) != 0;
+        if (off != kOutOfRange && joint == kJoints && (words[2 * island + 1] & ~kJointOpen) == 0) {
             const int at = __float_as_int(q.b.x);
             float p = lds[at + comp], a = lds[at + 2];
-            const float sep = quad_position(q, quad, p, a, c);
+            if constexpr (kJoints) {
+                const bool solved = quad_joint_position(q, quad, p, lds[at + (comp ^ 1)], a, c);
+                if (quad == 0 && !solved) atomicOr(&words[2 * island + 1], kJointOpen);
+            } else {
+                const float sep = quad_position(q, quad, p, a, c);
+                if (quad == 0 && sep < __builtin_inff()) atomicMin(&words[2 * island], float_key(sep));
+            }
             lds[at + comp] = p;
             lds[at + 2] = a;
-            if (quad == 0 && sep < __builtin_inff()) atomicMin(&words[2 * island], float_key(sep));
         }
         // The wave's LDS operations run in order: nothing to wait for.
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -4793,8 +4982,8 @@ __device__ __attribute__((noinline)) void position_level_run(float4* recs, int n
 // solved by an iteration is left out of the later ones.
 template <class Level, class Add>
 __device__ __forceinline__ void position_levels(const DeviceState& d, const WorldCtx& x, const Bodies<true>& bs,
-                                                const IslandScratch& S, const LevelPlan& P, int nisl, Level level,
-                                                const StepParams& c, Add add) {
+                                                const IslandScratch& S, const LevelPlan& P, int nisl, bool joints,
+                                                Level level, const StepParams& c, Add add) {
     const int iters = int(c.posIters);
     if (iters == 0) {
         for (int is = x.lane; is < nisl; is += kWave) {
@@ -4811,17 +5000,18 @@ __device__ __forceinline__ void position_levels(const DeviceState& d, const Worl
     for (int it = 0; it < iters; ++it) {
         for (int is = x.lane; is < nisl; is += kWave) words[2 * is] = 0x7f800000;  // key of +infinity
         __syncthreads();
-        position_level_run(recs, P.n, P.rb, P.rounds, smem, 8 * x.nb,
-                           PositionConf{c.regResolutionRate, c.linearSlop, c.maxLinearCorrection});
+        const PositionConf pc{c.regResolutionRate, c.linearSlop, c.maxLinearCorrection, c.angularSlop, c.maxAngularCorrection};
+        position_level_run<false>(recs, P.n, P.rb, P.rounds, smem, 8 * x.nb, pc);
+        if (joints) position_level_run<true>(recs, P.n, P.rb, P.rounds, smem, 8 * x.nb, pc);
         __syncthreads();
         bool going = false;
         for (int base = 0; base < nisl; base += kWave) {
             const int is = base + x.lane;
-            bool on = is < nisl && words[2 * is + 1] == 0;
+            bool on = is < nisl && (words[2 * is + 1] & ~kJointOpen) == 0;
             if (on) {
                 const float minSep = key_float(words[2 * is]);
-                const bool solved = minSep >= c.regMinSeparation;
-                if (solved) words[2 * is + 1] = it + 1;
+                const bool solved = minSep >= c.regMinSeparation && words[2 * is + 1] == 0;
+                words[2 * is + 1] = solved ? it + 1 : 0;
                 on = !solved && it + 1 < iters;
                 if (!on) S.isl_word[is] = solved ? std::uint32_t(it + 1) : 0u;
                 add(PosResult{minSep, solved ? it + 1 : 0}, !on);
@@ -4967,11 +5157,12 @@ __device__ __forceinline__ SolveSummary solve_islands(const DeviceState& d, cons
     // The level form needs the body state and two words per island in LDS.
     const bool levels = kLds && !kTape && x.nb <= kLevelMaxBodies &&
                         x.nb * 40 + prx::kStageFloat4 * 16 <= int(c.ldsBytes);
+    const bool revolute = c.jointKinds == 0 && nce + nje <= x.cap;
     auto level = [&](int is) {
-        return levels && level_island(S.istart[is + 1].y - S.istart[is].y, S.jstart[is + 1] - S.jstart[is], coopMin);
+        return levels && level_island(S.istart[is + 1].y - S.istart[is].y, S.jstart[is + 1] - S.jstart[is], coopMin, revolute);
     };
     bool anyLevel = false;
-    LevelPlan plan{0, 0, 0, nullptr, nullptr};
+    LevelPlan plan{0, 0, 0, 0, nullptr, nullptr};
     if constexpr (kLds && !kTape) {
         const LevelScratch L(d, x);
         for (int base = 0; base < nisl; base += kWave) {
@@ -4979,12 +5170,14 @@ __device__ __forceinline__ SolveSummary solve_islands(const DeviceState& d, cons
             const bool lv = is < nisl && level(is);
             if (is < nisl)
                 for (int e = S.istart[is].y; e < S.istart[is + 1].y; ++e) L.island[e] = lv ? is : -1;
+            if (is < nisl && revolute)
+                for (int e = S.jstart[is]; e < S.jstart[is + 1]; ++e) L.island[nce + e] = lv ? is : -1;
             anyLevel = anyLevel || __ballot(lv) != 0;
         }
         __syncthreads();
         if (anyLevel) {
-            plan = level_plan(d, x, stage, nce);
-            velocity_levels(d, x, bs, S, plan, nisl, level, c, addVel);
+            plan = level_plan(d, x, stage, nce, revolute ? nje : 0);
+            velocity_levels(d, x, bs, S, plan, nisl, nce, revolute && nje > 0, level, c, addVel);
         }
     }
     for (int is = x.lane; is < nisl; is += kWave) {
@@ -5021,7 +5214,7 @@ __device__ __forceinline__ SolveSummary solve_islands(const DeviceState& d, cons
         // An island's smallest separation is over all its iterations; its
         // result is counted with the last.
         if (anyLevel)
-            position_levels(d, x, bs, S, plan, nisl, level, c, [&](const PosResult& r, bool last) {
+            position_levels(d, x, bs, S, plan, nisl, revolute && nje > 0, level, c, [&](const PosResult& r, bool last) {
                 if (last) addPos(r);
                 else aMin = fmin_std(aMin, r.minSep);
             });

@@ -33,7 +33,18 @@ CASES = [
     ("pile", [2, 1, 64, 64], 90, dict(do_warm_start=0)),
     ("pyramid", [8], 60, dict(do_blocksolve=0)),
     ("terrain", [1, 0], 120, {}),
-    ("chain", [1, 0], 90, {}),
+    # Islands with joints: all revolute (level form), limits and motors among
+    # them, contacts piled on them; early exits; kinds that stay on a lane.
+    ("chain", [1, 0], 150, {}),
+    ("chain", [1, 1, 4, 0], 60, {}),
+    ("chain", [1, 2, 3, 0], 60, {}),
+    ("chain", [2, 0, 32, 64], 220, {}),
+    ("chain", [2, 1, 12, 30, 0], 150, dict(reg_min_momentum=0.02)),
+    ("chain", [2, 2, 12, 30], 150, dict(reg_min_momentum=-1.0, do_warm_start=0)),
+    ("chain", [2, 3, 12, 30], 120, dict(reg_velocity_iters=32, reg_position_iters=1)),
+    ("joints", [1, 0], 150, {}),
+    ("joints", [2, 1, 3, 40], 150, dict(reg_min_momentum=0.02)),
+    ("gears", [1, 0], 90, {}),
 ]
 
 
