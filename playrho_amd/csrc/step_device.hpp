@@ -4071,13 +4071,14 @@ __device__ __forceinline__ int* island_words(const WorldCtx& x) { return reinter
 //           points 0 and 1 from body s
 //   [2] [3] per body: -+ inverse mass, -+ inverse rotational inertia (negative
 //           for A: its changes are added with the sign flipped), the LDS
-//           float index of its velocity
+//           float index of its velocity, M01
 //   [4]     tangent x, normal x, tangent y, normal y
 //   [5]     friction, tangent speed, tangent masses of points 0, 1
 //   [6]     biases 0, 1, normal masses 0, 1
-//   [7]     K00, K11, K01, points | island << 8
-//   [8]     M00, M11, M01, -
+//   [7]     K00, K11, K01, kPoint1 | kBlockSolve | island << 8
+//   [8]     M00, M11, the update's iteration bits and largest increment (below)
 //   [9]     normal and tangent impulse of point 0, of point 1
+constexpr std::uint32_t kPoint1 = 2u, kBlockSolve = 4u;
 __device__ __forceinline__ void store_quad_vc(float4* o, const Vc& vc, const BodyC& A, const BodyC& B, int nb, int island) {
     const V2 tg = fwdperp(vc.normal);
     auto q = [](V2 r0, V2 r1) {
@@ -4086,13 +4087,16 @@ __device__ __forceinline__ void store_quad_vc(float4* o, const Vc& vc, const Bod
     };
     o[0] = q(vc.p[0].relA, vc.p[1].relA);
     o[1] = q(vc.p[0].relB, vc.p[1].relB);
-    o[2] = float4{-A.invMass, -A.invRotI, __int_as_float(4 * (nb + vc.bA)), 0.0f};
-    o[3] = float4{B.invMass, B.invRotI, __int_as_float(4 * (nb + vc.bB)), 0.0f};
+    o[2] = float4{-A.invMass, -A.invRotI, __int_as_float(4 * (nb + vc.bA)), vc.M01};
+    o[3] = float4{B.invMass, B.invRotI, __int_as_float(4 * (nb + vc.bB)), vc.M01};
     o[4] = float4{tg.x, vc.normal.x, tg.y, vc.normal.y};
     o[5] = float4{vc.friction, vc.tangentSpeed, vc.p[0].tm, vc.p[1].tm};
     o[6] = float4{vc.p[0].bias, vc.p[1].bias, vc.p[0].nm, vc.p[1].nm};
-    o[7] = float4{vc.K00, vc.K11, vc.K01, __uint_as_float(vc.n | (std::uint32_t(island) << 8))};
-    o[8] = float4{vc.M00, vc.M11, vc.M01, 0.0f};
+    const bool block = vc.n > 1 && !(vc.K00 == 0.0f && vc.K11 == 0.0f && vc.K01 == 0.0f);
+    o[7] = float4{vc.K00, vc.K11, vc.K01,
+                  __uint_as_float((vc.n > 1 ? kPoint1 : 0u) | (block ? kBlockSolve : 0u) |
+                                  (std::uint32_t(island) << 8))};
+    o[8] = float4{vc.M00, vc.M11, 0.0f, 0.0f};
     o[9] = float4{vc.p[0].ni, vc.p[0].ti, vc.p[1].ni, vc.p[1].ti};
 }
 
@@ -4144,6 +4148,7 @@ __device__ __forceinline__ void store_quad_joint(float4* v, float4* o, const flo
     v[5] = m;
     v[6] = float4{n.x, n.y, n.z, mo.x};
     v[7] = float4{mo.y, 0.0f, 0.0f, __uint_as_float(kJointTag | flags | (limit << 3) | (std::uint32_t(island) << 8))};
+    v[8] = float4{0.0f, 0.0f, 0.0f, 0.0f};
     v[9] = u[3];
     o[0] = float4{__int_as_float(4 * bA), -ms.x, -ms.y, 0.0f};
     o[1] = float4{__int_as_float(4 * bB), ms.z, ms.w, 0.0f};
@@ -4304,6 +4309,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rounds_rsrc(const int2* rb, in
 }
 
 using U4 = __attribute__((ext_vector_type(4))) unsigned;
+using U2 = __attribute__((ext_vector_type(2))) unsigned;
 
 // Exchanges within an update's four lanes (2 s + c).
 template <int kPerm>
@@ -4338,71 +4344,92 @@ struct QuadBody {
         w = w + si * L;
     }
 };
-// Normal or tangential relative velocity on body B's lanes.
-__device__ __forceinline__ float quad_closing(const QuadBody& me, float q, float dir) {
-    const float u = me.v + q * me.w;
-    const float m = (u - other_body(u)) * dir;
+// Normal or tangential relative velocity, on all four lanes: body A's are
+// negated before the exchange, so that both bodies' lanes add B's and minus A's
+// (a + b and b + a, x - y and x + -y are the same to the bit).
+__device__ __forceinline__ float quad_closing(const QuadBody& me, float q, float dir, float sign) {
+    const float u = sign * (me.v + q * me.w);
+    const float m = (u + other_body(u)) * dir;
     return (0.0f + m) + other_comp(m);
 }
 __device__ __forceinline__ float quad_arm(float q, float P) {
     const float m = q * P;
     return m + other_comp(m);
 }
-__device__ __forceinline__ void quad_tangent(QuadBody& me, const QuadRec& r, float q, float tm, float ni, float& ti,
+// maxInc is never a NaN, so the larger number is what fmax_std gives.
+__device__ __forceinline__ void quad_tangent(QuadBody& me, const QuadRec& r, float sign, float q, float tm, float ni, float& ti,
                                              float& maxInc) {
-    const float lambda = tm * (r.f.y - quad_closing(me, q, r.tn.x));
+    const float lambda = tm * (r.f.y - quad_closing(me, q, r.tn.x, sign));
     const float maxI = r.f.x * ni;
-    const float inc = from_b(clamp_std(ti + lambda, -maxI, maxI) - ti);
+    const float inc = clamp_std(ti + lambda, -maxI, maxI) - ti;
     const float P = inc * r.tn.x;
     me.apply(P, quad_arm(q, P));
-    maxInc = fmax_std(maxInc, __builtin_fabsf(inc));
+    maxInc = fmaxf(maxInc, __builtin_fabsf(inc));
     ti = ti + inc;
 }
-__device__ __forceinline__ void quad_normal(QuadBody& me, const QuadRec& r, float q, float nm, float bias, float& ni,
+__device__ __forceinline__ void quad_normal(QuadBody& me, const QuadRec& r, float sign, float q, float nm, float bias, float& ni,
                                             float& maxInc) {
-    const float lambda = nm * (bias - quad_closing(me, q, r.tn.y));
-    const float inc = from_b(fmax_std(ni + lambda, 0.0f) - ni);
+    const float lambda = nm * (bias - quad_closing(me, q, r.tn.y, sign));
+    const float inc = fmax_std(ni + lambda, 0.0f) - ni;
     const float P = inc * r.tn.y;
     me.apply(P, quad_arm(q, P));
-    maxInc = fmax_std(maxInc, __builtin_fabsf(inc));
+    maxInc = fmaxf(maxInc, __builtin_fabsf(inc));
     ni = ni + inc;
 }
-__device__ __forceinline__ void quad_block(QuadBody& me, const QuadRec& r, int lane, float& ni0, float& ni1, float& maxInc) {
-    const float vn0 = quad_closing(me, r.q.x, r.tn.y);
-    const float vn1 = quad_closing(me, r.q.y, r.tn.y);
-    float t0 = 0.0f;
-    t0 += r.k.x * ni0;
-    t0 += r.k.z * ni1;
-    float t1 = 0.0f;
-    t1 += r.k.z * ni0;
-    t1 += r.k.y * ni1;
-    const float bx = (vn0 - r.b.x) - t0, by = (vn1 - r.b.y) - t1;
-    float x0 = 0.0f;
-    x0 += r.m.x * bx;
-    x0 += r.m.z * by;
-    float x1 = 0.0f;
-    x1 += r.m.z * bx;
-    x1 += r.m.y * by;
-    const float c1n0 = -x0, c1n1 = -x1;
-    const bool ok1 = c1n0 >= 0.0f && c1n1 >= 0.0f;
-    const float c2n0 = -r.b.z * bx;
-    const bool ok2 = c2n0 >= 0.0f && r.k.z * c2n0 + by >= 0.0f;
-    const float c3n1 = -r.b.w * by;
-    const bool ok3 = c3n1 >= 0.0f && r.k.z * c3n1 + bx >= 0.0f;
-    const bool ok4 = bx >= 0.0f && by >= 0.0f;
-    const float n0 = ok1 ? c1n0 : (ok2 ? c2n0 : 0.0f);
-    const float n1 = ok1 ? c1n1 : (ok2 ? 0.0f : (ok3 ? c3n1 : 0.0f));
-    const float d0 = from_b(n0 - ni0), d1 = from_b(n1 - ni1);
-    const float P0 = d0 * r.tn.y, P1 = d1 * r.tn.y;
+// The normal impulses: solve_dir of a single point or block_solve of two, lanes
+// of either kind in one pass (what both need once, the block solve's own part
+// where some lane has it).  Returns whether a block solve's impulse changed
+// (the increment that block_solve reports is the impulses themselves).
+__device__ __forceinline__ bool quad_normals(QuadBody& me, const QuadRec& r, float sign, bool block, float& ni0, float& ni1,
+                                             float& maxInc) {
+    const float vn0 = quad_closing(me, r.q.x, r.tn.y, sign);
+    float n0 = fmax_std(ni0 + r.b.z * (r.b.x - vn0), 0.0f), n1 = ni1;
+    float d0 = n0 - ni0, P1 = 0.0f, L1 = 0.0f;
+    float reported = __builtin_fabsf(d0);
+    bool valid = true, changed = false;
+    if (block) {
+        const float vn1 = quad_closing(me, r.q.y, r.tn.y, sign);
+        float t0 = 0.0f;
+        t0 += r.k.x * ni0;
+        t0 += r.k.z * ni1;
+        float t1 = 0.0f;
+        t1 += r.k.z * ni0;
+        t1 += r.k.y * ni1;
+        const float bx = (vn0 - r.b.x) - t0, by = (vn1 - r.b.y) - t1;
+        float x0 = 0.0f;
+        x0 += r.m.x * bx;
+        x0 += r.s.w * by;
+        float x1 = 0.0f;
+        x1 += r.s.w * bx;
+        x1 += r.m.y * by;
+        const float c1n0 = -x0, c1n1 = -x1;
+        const bool ok1 = c1n0 >= 0.0f && c1n1 >= 0.0f;
+        const float c2n0 = -r.b.z * bx;
+        const bool ok2 = c2n0 >= 0.0f && r.k.z * c2n0 + by >= 0.0f;
+        const float c3n1 = -r.b.w * by;
+        const bool ok3 = c3n1 >= 0.0f && r.k.z * c3n1 + bx >= 0.0f;
+        const bool ok4 = bx >= 0.0f && by >= 0.0f;
+        // With no valid case everything stays as it is.
+        valid = ok1 || ok2 || ok3 || ok4;
+        n0 = ok1 ? c1n0 : (ok2 ? c2n0 : 0.0f);
+        n1 = ok1 ? c1n1 : (ok2 ? 0.0f : (ok3 ? c3n1 : 0.0f));
+        d0 = n0 - ni0;
+        const float d1 = n1 - ni1;
+        P1 = d1 * r.tn.y;
+        L1 = quad_arm(r.q.y, P1);
+        reported = fmaxf(__builtin_fabsf(n0), __builtin_fabsf(n1));
+        changed = valid && (d0 != 0.0f || d1 != 0.0f);
+    }
+    const float P0 = d0 * r.tn.y, L0 = quad_arm(r.q.x, P0);
     QuadBody next = me;
-    next.apply(P0 + P1, quad_arm(r.q.x, P0) + quad_arm(r.q.y, P1));
-    // With no valid case (on body B's lanes) everything stays as it is.
-    const unsigned long long none = __ballot(!(ok1 || ok2 || ok3 || ok4));
-    if ((none >> (lane | 2)) & 1) return;
-    me = next;
-    ni0 = n0;
-    ni1 = n1;
-    maxInc = fmax_std(maxInc, fmax_std(__builtin_fabsf(n0), __builtin_fabsf(n1)));
+    next.apply(block ? P0 + P1 : P0, block ? L0 + L1 : L0);
+    if (valid) {
+        me = next;
+        ni0 = n0;
+        ni1 = n1;
+        maxInc = fmaxf(maxInc, reported);
+    }
+    return changed;
 }
 
 // A revolute joint's warm start or velocity update, computed whole by each of
@@ -4465,6 +4492,7 @@ __device__ __forceinline__ bool quad_joint(QuadBody& me, QuadRec& r, int quad, f
 // branch around them, and one address space for the bounds, the waits the
 // compiler places count exactly the operations in flight.  Islands marked in
 // their words are left out of a masked run.
+constexpr int kChanged = 0x10000;  // shifted by the iteration, as 1 is by one that counts as such
 enum LevelPass { kPassWarm, kPassWarmMasked, kPassIterations, kPassMasked };
 enum LevelItems { kContactItems, kJointItems, kAllItems };
 template <LevelPass kPass, LevelItems kItems>
@@ -4483,20 +4511,26 @@ __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n
     constexpr bool kMasked = kPass == kPassMasked || kPass == kPassWarmMasked;
     const int shift = __builtin_ctz(unsigned(4 * width)), groups = kWave >> shift;
     const int group = lane >> shift, j = (lane >> 2) & (width - 1), quad = lane & 3, comp = lane & 1;
-    const int turn = groups * period;
+    const int turn = 8 * groups * period;
+    const float sign = (quad & 2) ? 1.0f : -1.0f;
     constexpr int kStep = prx::kQuadVc * 16;
-    int r = -group * period, it = group;  // the group's round and iteration at the tick read ahead
+    // The group's round at the tick read ahead, as a byte offset into the bounds
+    // (past their end before its first iteration and after its last), and its
+    // iteration.
+    int r = -8 * group * period, it = group;
+    if (it >= iters) r = kOutOfRange;
     struct At {
         int2 b;
         int it, off;
     };
     auto bounds = [&](At& a) {
-        const bool on = r >= 0 && it < iters;
-        a.b = __builtin_bit_cast(int2, __builtin_amdgcn_raw_buffer_load_b64(table, on ? r * 8 : kOutOfRange, 0, 0));
+        const int off = int(min(unsigned(r), unsigned(kOutOfRange)));
+        a.b = __builtin_bit_cast(int2, __builtin_amdgcn_raw_buffer_load_b64(table, off, 0, 0));
         a.it = it;
-        if (++r == turn) {
-            r = 0;
+        r += 8;
+        if (r == turn) {
             it += groups;
+            r = it < iters ? 0 : kOutOfRange;
         }
     };
     auto f2 = [&](int off) {
@@ -4506,7 +4540,7 @@ __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n
         return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rec, off, 0, 0));
     };
     auto fetch = [&](At& a, QuadRec& q) {
-        const int off = a.off = j < a.b.y ? (a.b.x + j) * kStep : kOutOfRange;
+        const int off = a.off = j < a.b.y ? __mul24(a.b.x, kStep) + j * kStep : kOutOfRange;
         q.q = f2(off + 8 * quad);
         q.s = f4(off + 32 + 8 * (quad & 2));
         if constexpr (kItems != kJointItems) q.tn = f2(off + 64 + 8 * comp);
@@ -4518,6 +4552,10 @@ __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n
         q.k = f4(off + 112);
         q.i = f4(off + 144);
     };
+    auto mark = [](QuadRec& q, int bits, float inc) {
+        q.m.z = __int_as_float(__float_as_int(q.m.z) | bits);
+        q.m.w = fmaxf(q.m.w, inc);
+    };
     auto solve = [&](const At& at, QuadRec& q) {
         const int island = int(__float_as_uint(q.k.w) >> 8);
         bool on = at.off != kOutOfRange;
@@ -4528,17 +4566,20 @@ __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n
             const int vi = __float_as_int(q.s.z);
             QuadBody me{lds[vi + comp], lds[vi + 2], q.s.x, q.s.y};
             if (kItems != kContactItems && (n & kJointTag)) {
+                const float4 before = q.i;
                 const bool same = quad_joint<kWarm>(me, q, quad, lds[vi + (comp ^ 1)], n);
-                if (!kWarm && quad == 2 && !same)
-                    atomicOr(&words[2 * island], kMasked ? kJointMoved : 1 << at.it);
+                const bool changed = q.i.x != before.x || q.i.y != before.y || q.i.z != before.z || q.i.w != before.w;
+                if constexpr (kMasked && !kWarm) {
+                    if (quad == 2 && !same) atomicOr(&words[2 * island], kJointMoved);
+                } else if constexpr (!kWarm) {
+                    mark(q, (same ? (changed ? kChanged : 0) : 1) << at.it, 0.0f);
+                }
             } else if constexpr (kItems == kJointItems) {
             } else if constexpr (kWarm) {
                 QuadBody dl{0.0f, 0.0f, q.s.x, q.s.y};
-                if (n > 0) {
-                    const float Pn = q.i.x * q.tn.y + q.i.y * q.tn.x;
-                    dl.apply(Pn, quad_arm(q.q.x, Pn));
-                }
-                if (n > 1) {
+                const float P0 = q.i.x * q.tn.y + q.i.y * q.tn.x;
+                dl.apply(P0, quad_arm(q.q.x, P0));
+                if (n & kPoint1) {
                     const float Pn = q.i.z * q.tn.y + q.i.w * q.tn.x;
                     dl.apply(Pn, quad_arm(q.q.y, Pn));
                 }
@@ -4546,26 +4587,29 @@ __device__ __attribute__((noinline)) void velocity_level_run(float4* recs, int n
                 me.w = me.w + dl.w;
             } else {
                 float inc = 0.0f;
-                if (n > 1) quad_tangent(me, q, q.q.y, q.f.w, q.i.z, q.i.w, inc);
-                if (n > 0) quad_tangent(me, q, q.q.x, q.f.z, q.i.x, q.i.y, inc);
-                if (n == 1 || (q.k.x == 0.0f && q.k.y == 0.0f && q.k.z == 0.0f)) {
-                    if (n > 1) quad_normal(me, q, q.q.y, q.b.w, q.b.y, q.i.z, inc);
-                    if (n > 0) quad_normal(me, q, q.q.x, q.b.z, q.b.x, q.i.x, inc);
+                // A solved contact has a point 0.
+                if (n & kPoint1) quad_tangent(me, q, sign, q.q.y, q.f.w, q.i.z, q.i.w, inc);
+                quad_tangent(me, q, sign, q.q.x, q.f.z, q.i.x, q.i.y, inc);
+                if ((n & (kPoint1 | kBlockSolve)) == kPoint1)
+                    quad_normal(me, q, sign, q.q.y, q.b.w, q.b.y, q.i.z, inc);
+                const bool changed = quad_normals(me, q, sign, (n & kBlockSolve) != 0, q.i.x, q.i.z, inc);
+                if constexpr (kMasked) {
+                    if (quad == 2 && inc > 0.0f) atomicMax(&words[2 * island + 1], __float_as_int(inc));
                 } else {
-                    quad_block(me, q, lane, q.i.x, q.i.z, inc);
-                }
-                if (quad == 2 && inc > 0.0f) {
-                    atomicOr(&words[2 * island], 1 << at.it);
-                    atomicMax(&words[2 * island + 1], __float_as_int(inc));
+                    // A NaN increment is not reported, but is a change.
+                    const float all = (q.i.x + q.i.y) + (q.i.z + q.i.w);
+                    mark(q, (inc > 0.0f ? 1 : ((changed || __builtin_isnan(all)) ? kChanged : 0)) << at.it, inc);
                 }
             }
             lds[vi + comp] = me.v;
             lds[vi + 2] = me.w;
         }
         if constexpr (!kWarm) {
-            // Body B's first lane holds the impulses and stores them.
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, q.i), rec,
-                                                   (on && quad == 2 ? at.off : kOutOfRange) + 144, 0, 0);
+            // One lane stores the impulses and the marks.
+            const int off = on && quad == 2 ? at.off : kOutOfRange;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, q.i), rec, off + 144, 0, 0);
+            if constexpr (!kMasked)
+                __builtin_amdgcn_raw_buffer_store_b64(U2{__float_as_uint(q.m.z), __float_as_uint(q.m.w)}, rec, off + 136, 0, 0);
         }
         // The wave's LDS operations run in order: nothing to wait for.
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -4771,13 +4815,18 @@ struct SolveSummary {
 // Warm start and velocity sweeps of the level islands.
 //
 // Overlapped iterations run past an island's early exit.  The exit's bound is
-// zero unless set otherwise: an island exits with the first iteration in which
-// no impulse changed and no joint moved a body (its bit in the island's word
-// stays clear).  Such an
-// island is swept again from its starting velocities and impulses: the early
-// exit is what makes that short, so one below kLevelRedo contacts goes to its
-// lane, a larger one through plain iterations.  With a positive bound all
-// level islands take plain iterations, with a negative one none exits.
+// zero unless set otherwise: an island exits with the first iteration that
+// reports no increment and moves no body by a joint (its bit in the island's
+// word stays clear).  Mostly that iteration changed nothing at all, and then
+// neither do those after it: same inputs, same outputs.  Zeros keep their signs
+// too: an increment of zero is +0, so the products added to a body's zeros have
+// the signs they had, and what one sum of them made +0 stays so.  Only where
+// the iteration did change something (a block solve reports the impulses, not
+// their change; a joint's impulses may change without moving a body: kChanged)
+// is the island swept again from its starting velocities and impulses, on its
+// lane below kLevelRedo updates, else through plain iterations.  With a
+// positive bound all level islands take plain iterations, with a negative one
+// none exits.
 constexpr int kLevelRedo = 32;
 template <class Level, class Add>
 __device__ __forceinline__ void velocity_levels(const DeviceState& d, const WorldCtx& x, const Bodies<true>& bs,
@@ -4801,7 +4850,7 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
     };
     constexpr int kOut = int(0x80000000u);  // left out of masked runs
     const int iters = int(c.velIters);
-    const bool overlap = c.regMinMomentum <= 0.0f && iters <= 31;
+    const bool overlap = c.regMinMomentum <= 0.0f && iters <= 15;
     for (int is = x.lane; is < nisl; is += kWave) {
         words[2 * is] = 0;
         words[2 * is + 1] = 0;
@@ -4810,6 +4859,12 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
     if (c.warmStart) warm(std::false_type{});
     if (overlap && iters > 0) {
         sweep(std::false_type{}, iters);
+        for (int pos = x.lane; pos < P.n; pos += kWave) {
+            const float4 m = v2[std::size_t(pos) * prx::kQuadVc + 8];
+            const int is = L.island[P.order[pos]];
+            atomicOr(&words[2 * is], __float_as_int(m.z));
+            atomicMax(&words[2 * is + 1], __float_as_int(m.w));
+        }
         __syncthreads();
     }
     // Islands to sweep again, on their lane or by plain iterations.
@@ -4818,14 +4873,17 @@ __device__ __forceinline__ void velocity_levels(const DeviceState& d, const Worl
         const int is = base + x.lane;
         bool lane = false, plain = false;
         if (is < nisl && level(is)) {
-            const int ran = (1 << (iters & 31)) - 1;
-            const bool exits = overlap && c.regMinMomentum == 0.0f && iters > 1 && ((words[2 * is] | (1 << (iters - 1))) & ran) != ran;
+            const int word = words[2 * is];
+            const int still = ~word & ((1 << (iters & 15)) - 1);  // iterations without an increment
+            const int exit = __builtin_ctz(unsigned(still) | 0x10000u);
+            const bool early = overlap && c.regMinMomentum == 0.0f && exit + 1 < iters;
+            const bool exits = early && (word & (kChanged << exit)) != 0;
             plain = !overlap;
             if (exits) {
                 lane = S.istart[is + 1].y - S.istart[is].y + S.jstart[is + 1] - S.jstart[is] < kLevelRedo;
                 plain = !lane;
             } else if (overlap) {
-                add(VelResult{__int_as_float(words[2 * is + 1]), iters});
+                add(VelResult{__int_as_float(words[2 * is + 1]), early ? exit + 1 : iters});
             }
             words[2 * is] = lane ? 1 : (plain ? 0 : kOut);
             if (exits)
