@@ -126,14 +126,15 @@ PRX_HD double MulAdd(double a, double b, double c) {
 // Selecting by a flag instead of a table pointer keeps every coefficient a
 // compile-time constant: no per-lane table load inside the solver chains.
 template <bool Fma>
-PRX_HD float Poly(double x, double x2, const SinCosTab& p, int n, bool negCos) {
-    if ((n & 1) == 0) {
-        const double x3 = x * x2;
-        const double s1 = MulAdd<Fma>(x2, p.s3, p.s2);
-        const double x7 = x3 * x2;
-        const double s = MulAdd<Fma>(x3, p.s1, x);
-        return float(MulAdd<Fma>(x7, s1, s));
-    }
+PRX_HD float PolySin(double x, double x2, const SinCosTab& p) {
+    const double x3 = x * x2;
+    const double s1 = MulAdd<Fma>(x2, p.s3, p.s2);
+    const double x7 = x3 * x2;
+    const double s = MulAdd<Fma>(x3, p.s1, x);
+    return float(MulAdd<Fma>(x7, s1, s));
+}
+template <bool Fma>
+PRX_HD float PolyCos(double x2, const SinCosTab& p, bool negCos) {
     const double x4 = x2 * x2;
     const double c2 = MulAdd<Fma>(x2, p.c4, p.c3);
     const double c1 = MulAdd<Fma>(x2, p.c1, p.c0);
@@ -141,6 +142,10 @@ PRX_HD float Poly(double x, double x2, const SinCosTab& p, int n, bool negCos) {
     const double c = MulAdd<Fma>(x4, p.c2, c1);
     const float r = float(MulAdd<Fma>(x6, c2, c));
     return negCos ? -r : r;
+}
+template <bool Fma>
+PRX_HD float Poly(double x, double x2, const SinCosTab& p, int n, bool negCos) {
+    return (n & 1) == 0 ? PolySin<Fma>(x, x2, p) : PolyCos<Fma>(x2, p, negCos);
 }
 
 // The published sign table {1, -1, -1, 1}[i & 3].
@@ -223,7 +228,9 @@ PRX_HD float CosF(float y) {
 // (fma(-0, pi/2, x) = x), so the small-argument polynomials are the fast
 // path's and one path serves every |y| < 120 (the tiny-argument results are
 // selected at the end): lanes of a wave with angles on either side of pi/4
-// run the same instructions.
+// run the same instructions.  Each polynomial is evaluated once and the quadrant
+// picks which is which afterwards: picking first, lanes in odd and even
+// quadrants took both branches twice.
 template <bool Fma>
 PRX_HD void SinCosF(float y, float* sinOut, float* cosOut) {
     double x = y;
@@ -245,10 +252,10 @@ PRX_HD void SinCosF(float y, float* sinOut, float* cosOut) {
     }
     const double xs = x * s, x2 = x * x;
     const bool tiny = t < AbsTop12(0x1p-12f);
-    const float sv = Poly<Fma>(xs, x2, p, n, neg);
-    const float cv = Poly<Fma>(xs, x2, p, n ^ 1, neg);
-    *sinOut = tiny ? y : sv;
-    *cosOut = tiny ? 1.0f : cv;
+    const float sp = PolySin<Fma>(xs, x2, p), cp = PolyCos<Fma>(x2, p, neg);
+    const bool odd = (n & 1) != 0;
+    *sinOut = tiny ? y : (odd ? cp : sp);
+    *cosOut = tiny ? 1.0f : (odd ? sp : cp);
 }
 
 }  // namespace prx_math

@@ -4108,7 +4108,8 @@ __device__ __forceinline__ void store_quad_vc(float4* o, const Vc& vc, const Bod
 //           inverse rotational inertia (negative for A)
 //   [2] [3] X: local centre, local point, local point, local normal
 //   [4] [5] Y: local centre, manifold points 0 and 1
-//   [6]     total radius, total inverse mass, type | points << 8 | island << 16
+//   [6]     total radius, total inverse mass, type | points << 8 | island << 16,
+//           separation
 __device__ __forceinline__ void store_quad_pc(float4* o, const Pc& pc, int island) {
     const bool faceB = pc.m.type == kFaceB;
     const BodyC& X = faceB ? pc.B : pc.A;
@@ -4135,7 +4136,7 @@ __device__ __forceinline__ void store_quad_pc(float4* o, const Pc& pc, int islan
 //   [0] [1] as a contact's
 //   [2] [3] A: local anchor, reference angle, lower limit; upper limit, motor mass
 //   [4] [5] B: the same with its own anchor
-//   [6]     -, -, kJointTag | flags << 8 | limit << 11 | island << 16
+//   [6]     -, -, kJointTag | flags << 8 | limit << 11 | island << 16, infinity
 constexpr std::uint32_t kJointTag = 0x80u;
 __device__ __forceinline__ void store_quad_joint(float4* v, float4* o, const float4* u, int nb, int island) {
     const float4 r = u[0], m = u[1], n = u[2], ms = u[4], mo = u[5], la = u[6], ang = u[7];
@@ -4155,7 +4156,8 @@ __device__ __forceinline__ void store_quad_joint(float4* v, float4* o, const flo
     o[2] = float4{la.x, la.y, ang.x, ang.y};
     o[4] = float4{la.z, la.w, ang.x, ang.y};
     o[3] = o[5] = float4{ang.z, n.z, 0.0f, 0.0f};
-    o[6] = float4{0.0f, 0.0f, __uint_as_float(kJointTag | (flags << 8) | (limit << 11) | (std::uint32_t(island) << 16)), 0.0f};
+    o[6] = float4{0.0f, 0.0f, __uint_as_float(kJointTag | (flags << 8) | (limit << 11) | (std::uint32_t(island) << 16)),
+                  __builtin_inff()};
 }
 
 // Builds the plan of the slots whose island (LevelScratch::island) is not
@@ -5000,19 +5002,23 @@ __device__ __attribute__((noinline)) void position_level_run(float4* recs, int n
     auto solve = [&](int off, const QuadPos& q) {
         const int island = int(__float_as_uint(q.k.z) >> 16);
         const bool joint = (__float_as_uint(q.k.z) & kJointTag) != 0;
-        if (off != kOutOfRange && joint == kJoints && (words[2 * island + 1] & ~kJointOpen) == 0) {
+        const bool on = off != kOutOfRange && joint == kJoints && (words[2 * island + 1] & ~kJointOpen) == 0;
+        float sep = 0.0f;
+        if (on) {
             const int at = __float_as_int(q.b.x);
             float p = lds[at + comp], a = lds[at + 2];
             if constexpr (kJoints) {
                 const bool solved = quad_joint_position(q, quad, p, lds[at + (comp ^ 1)], a, c);
                 if (quad == 0 && !solved) atomicOr(&words[2 * island + 1], kJointOpen);
             } else {
-                const float sep = quad_position(q, quad, p, a, c);
-                if (quad == 0 && sep < __builtin_inff()) atomicMin(&words[2 * island], float_key(sep));
+                sep = quad_position(q, quad, p, a, c);
             }
             lds[at + comp] = p;
             lds[at + 2] = a;
         }
+        // One lane stores the separation: cheaper than a minimum in LDS.
+        if constexpr (!kJoints)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sep), rec, (on && quad == 0 ? off : kOutOfRange) + 108, 0, 0);
         // The wave's LDS operations run in order: nothing to wait for.
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     };
@@ -5034,6 +5040,8 @@ __device__ __attribute__((noinline)) void position_level_run(float4* recs, int n
         atB = atA;
         atA = atC;
     }
+    // The run's stores complete before other lanes read the records back.
+    __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
 // Position sweeps of the level islands, iteration after iteration; an island
@@ -5061,6 +5069,12 @@ __device__ __forceinline__ void position_levels(const DeviceState& d, const Worl
         const PositionConf pc{c.regResolutionRate, c.linearSlop, c.maxLinearCorrection, c.angularSlop, c.maxAngularCorrection};
         position_level_run<false>(recs, P.n, P.rb, P.rounds, smem, 8 * x.nb, pc);
         if (joints) position_level_run<true>(recs, P.n, P.rb, P.rounds, smem, 8 * x.nb, pc);
+        // The iteration's smallest separation of each island still swept.
+        for (int pos = x.lane; pos < P.n; pos += kWave) {
+            const float4 k = recs[std::size_t(pos) * prx::kQuadPc + 6];
+            const int is = int(__float_as_uint(k.z) >> 16);
+            if (k.w < __builtin_inff() && (words[2 * is + 1] & ~kJointOpen) == 0) atomicMin(&words[2 * is], float_key(k.w));
+        }
         __syncthreads();
         bool going = false;
         for (int base = 0; base < nisl; base += kWave) {
