@@ -874,7 +874,10 @@ __device__ __forceinline__ void toi_phase(const DeviceState& d, const WorldCtx& 
     }
     for (int b = x.lane; b < x.nb; b += kWave) d.t_isl_b[x.bo + b] = 0;
     __syncthreads();
-    build_adjacency<true>(d, x, k.nc, S);
+    // The bodies' contact lists serve the events: built before the first one, so
+    // that a step without events goes without (a settled world of 400 bodies,
+    // with the listing of the candidates below: a step 2.00 -> 1.62 ms).
+    bool adjacent = false;
     for (int pass = 0;; ++pass) {
         // Per-lane maxima and counts of the times of impact this pass computes.
         std::uint32_t lMaxDist = 0, lMaxToi = 0, lMaxRoot = 0, lUpdated = 0, lAtMax = 0;
@@ -885,31 +888,27 @@ __device__ __forceinline__ void toi_phase(const DeviceState& d, const WorldCtx& 
             ++lUpdated;
         };
         // UpdateContactTOIs.
-        if (pass == 0) {
-            for (int i = x.lane; i < k.nc; i += kWave) {
-                const int need = needs_toi(d, x, i, c);
-                if (need == 1) addToi(contact_toi(d, x, i, c));
-                else if (need == 2) ++lAtMax;
-            }
-        } else {
-            // The filters do not change during the pass (they read the
-            // contact's own TOI state, its flags and the bodies' awake
-            // flags), so the wave lists the candidates in order and lane 0
-            // computes them one after another.
-            int ncand = 0;
-            for (int base = 0; base < k.nc; base += kWave) {
-                const int i = base + x.lane;
-                const int nd = (i < k.nc) ? needs_toi(d, x, i, c) : 0;
-                const bool need = nd == 1;
-                if (nd == 2) ++lAtMax;
-                const unsigned long long m = __ballot(need);
-                if (need) S.icont[ncand + __popcll(m & lanes_below(x.lane))] = i;
-                ncand += __popcll(m);
-            }
-            __syncthreads();
-            if (x.lane == 0)
-                for (int q = 0; q < ncand; ++q) addToi(contact_toi(d, x, S.icont[q], c));
+        // The filters do not change during the pass (they read the contact's
+        // own TOI state, its flags and the bodies' awake flags), so the wave
+        // lists the candidates in order.  In the first pass no body has been
+        // advanced and the times are independent: side by side (33 of a settled
+        // pile's 1100 contacts are candidates; taken 64 contacts at a time, two
+        // lanes of each chunk worked).  Later lane 0 computes them one after
+        // another.
+        int ncand = 0;
+        for (int base = 0; base < k.nc; base += kWave) {
+            const int i = base + x.lane;
+            const int nd = (i < k.nc) ? needs_toi(d, x, i, c) : 0;
+            const bool need = nd == 1;
+            if (nd == 2) ++lAtMax;
+            const unsigned long long m = __ballot(need);
+            if (need) S.icont[ncand + __popcll(m & lanes_below(x.lane))] = i;
+            ncand += __popcll(m);
         }
+        __syncthreads();
+        const int step = pass == 0 ? kWave : 1;
+        for (int q = pass == 0 ? x.lane : (x.lane == 0 ? 0 : ncand); q < ncand; q += step)
+            addToi(contact_toi(d, x, S.icont[q], c));
         {
             const std::uint32_t upd = wave_sum(lUpdated), atm = wave_sum(lAtMax);
             const std::uint32_t md = wave_max(lMaxDist), mt = wave_max(lMaxToi), mr = wave_max(lMaxRoot);
@@ -945,6 +944,8 @@ __device__ __forceinline__ void toi_phase(const DeviceState& d, const WorldCtx& 
             if (bi != 0x7fffffff) k.status |= prx::kStatusToiLimit;
             break;
         }
+        if (!adjacent) build_adjacency<true>(d, x, k.nc, S);
+        adjacent = true;
         if (x.lane == 0) {
             ++st[prx::kStToiContactsFound];
             if (!d.t_isl_c[x.co + bi]) {
@@ -997,7 +998,7 @@ __device__ __forceinline__ void toi_phase(const DeviceState& d, const WorldCtx& 
                 d.t_isl_c[x.co + i] = 0;
             }
             __syncthreads();
-            build_adjacency<true>(d, x, k.nc, S);
+            adjacent = false;
         }
     }
     // ResetBodiesForSolveTOI / ResetContactsForSolveTOI.
