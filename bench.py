@@ -248,7 +248,7 @@ def large_world(args, pa, conf):
     out = {
         "workload": "one drop world: %d bodies (half disks r U[0.25,0.75], half 3..8-gons R U[0.3,0.8], "
                     "friction U[0.2,0.8]) into a 400 x 400 static box of 4 edges, seed %d, dt=1/60 8/3 "
-                    "iterations doToi=true (TOI against static shapes), LBVH broadphase, graph-coloured "
+                    "iterations doToi=true (TOI against static shapes), graph-coloured "
                     "Gauss-Seidel" % (args.big_bodies, args.seed),
         "steps": args.big_steps,
         "value": dyn * args.big_steps / wall,

@@ -261,7 +261,10 @@ typedef struct prx_batch_conf {
     uint32_t use_graph;         /* replay steps from a captured hipGraph */
     uint32_t order;             /* 0: largest worlds first, 1: as given */
     uint32_t coop_min_contacts; /* islands with at least this many constraints are
-                                   swept by the whole wavefront (default 32) */
+                                   swept by the whole wavefront (default 32), and
+                                   those of four or more together with others in
+                                   rounds; the greatest values keep every island
+                                   on one lane.  Same results either way */
     uint32_t lds_bytes;         /* dynamic LDS per workgroup; 0: the minimum the
                                    batch needs.  Larger values leave fewer
                                    workgroups per CU (160 KB of LDS per CU), so
