@@ -4481,19 +4481,22 @@ __device__ __forceinline__ bool quad_joint(QuadBody& me, QuadRec& r, int quad, f
 
 // Iterations [0, iters) of the plan's velocity sweep, overlapped as its period
 // allows (one iteration: a plain pass).  Lane 4 (width g + j) + 2 s + c serves
-// update j of group g's round (a group is 4 `width` lanes); group g runs iterations
-// g, g + groups, ...  Bound by
-// the instructions of one round after another, about 2000 cycles each (no other
-// wave of the world can help): a pile of 400 bodies takes 2.2M cycles for the
-// velocity sweeps and 1.2M for the position sweeps, from 3.1M and 1.8M with
-// two lanes an update, one iteration after another.  A round's records are
-// read while the round before is solved, and its bounds one round earlier
-// still.  The records are read and the impulses written by buffer
-// instructions that every lane issues in every round, lanes without an update
-// at an offset past the buffer's end (no memory is touched for them): with no
-// branch around them, and one address space for the bounds, the waits the
-// compiler places count exactly the operations in flight.  Islands marked in
-// their words are left out of a masked run.
+// update j of group g's round (a group is 4 `width` lanes); group g runs
+// iterations g, g + groups, ...  Bound by the instructions of one round after
+// another, no other wave of the world can help: 1000 cycles for single points,
+// 1400 for two-point contacts or a mix, 360 of them without the updates.  LDS
+// atomics for the marks cost 200, a path of its own for either kind another
+// 200 in a mixed round.  A pile of 400 bodies: 3.1M -> 2.0M cycles for the
+// velocity and 1.8M -> 1.1M for the position sweeps against two lanes an
+// update, one iteration after another.
+//
+// A round's records are read while the round before is solved, and its bounds
+// one round earlier still.  The records are read and the impulses written by
+// buffer instructions that every lane issues in every round, lanes without an
+// update at an offset past the buffer's end (no memory is touched for them):
+// with no branch around them, and one address space for the bounds, the waits
+// the compiler places count exactly the operations in flight.  Islands marked
+// in their words are left out of a masked run.
 constexpr int kChanged = 0x10000;  // shifted by the iteration, as 1 is by one that counts as such
 enum LevelPass { kPassWarm, kPassWarmMasked, kPassIterations, kPassMasked };
 enum LevelItems { kContactItems, kJointItems, kAllItems };
