@@ -603,7 +603,10 @@ int prx_lbvh_pairs_noalloc(const float* aabbs, const int32_t* bodies, const uint
  * dynamic bodies of |final position - target|^2.  The forward pass keeps a
  * checkpoint every `every` steps; the backward pass recomputes each segment
  * from its checkpoint, recording the solves, and reverses them.  Sleeping
- * is not differentiated (a body put to sleep has its velocity zeroed). */
+ * is not differentiated (a body put to sleep has its velocity zeroed).
+ * Bodies that are not dynamic have zero gradients, but for the velocity of a
+ * kinematic disk reversed by the first kernel: it collects the terms of the
+ * contacts it is body B of (those with bodies created before it). */
 typedef struct prx_adjoint prx_adjoint;
 int prx_adjoint_create(prx_batch* batch, int nsteps, int every, const prx_step_conf* conf, prx_adjoint** out);
 void prx_adjoint_destroy(prx_adjoint* adj);

@@ -179,11 +179,17 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
     int* const iters = kLds ? start + cap + 1 : plan + 2 * cap + 1;
     int* const lvl = plan + 4 * cap;
     auto vcrec = [&](int e) { return t.vc + (std::size_t(co) + std::size_t(e)) * prx::kTapeVc; };
-    if constexpr (kLds) {
-        for (int b = lane; b < nb; b += kWave) {
-            X[b] = a.xbar[bo + b];
-            V[b] = a.vbar[bo + b];
-        }
+    // A kinematic disk has no mass but moves at its own velocity, which the
+    // contacts it is body B of read: it collects their terms (its mark is the
+    // fourth component of its adjoints) and orders the updates that add to them.
+    auto kinematic = [&](int b) {
+        return (d.bflags[bo + b] & (prx::kSpeedable | prx::kAccelerable)) == prx::kSpeedable;
+    };
+    for (int b = lane; b < nb; b += kWave) {
+        const float4 xb = a.xbar[bo + b], vb = a.vbar[bo + b];
+        const float mark = kinematic(b) ? 1.0f : 0.0f;
+        X[b] = float4{xb.x, xb.y, xb.z, mark};
+        V[b] = float4{vb.x, vb.y, vb.z, mark};
     }
     // Impulse adjoints carried in from the next step, by contact id: the
     // step's final impulses warm-started the next step where the manifold
@@ -209,8 +215,9 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
     const RoundPlan rp = plan_rounds(n, nb, kWave, lane, [&](int e) {
         const float4* vc = vcrec(e);
         const float4 ms = vc[8];
+        const int bB = __float_as_int(vc[5].z);
         return int2{(ms.x != 0.0f || ms.y != 0.0f) ? __float_as_int(vc[2].w) : -1,
-                    (ms.z != 0.0f || ms.w != 0.0f) ? __float_as_int(vc[5].z) : -1};
+                    (ms.z != 0.0f || ms.w != 0.0f || kinematic(bB)) ? bB : -1};
     }, last, lvl, order, start);
     const int rounds = rp.rounds;
     __syncthreads();
@@ -262,7 +269,9 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
                 if (npts != 1u || (type != 1u && type != 2u)) unmodelled = 1;
                 else ++posUpdates;
                 if (npts == 1u && (type == 1u || type == 2u) && K > 0.0f) {
-                    const V2 xbA = dynA ? v2(X[bA]) : V2{0.0f, 0.0f}, xbB = v2(X[bB]);
+                    const float4 xb4 = X[bB];
+                    const bool movB = ms.z != 0.0f || ms.w != 0.0f || xb4.w != 0.0f;
+                    const V2 xbA = dynA ? v2(X[bA]) : V2{0.0f, 0.0f}, xbB = v2(xb4);
                     const float s = cur.g0.w;  // separation the forward update used
                     const float inner = c.regResolutionRate * (s + c.linearSlop);
                     const float Cc = -clamp_std(inner, -c.maxLinearCorrection, 0.0f);
@@ -279,7 +288,7 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
                             const float nn = dot(nn2, nbar);
                             const V2 dbar = mul(nbar - mul(nn2, nn), 1.0f / L) + mul(nn2, sbar);
                             if (dynA) add_body(X + bA, -dbar, 0.0f);
-                            if (ms.z != 0.0f || ms.w != 0.0f) add_body(X + bB, dbar, 0.0f);
+                            if (movB) add_body(X + bB, dbar, 0.0f);
                         }
                     } else {
                         // Face A: A is the polygon (static: its plane and normal
@@ -287,7 +296,7 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
                         const V2 nrm = v2(cur.v0);
                         const float Cbar = dot(gP, nrm) / K;
                         const float sbar = active ? -c.regResolutionRate * Cbar : 0.0f;
-                        if (ms.z != 0.0f || ms.w != 0.0f) add_body(X + bB, mul(nrm, sbar), 0.0f);
+                        if (movB) add_body(X + bB, mul(nrm, sbar), 0.0f);
                     }
                 }
             }
@@ -340,7 +349,7 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
                 const float nm = cur.v4.z, tm = cur.v4.w, bias = cur.v5.x;
                 const float mA = cur.v8.x, iA = cur.v8.y, mB = cur.v8.z, iB = cur.v8.w;
                 const int bA = __float_as_int(cur.v2.w), bB = __float_as_int(cur.v5.z);
-                const bool movA = mA != 0.0f || iA != 0.0f, movB = mB != 0.0f || iB != 0.0f;
+                const bool movA = mA != 0.0f || iA != 0.0f;
                 const V2 vA{cur.g0.x, cur.g0.y}, vB{cur.g1.x, cur.g1.y};
                 const float wA = cur.g0.z, wB = cur.g1.z, ltOld = cur.g0.w, lnOld = cur.g1.w;
                 // Forward recomputation of this update.
@@ -362,7 +371,8 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
                 // Adjoints of the outputs (a body that does not move has none
                 // that reaches another).
                 const float4 zero{0.0f, 0.0f, 0.0f, 0.0f};
-                const float4 va4 = movA ? V[bA] : zero, vb4 = movB ? V[bB] : zero;
+                const float4 va4 = movA ? V[bA] : zero, vb4 = V[bB];
+                const bool movB = mB != 0.0f || iB != 0.0f || vb4.w != 0.0f;
                 V2 vbA = v2(va4), vbB = v2(vb4);
                 float wbA = va4.z, wbB = vb4.z;
                 float2 lb = lb0;
@@ -492,7 +502,7 @@ __global__ __launch_bounds__(64) void k_adjoint_step(DeviceState d, Tape t, AdjS
             const float4 ms = vc[8];
             const float mA = ms.x, iA = ms.y, mB = ms.z, iB = ms.w;
             const int bA = __float_as_int(vc[2].w), bB = __float_as_int(vc[5].z);
-            const bool movA = mA != 0.0f || iA != 0.0f, movB = mB != 0.0f || iB != 0.0f;
+            const bool movA = mA != 0.0f || iA != 0.0f, movB = mB != 0.0f || iB != 0.0f || V[bB].w != 0.0f;
             const float4 c0 = a.cbar[slot * 3 + 0], c1 = a.cbar[slot * 3 + 1], c2 = a.cbar[slot * 3 + 2];
             V2 nbar{c0.x, c0.y}, rAbar{c0.z, c0.w}, rBbar{c1.x, c1.y}, tbar{c1.z, c1.w};
             const float nmbar = c2.x, tmbar = c2.y, biasbar = c2.z, fbarC = c2.w;
