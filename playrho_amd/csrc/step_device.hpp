@@ -3163,14 +3163,17 @@ __device__ __forceinline__ int find_islands(const DeviceState& d, const WorldCtx
 // LDS words: off (nb + 1), the stack (nb; reached static bodies from its top,
 // :1386-1398), the entries contact << 16 | other body; then the bytes of the
 // bodies (0 to reach, 1 reached, 2 static, 3 static and counted for the
-// island; 8: not enabled, 16: may start an island), contacts and joints; then
-// the bodies' joint ranges and list.  The wave's LDS operations run in order,
-// so a compiler fence is enough.  Returns islands, most bodies of one.
+// island; 8: not enabled, 16: may start an island), contacts and joints; then,
+// where they fit too (kJointsLds), the bodies' joint ranges and list, which are
+// read from global memory otherwise (joint_range, joint_list).  The wave's LDS
+// operations run in order, so a compiler fence is enough.  Returns islands, most
+// bodies of one.
 using LdsByte = __attribute__((address_space(3))) std::uint8_t;
-template <bool kJoints>
+enum IslandJoints { kNoJoints, kJointsLds, kJointsGlobal };
+template <IslandJoints kJoints>
 __device__ __attribute__((noinline)) int2 search_islands(LdsWord* smem, int nb, int nc, int nj, int nent, int* ibody,
                                                          int* bisland, int* icont, int2* istart, int* jstart, int* ijoint,
-                                                         int nisl) {
+                                                         const int2* joint_range, const int2* joint_list, int nisl) {
     nb = __builtin_amdgcn_readfirstlane(nb);
     nisl = __builtin_amdgcn_readfirstlane(nisl);
     ibody = uniform_ptr(ibody);
@@ -3179,6 +3182,8 @@ __device__ __attribute__((noinline)) int2 search_islands(LdsWord* smem, int nb, 
     istart = uniform_ptr(istart);
     jstart = uniform_ptr(jstart);
     ijoint = uniform_ptr(ijoint);
+    joint_range = uniform_ptr(joint_range);
+    joint_list = uniform_ptr(joint_list);
     const int lane = int(threadIdx.x);
     LdsWord* const off = smem;
     LdsWord* const stack = off + nb + 1;
@@ -3201,7 +3206,7 @@ __device__ __attribute__((noinline)) int2 search_islands(LdsWord* smem, int nb, 
         for (unsigned long long left = seeds(); left; left = seeds()) {
             int bb = base + __builtin_ctzll(left);
             istart[nisl] = int2{nbe, nce};
-            if constexpr (kJoints) jstart[nisl] = nje;
+            if constexpr (kJoints != kNoJoints) jstart[nisl] = nje;
             else jstart[nisl] = 0;
             islb[bb] |= 1;
             order();
@@ -3252,13 +3257,15 @@ __device__ __attribute__((noinline)) int2 search_islands(LdsWord* smem, int nb, 
                     nce += __popcll(m);
                     reach(fresh, ob, mark, r0, r1);
                 }
-                if constexpr (kJoints) {
+                if constexpr (kJoints != kNoJoints) {
                     // AddJointsToIsland (AabbTreeWorld.cpp:1446-1470).
-                    const int j0 = __builtin_amdgcn_readfirstlane(jrange[2 * bb]), j1 = j0 + __builtin_amdgcn_readfirstlane(jrange[2 * bb + 1]);
+                    const int2 range = kJoints == kJointsLds ? int2{jrange[2 * bb], jrange[2 * bb + 1]} : joint_range[bb];
+                    const int j0 = __builtin_amdgcn_readfirstlane(range.x), j1 = j0 + __builtin_amdgcn_readfirstlane(range.y);
                     for (int j = j0; j < j1; j += kWave) {
                         const bool has = j + lane < j1;
                         const int at = has ? j + lane : j;
-                        const int ji = jlist[2 * at], other = jlist[2 * at + 1];
+                        const int2 entry = kJoints == kJointsLds ? int2{jlist[2 * at], jlist[2 * at + 1]} : joint_list[at];
+                        const int ji = entry.x, other = entry.y;
                         // A target joint has no other body (-1).
                         const int ob = other >= 0 ? other : 0;
                         const int taken = islj[ji], mark = other >= 0 ? int(islb[ob]) : 1, r0 = off[ob], r1 = off[ob + 1];
@@ -3340,7 +3347,12 @@ __device__ __forceinline__ int find_islands_lds(const DeviceState& d, const Worl
     std::uint8_t* islc = islb + nb;
     std::uint8_t* islj = islc + nc;
     const int marks = 4 * (2 * nb + 1 + nent) + nb + nc + x.nj;
-    if (marks + (x.nj > 0 ? 7 + 8 * (nb + 2 * x.nj) : 0) > ldsAvail) return -1;
+    if (marks > ldsAvail) return -1;
+    // Dense joint worlds (a cloth: two joints a body) have no room for the lists
+    // from about 260 bodies.  400 bodies with 685 joints, adjacency and search:
+    // 532k cycles with the lists in LDS, 640k with them read from memory, 1395k
+    // by the one-lane search that takes the worlds refused here.
+    const bool lists = x.nj > 0 && marks + 7 + 8 * (nb + 2 * x.nj) <= ldsAvail;
     for (int b = x.lane; b < nb; b += kWave) stack[b] = off[b];
     __syncthreads();
     for (int i = x.lane; i < nc; i += kWave) {
@@ -3372,7 +3384,7 @@ __device__ __forceinline__ int find_islands_lds(const DeviceState& d, const Worl
     for (int i = x.lane; i < x.nj; i += kWave) islj[i] = 0;
     // The bodies' joints behind the marks.
     int2* const jrange = reinterpret_cast<int2*>(g_smem) + (marks + 7) / 8;
-    if (x.nj > 0) {
+    if (lists) {
         for (int b = x.lane; b < nb; b += kWave) jrange[b] = d.bjoint[x.bo + b];
         for (int i = x.lane; i < 2 * x.nj; i += kWave) jrange[nb + i] = d.bjoint_list[2 * x.jo + i];
     }
@@ -3399,11 +3411,15 @@ __device__ __forceinline__ int find_islands_lds(const DeviceState& d, const Worl
         nsingle += __popcll(m);
     }
     __syncthreads();
-    const int2 found = x.nj > 0
-        ? search_islands<true>((LdsWord*)reinterpret_cast<int*>(g_smem), nb, nc, x.nj, nent, S.ibody, S.bisland, S.icont,
-                               S.istart, S.jstart, S.ijoint, nsingle)
-        : search_islands<false>((LdsWord*)reinterpret_cast<int*>(g_smem), nb, nc, 0, nent, S.ibody, S.bisland, S.icont,
-                                S.istart, S.jstart, S.ijoint, nsingle);
+    auto search = [&](auto joints) {
+        return search_islands<decltype(joints)::value>((LdsWord*)reinterpret_cast<int*>(g_smem), nb, nc, x.nj, nent, S.ibody,
+                                                       S.bisland, S.icont, S.istart, S.jstart, S.ijoint, d.bjoint + x.bo,
+                                                       d.bjoint_list + 2 * x.jo, nsingle);
+    };
+    int2 found;
+    if (x.nj == 0) found = search(std::integral_constant<IslandJoints, kNoJoints>{});
+    else if (lists) found = search(std::integral_constant<IslandJoints, kJointsLds>{});
+    else found = search(std::integral_constant<IslandJoints, kJointsGlobal>{});
     __syncthreads();
     maxBodies = __builtin_amdgcn_readfirstlane(found.y);
     return __builtin_amdgcn_readfirstlane(found.x);
