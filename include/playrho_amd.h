@@ -525,10 +525,10 @@ int prx_batch_download(prx_batch* batch);
 /* Measures the last prx_batch_step call's kernel time (ms, HIP events on the
  * launch stream) and the number of step launches it covered. */
 int prx_batch_last_timing(prx_batch* batch, float* ms, int* launches);
-/* Sum over worlds of dynamic bodies, and of contacts (after download). */
+/* Sum over worlds of dynamic bodies. */
 uint64_t prx_batch_dynamic_bodies(const prx_batch* batch);
-/* Totals over the batch's worlds from the last download: out[0] awake
- * dynamic bodies, out[1] proxies, out[2] sum over proxies of (8 + 16 x vertex
+/* Totals over the batch's worlds (downloaded first where the device holds a
+ * newer state): out[0] awake dynamic bodies, out[1] proxies, out[2] sum over proxies of (8 + 16 x vertex
  * count) bytes, out[3] contacts, out[4] touching contacts. */
 int prx_batch_counts(prx_batch* batch, uint64_t out[5]);
 /* Per-world phase timings: enable != 0 turns collection on (subsequent steps

@@ -780,7 +780,7 @@ class Batch:
         return {k: getattr(best, k) for k, _ in BatchConf._fields_}
 
     def counts(self):
-        """(awake dynamic bodies, proxies, shape bytes, contacts, touching) after download()."""
+        """(awake dynamic bodies, proxies, shape bytes, contacts, touching)."""
         out = np.zeros(5, dtype=np.uint64)
         _check(lib().prx_batch_counts(self.h, out.ctypes.data))
         return tuple(int(x) for x in out)

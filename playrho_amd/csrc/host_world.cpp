@@ -3119,6 +3119,10 @@ std::uint64_t prx_batch_dynamic_bodies(const prx_batch* b) {
 int prx_batch_counts(prx_batch* b, std::uint64_t out[5]) {
     if (!b || !out) return Fail(PRX_E_INVALID_ARGUMENT, "null argument");
     for (int i = 0; i < 5; ++i) out[i] = 0;
+    // The counts are of the host mirrors, which reading bodies leaves as they are.
+    for (prx_world* w : b->worlds)
+        if (w && w->owner == b)
+            if (int st = Refresh(w)) return st;
     for (const prx_world* w : b->worlds) {
         if (!w) continue;
         for (const auto& hb : w->bodies)
