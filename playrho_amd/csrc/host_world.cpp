@@ -1714,10 +1714,22 @@ int StepBatch(prx_batch* b, const prx_step_conf* conf, int nsteps) {
     }
     PRX_HIP(hipEventRecord(b->ev1, b->stream));
     b->last_launches = nsteps;
+    if (nsteps == 0) return PRX_OK;
     for (prx_world* w : b->worlds)
         if (w) w->host_stale = true;
     b->view_valid = false;
     return PRX_OK;
+}
+
+// The listener calls of edits go with the first step after them.  Before a
+// later step they are dropped, as that step's own record is: a download, which
+// joins them to the record, need not have come between.
+void DropCallsOfPastEdits(prx_batch* b) {
+    for (prx_world* w : b->worlds) {
+        if (!w || !w->host_stale) continue;
+        w->pre_events.clear();
+        w->pre_nevents = 0;
+    }
 }
 
 int SetSweepPosition(prx_world* w, std::uint32_t body, float px, float py, float angle);
@@ -2506,6 +2518,7 @@ int prx_step(prx_world* w, const prx_step_conf* conf, prx_step_stats* stats) {
         if (int st = CreateBatch(one, 1, &bc, &b)) return st;
         w->solo = b;
     }
+    DropCallsOfPastEdits(w->solo);
     if (int st = StepRecorded(w->solo, conf)) return st;
     if (int st = DeliverEvents(w->solo)) return st;
     if (stats) {
@@ -3077,6 +3090,7 @@ void prx_batch_destroy(prx_batch* b) {
 
 int prx_batch_step(prx_batch* b, const prx_step_conf* conf, int nsteps) {
     if (!b) return Fail(PRX_E_INVALID_ARGUMENT, "null batch");
+    DropCallsOfPastEdits(b);
     if (!HasListener(b)) return StepBatch(b, conf, nsteps);
     // Worlds with listeners: one step at a time, each step's calls delivered
     // before the next step.
