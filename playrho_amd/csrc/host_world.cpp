@@ -1249,13 +1249,11 @@ int BuildBatch(prx_batch* b) {
         E += std::size_t(h.ev_cap);
         if (E > std::size_t(0x7fffffff)) return Fail(PRX_E_LENGTH, "contact listener records exceed 2^31 words");
     }
-    int maxNb = 0;
-    for (const prx_world* w : b->worlds) maxNb = std::max<int>(maxNb, int(w->bodies.size()));
-    // Body constraint state (32 B per body), two words per island (at most one
-    // island per body) and the record stage; worlds whose bodies do not fit
-    // keep them in global scratch.
-    const int stageBytes = prx::kStageFloat4 * 16;
-    b->lds_min = std::min<int>(64 * 1024, std::max<int>(1024 + stageBytes, ((maxNb * 40 + stageBytes + 255) / 256) * 256));
+    // The most that any of the worlds makes use of; worlds whose bodies do not
+    // fit keep them in global scratch.
+    int lds = 1024 + prx::kStageFloat4 * 16;
+    for (const prx_world* w : b->worlds) lds = std::max(lds, prx::StepLdsBytes(int(w->bodies.size())));
+    b->lds_min = std::min(64 * 1024, (lds + 255) / 256 * 256);
     b->totB = B;
     b->totP = P;
     b->totS = S;

@@ -318,5 +318,15 @@ constexpr int kStageRecords = 16;
 // the most bodies a world may have (one int per body in the record stage).
 constexpr int kLevelInts = 8;
 constexpr int kStageFloat4 = kStageRecords * kVcStride;
+constexpr int kLevelMaxBodies = kStageFloat4 * 4;
+
+// Dynamic LDS in bytes that a step of a world with nbodies bodies makes use of:
+// the body constraint state (32 a body), for worlds of the level form two words
+// per island (at most one island a body), and the record stage.  The eight bytes
+// are for those worlds alone: with them, 1024 piles of 1100 bodies fitted 3
+// instead of 4 to a CU and a step took 35.0 instead of 20.3 ms.
+constexpr int StepLdsBytes(int nbodies) {
+    return nbodies * (nbodies <= kLevelMaxBodies ? 40 : 32) + kStageFloat4 * 16;
+}
 
 }  // namespace prx

@@ -4045,7 +4045,7 @@ __device__ __forceinline__ PosResult island_position_wave(const DeviceState& d, 
 // (kJointRound).  Chain worlds of 32 links with 54 to 85 contacts: periods of
 // 7 to 24 rounds, 120 to 221 rounds for the eight iterations, 170 to 224 with
 // two side by side, and 300 to 400 one after another.
-constexpr int kLevelMaxBodies = prx::kStageFloat4 * 4;
+using prx::kLevelMaxBodies;
 constexpr int kLevelMinConstraints = 4;
 // Updates per round: four lanes serve one update.
 constexpr int kLevelRound = 8;
@@ -5246,8 +5246,7 @@ __device__ __forceinline__ SolveSummary solve_islands(const DeviceState& d, cons
         return (S.istart[is + 1].y - S.istart[is].y) + (S.jstart[is + 1] - S.jstart[is]);
     };
     // The level form needs the body state and two words per island in LDS.
-    const bool levels = kLds && !kTape && x.nb <= kLevelMaxBodies &&
-                        x.nb * 40 + prx::kStageFloat4 * 16 <= int(c.ldsBytes);
+    const bool levels = kLds && !kTape && x.nb <= kLevelMaxBodies && prx::StepLdsBytes(x.nb) <= int(c.ldsBytes);
     const bool revolute = c.jointKinds == 0 && nce + nje <= x.cap;
     auto level = [&](int is) {
         return levels && level_island(S.istart[is + 1].y - S.istart[is].y, S.jstart[is + 1] - S.jstart[is], coopMin, revolute);
