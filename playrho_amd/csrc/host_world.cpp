@@ -28,6 +28,7 @@
 #include "big_world.hpp"
 #include "layout.hpp"
 #include "scenes.hpp"
+#include "schedule.hpp"
 #include "sincosf.hpp"
 
 extern "C" hipError_t prx_launch_step(const prx::DeviceState* d, const prx::StepParams* c, int first, int count,
@@ -3216,11 +3217,12 @@ int prx_batch_autotune(prx_batch* b, const prx_step_conf* step, int nsteps, prx_
             cur = c;
         }
     }
-    const std::uint32_t coopCands[] = {8u, 16u, 32u, 64u, 128u, 0xffffffffu};
-    for (std::uint32_t k : coopCands) {
+    bool allLevel = !b->joint_kinds;
+    for (const prx_world* w : b->worlds) allLevel = allLevel && int(w->bodies.size()) <= prx::kLevelMaxBodies;
+    for (std::uint32_t k : prx::CoopCandidates(allLevel)) {
         prx_batch_conf c = cur;
         c.coop_min_contacts = k;
-        if (c.coop_min_contacts == cur.coop_min_contacts) continue;
+        if (prx::SameSweeps(k, cur.coop_min_contacts, allLevel)) continue;
         float ms = 0;
         if (int st = trial(c, &ms)) return st;
         if (ms < bestMs * kSwitchMargin) {
