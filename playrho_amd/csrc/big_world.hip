@@ -944,13 +944,15 @@ __global__ __launch_bounds__(kGrid) void k_col_commit(DeviceState d, BigState g,
 // launches.  The lowest list position wins a claim, so a round colours a tenth
 // to a half of what is left: of 49,000 touching contacts 22,000 are left after
 // 4 rounds and 1,000 after 8, of which the rest take 6 to 8 rounds more.  With
-// 4 grid rounds this kernel took 340 us.
+// 4 grid rounds this kernel took 340 us.  A round that colours nothing is the
+// last: the lowest position with a free colour always wins, so what is left
+// touches a body that has contacts of every colour, and is solved serially.
 constexpr int kGridRounds = 8;
 __global__ __launch_bounds__(kBlock) void k_col_rest(DeviceState d, BigState g, int first) {
     __shared__ int s_left, s_ncol;
     const int n = g.counters[prx::kBigWork];
     if (n == 0) return;
-    int round = first;
+    int round = first, before = n;
     for (; round < prx::kBigColorRounds; ++round) {
         if (threadIdx.x == 0) s_left = s_ncol = 0;
         for (int k = int(threadIdx.x); k < n; k += kBlock) {
@@ -971,10 +973,11 @@ __global__ __launch_bounds__(kBlock) void k_col_rest(DeviceState d, BigState g, 
         const int rest = s_left;
         if (threadIdx.x == 0 && s_ncol > g.counters[prx::kBigColors]) g.counters[prx::kBigColors] = s_ncol;
         __syncthreads();
-        if (rest == 0) {
+        if (rest == 0 || rest == before) {  // all coloured, or none left has a colour free
             ++round;
             break;
         }
+        before = rest;
     }
     if (threadIdx.x == 0) g.counters[prx::kBigRounds] = round;
 }
@@ -1308,7 +1311,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_big_solve_small(DeviceState d, 
         bs.set_vel(b, d.s_bc_vel[b]);
     }
     // Colours.
-    int colors = 0;
+    int colors = 0, before = m;
     for (int round = 0; round < prx::kBigColorRounds; ++round) {
         if (tid == 0) {
             s_left = 0;
@@ -1330,7 +1333,8 @@ __global__ __launch_bounds__(kSmallBlock) void k_big_solve_small(DeviceState d, 
         colors = s_ncol;
         if (tid == 0) g.counters[prx::kBigRounds] = round + 1;
         __syncthreads();
-        if (rest == 0) break;
+        if (rest == 0 || rest == before) break;
+        before = rest;
     }
     // Colour order.
     if (tid < kBuckets) s_cnt[tid] = 0;

@@ -292,3 +292,43 @@ def test_big_solve_forms_agree(bodies, toi):
         assert np.array_equal(small[k].view(np.uint32), grid[k][:n].view(np.uint32)), k
     for k in ("cu", "ct", "cf", "paabb"):
         assert np.array_equal(small[k].view(np.uint32), grid[k].view(np.uint32)), k
+
+
+def test_big_body_with_more_contacts_than_colours():
+    """A plank on the floor carries 48 disks: its contacts outnumber the
+    colours, the rest are solved serially in list order, with the same bits in
+    the one-workgroup form and the grid's."""
+    import ctypes
+    conf = pa.StepConf(do_toi=0)
+    states = []
+    for extra in (0, 4200):
+        w = pa.World()
+
+        def body(kind, **kw):
+            shape = pa.ShapeConf(density=1.0, friction=0.4, vertex_radius=-1.0, category_bits=1, mask_bits=0xffff,
+                                 **{k: kw.pop(k) for k in ("radius", "hx", "hy") if k in kw})
+            shape.kind = {"disk": 0, "box": 2}[kind]
+            ids = (ctypes.c_uint32 * 1)(w.create_shape(shape))
+            return w.create_body(pa.BodyConf(allow_sleep=1, awake=1, enabled=1, shapes=ids, nshapes=1, **kw))
+
+        body("box", hx=40.0, hy=1.0, type=0, location=(0.0, -1.0))
+        plank = body("box", hx=26.0, hy=0.5, type=2, location=(0.0, 0.5), linear_acceleration=(0.0, -10.0))
+        for k in range(48):
+            body("disk", radius=0.4, type=2, location=(k - 23.5, 1.39), linear_acceleration=(0.0, -10.0))
+        for _ in range(extra):
+            w.create_body(pa.BodyConf())
+        big = pa.BigWorld(w)
+        print("plank", extra, flush=True)
+        for steps in (1, 39):
+            big.step(conf, steps)
+            big.sync()
+        touching = [c for c in w.contacts() if c.point_count and plank in (c.body_a, c.body_b)]
+        assert len(touching) > 40 and big.metrics()["colors"] == 16
+        states.append(dumpfmt.read_state(dumpfmt.Reader(w.state_record())))
+        y = states[-1]["bodies"][2:50, 4]
+        assert np.all(np.abs(y - 1.4) < 0.02), y
+    small, grid = states
+    n = small["bodies"].shape[0]
+    assert np.array_equal(small["bodies"].view(np.uint32), grid["bodies"][:n].view(np.uint32))
+    for k in ("cu", "ct", "cf", "paabb"):
+        assert np.array_equal(small[k].view(np.uint32), grid[k].view(np.uint32)), k
