@@ -40,7 +40,14 @@ constexpr int kBlock = prx::kBigBlock;  // threads of the single-workgroup kerne
 constexpr int kGrid = 256;              // threads per workgroup of the grid-wide kernels
 constexpr int kSweepBlocks = 64;        // workgroups of a colour sweep launch (16,384 threads)
 constexpr int kSmallBlock = 1024;       // threads of the one-workgroup solve and sweeps
-constexpr int kSmallBodies = 4096;      // bodies whose solver state fits one workgroup's LDS beside its tables
+// The most bodies of a world that one workgroup solves (k_big_solve_small); its
+// state would fit LDS up to 4096.  A step by one workgroup and by the grid's
+// launches, boxes of settled drops: 1000 bodies 451 and 534 us, 1500: 530 and
+// 579, 2000: 608 and 603, 2500: 676 and 616, 4000: 935 and 667.  While few have
+// landed the one workgroup stays ahead (4000 bodies: 338 and 463 us at step 20,
+// 605 and 637 at 140, 957 and 742 at 230); the settled state decides, since that
+// is where a world spends its time.
+constexpr int kSmallBodies = 2048;
 constexpr int kBigToiPasses = 2;  // time-of-impact passes per step against static shapes
 // Bound on tree depth for the parent walks (a Karras tree over 30-bit codes
 // with index tie-breaks is at most 30 + 32 deep).

@@ -332,3 +332,25 @@ def test_big_body_with_more_contacts_than_colours():
     assert np.array_equal(small["bodies"].view(np.uint32), grid["bodies"][:n].view(np.uint32))
     for k in ("cu", "ct", "cf", "paabb"):
         assert np.array_equal(small[k].view(np.uint32), grid[k].view(np.uint32)), k
+
+
+def test_big_solve_forms_agree_at_the_limit():
+    """Worlds of 2048 bodies (the most that one workgroup solves), of one more
+    (the grid's launches) and of many more: the same bits."""
+    conf = pa.StepConf(do_toi=0)
+    states = []
+    for total in (2048, 2049, 6200):
+        w = pa.World.scene("drop", [400, 10, 40, 6])
+        while w.body_count < total:
+            w.create_body(pa.BodyConf())
+        print("bodies", total, flush=True)
+        big = pa.BigWorld(w)
+        big.step(conf, 80)
+        big.sync()
+        states.append(dumpfmt.read_state(dumpfmt.Reader(w.state_record())))
+    first = states[0]
+    assert (first["ct"][:, 0] & 0xff).any()
+    for other in states[1:]:
+        for k in ("bodies", "bflags", "cu", "ct", "cf", "paabb"):
+            n = len(first[k])
+            assert np.array_equal(first[k].view(np.uint32), other[k][:n].view(np.uint32)), k
