@@ -993,7 +993,10 @@ __global__ __launch_bounds__(kBlock) void k_col_rest(DeviceState d, BigState g, 
 // first, so that a wavefront's updates take one path of the velocity solve
 // (block or sequential) and of the position solve; the order within a colour
 // does not change a result.  Two buckets per colour, then the serial bucket
-// (list order).
+// (list order).  A box of settled drops, a step with the last launch of a sweep
+// taking colours of 256, 512, 1024, 2048, 4096 and 8192 contacts in all: 5000
+// bodies 670, 659, 675, 679, 750, 911 us; 10,000: 806, 800, 800, 853, 900, 1085;
+// 50,000: 1538, 1540, 1539, 1595, 1608, 1914.
 constexpr int kColourBuckets = 2 * prx::kBigMaxColors;
 constexpr int kBuckets = kColourBuckets + 1;
 __device__ __forceinline__ int colour_bucket(const DeviceState& d, const BigState& g, int e) {
@@ -1001,7 +1004,7 @@ __device__ __forceinline__ int colour_bucket(const DeviceState& d, const BigStat
     if (col < 0) return kColourBuckets;
     return 2 * col + (((d.m_hdr[g.list[e]].x >> 8) & 0xffu) == 2u ? 0 : 1);
 }
-constexpr int kTailContacts = 2048;
+constexpr int kTailContacts = 512;
 
 // Bucket counts of each workgroup's range of the touching list.
 __global__ __launch_bounds__(kGrid) void k_big_buckets(DeviceState d, BigState g) {
@@ -1112,7 +1115,9 @@ __global__ __launch_bounds__(kGrid) void k_big_records(DeviceState d, BigState g
 // so that launch starts at the first colour whose successors hold at most
 // kTailContacts contacts in all, and the grid's launches of later colours
 // return at once.  A launch for each of the 16 colours and the serial bucket
-// spent 2.5 us on every empty one.
+// spent 2.5 us on every empty one.  4, 6, 7, 8 and 10 launches, a step of 10,000
+// settled bodies: 895, 781, 798, 818 and 909 us, of 50,000: 2490, 1587, 1540,
+// 1558 and 1651 (4 and 10 measured with kTailContacts at 2048).
 constexpr int kGridColours = 7;
 
 // The sweeps' work on a constraint: its record (float4 kRec of them, read
