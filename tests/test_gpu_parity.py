@@ -59,12 +59,12 @@ def test_plain_step_matches_reference_every_step(name):
                 pytest.fail("%s: step %d differs from the reference in %s%s" % (name, step, part, detail))
 
 
-@pytest.mark.parametrize("coop_min,toi", [(None, False), (1, False), (1 << 30, False), (None, True)])
+@pytest.mark.parametrize("coop_min,toi", [(None, False), (1, False), (1 << 30, False), (0xffffffff, False), (None, True)])
 def test_batched_step_matches_reference(coop_min, toi):
     """All golden worlds of one doToi setting in one batch, one launch per
-    step.  coop_min 1 sweeps every island with contacts by the whole wavefront
-    (LDS-staged records), 1 << 30 sweeps every island on one lane; all equal
-    the reference."""
+    step.  coop_min 1 sweeps every island with contacts by the wavefront, 1 << 30
+    those of the level form only, 0xffffffff every island on one lane; all
+    equal the reference."""
     names = golden_cases.toi_names() if toi else golden_cases.regular_names()
     gs = [golden_cases.load(n) for n in names]
     worlds = [_recording(pa.World.from_desc(g["desc_conf"])) for g in gs]
