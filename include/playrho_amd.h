@@ -263,8 +263,8 @@ typedef struct prx_batch_conf {
     uint32_t coop_min_contacts; /* islands with at least this many constraints are
                                    swept by the whole wavefront (default 32), and
                                    those of four or more together with others in
-                                   rounds; the greatest values keep every island
-                                   on one lane.  Same results either way */
+                                   rounds; values from 0x7fffffff on keep every
+                                   island on one lane.  Same results either way */
     uint32_t lds_bytes;         /* dynamic LDS per workgroup; 0: the minimum the
                                    batch needs.  Larger values leave fewer
                                    workgroups per CU (160 KB of LDS per CU), so
@@ -550,7 +550,8 @@ int prx_batch_autotune(prx_batch* batch, const prx_step_conf* step, int nsteps,
  * reference counterpart as an API: it is Step(World&, const StepConf&)
  * (World.hpp:917-920) for one world too large for a single wavefront, with
  * the DynamicTree broadphase (DynamicTree.cpp:673-700, AabbTreeWorld.cpp:
- * 709-751) replaced by a linear BVH giving the same pair sets, and the
+ * 709-751) replaced by a direct search over the moved proxies giving the same
+ * pair sets, and the
  * island Gauss-Seidel solve (AabbTreeWorld.cpp:1563-1682) replaced by a
  * colour-parallel Gauss-Seidel over all awake bodies (no sleeping).  The
  * world's state moves to the device (its getters read it back). */

@@ -798,7 +798,8 @@ def device_sincos(angles):
 
 class BigWorld:
     """One large world stepped on the whole device (graph-coloured mode):
-    the reference's pair sets, colour-parallel Gauss-Seidel solve.  The World's getters read the device state back."""
+    the reference's pair sets, colour-parallel Gauss-Seidel solve.  The World's
+    getters read the device state back."""
 
     def __init__(self, world):
         self.world = world

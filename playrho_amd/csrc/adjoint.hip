@@ -20,7 +20,7 @@
 //   material mixing             friction sqrt(fA fB), restitution max(eA, eB) (Contact.hpp:57-69)
 //
 // One launch reverses one recorded step for every world: one wavefront per
-// world, one lane per island (islands share no dynamic body).
+// world, one lane per update of a round (updates that share no moving body).
 #include "adjoint_dual.hpp"
 #include "layout.hpp"
 #include "step_device.hpp"
@@ -1268,9 +1268,11 @@ __attribute__((amdgpu_waves_per_eu(4))) void k_adjoint_general(DeviceState d, Ta
         else contact_creation(code);
     }
     __syncthreads();
-    // The sums, in one order whatever the wavefronts' timing: the bodies' by
-    // one wavefront round after round (twelve lanes an item), the materials' by
-    // another.
+    // The sums: the bodies' by one wavefront round after round (twelve lanes an
+    // item), in one order whatever the wavefronts' timing; the materials' by
+    // another, slots in order, a wavefront's additions to one shape's word in
+    // the order its atomics take (the same from run to run as measured, but
+    // nothing that the hardware promises).
     if (wave == 0) {
         const int l = lane % 12;
         const bool toB = (l % 6) >= 3;

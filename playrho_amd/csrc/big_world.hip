@@ -257,6 +257,7 @@ __global__ __launch_bounds__(kGrid) void k_big_mark(DeviceState d, BigState g, S
 }
 
 constexpr int kMoveStride = 7;  // float4 of a contact record in the compaction's scratch (s_vc2)
+static_assert(kMoveStride <= prx::kQuadVc, "s_vc2 holds kQuadVc float4 a contact slot");
 
 __global__ __launch_bounds__(kGrid) void k_big_gather(DeviceState d, BigState g) {
     __shared__ int s_cnt[kGrid / kWave];

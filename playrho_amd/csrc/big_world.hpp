@@ -73,7 +73,6 @@ struct BigState {
     unsigned long long* claim;
     std::uint64_t* used;  // B: colours taken at the body
     int* tent;        // cap: proposed colour
-    int* win;         // cap
     int* colorStart;  // kBigMaxColors + 2
     // B: the earliest time of impact against a static shape, (float bits << 32
     // | contact index), ~0 for none.

@@ -240,9 +240,12 @@ struct DeviceState {
     float4* s_bc_vel;        // body constraint velocity x, y, w (nbodies)
     float4* s_vc;            // velocity constraints in island order, kVcStride float4 each
     float4* s_pc;            // position constraints in island order, kPcStride float4 each
-    float4* s_vc2;           // level form: velocity constraints of an island in level order
-    float4* s_pc2;           // level form: position constraints of an island in level order
-    int* s_lvl;              // level form: kLevelInts per slot (levels, order, level starts, rounds)
+    // Level form: velocity and position records of all the world's level
+    // islands in one level order, kQuadVc and kQuadPc float4 each (cap of them).
+    // The large world's compaction uses s_vc2 as scratch, 7 float4 a contact.
+    float4* s_vc2;
+    float4* s_pc2;
+    int* s_lvl;              // level form: kLevelInts per slot (levels, order, islands, rounds, level starts)
     float4* s_jc;            // joint constraints in island order, kJcStride float4 each (njoints)
     int* s_isl_joint;        // island joint lists (njoints)
     int* s_isl_jstart;       // island i: first joint entry (nbodies + 1, offset body_off + w)

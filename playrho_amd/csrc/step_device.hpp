@@ -4015,8 +4015,9 @@ __device__ __forceinline__ PosResult island_position_wave(const DeviceState& d, 
 }
 
 // ---------------------------------------------------------------------------
-// Level form of the wave-wide sweeps, for islands without joints in worlds of
-// at most kLevelMaxBodies bodies.  The Gauss-Seidel order is kept exactly: an
+// Level form of the wave-wide sweeps, for islands of contacts and, where all
+// joints of the batch are revolute, joints, in worlds of at most kLevelMaxBodies
+// bodies.  The Gauss-Seidel order is kept exactly: an
 // update's level is one more than the last level that touched either of its
 // bodies (bodies with zero inverse mass and inertia are never changed by an
 // update, so they order nothing), and the updates of one level touch
@@ -4499,8 +4500,9 @@ __device__ __forceinline__ bool quad_joint(QuadBody& me, QuadRec& r, int quad, f
 // allows (one iteration: a plain pass).  Lane 4 (width g + j) + 2 s + c serves
 // update j of group g's round (a group is 4 `width` lanes); group g runs
 // iterations g, g + groups, ...  Bound by the instructions of one round after
-// another, no other wave of the world can help: 1000 cycles for single points,
-// 1400 for two-point contacts or a mix, 360 of them without the updates.  LDS
+// another: 1000 cycles for single points, 1400 for two-point contacts or a mix.
+// 360 of them are not the updates' chain but bounds, record reads and impulse
+// stores, issued by the same (only) wave; a second one could take them.  LDS
 // atomics for the marks cost 200, a path of its own for either kind another
 // 200 in a mixed round.  A pile of 400 bodies: 3.1M -> 2.0M cycles for the
 // velocity and 1.8M -> 1.1M for the position sweeps against two lanes an

@@ -15,8 +15,10 @@
 // (ballot prefix counts), narrowphase (one lane per contact), candidate pair
 // tests, key sort, contact creation, per-body adjacency, synchronisation.
 // Order-dependent phases replay the reference order exactly: the island DFS
-// (one lane) and each island's Gauss-Seidel solve (one lane per island;
-// islands share no dynamic body, so they are independent).
+// (body after body, the wave looking at a body's contacts and joints side by
+// side) and the Gauss-Seidel solve (the updates of a round side by side, four
+// lanes each, where the level form takes the island; else a lane per island or
+// the whole wave for a large one; islands share no dynamic body).
 //
 // A batch of worlds is one launch: workgroup g steps world schedule[g]
 // (largest worlds first), so uneven world sizes balance across the 256 CUs.
