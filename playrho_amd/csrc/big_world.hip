@@ -207,8 +207,8 @@ __device__ __forceinline__ bool hash_has(const BigState& g, int pa, int pb) {
 // scratch, since its slot may hold a record not read yet) and k_big_contacts
 // copies them back.  Contacts before the first destroyed one stay where they
 // are and are not copied; in a settled world few or none move.  One 1024-thread
-// workgroup walking the list took 222 us a step at 73,000 contacts; the three
-// launches take about 13 us with the key set's insertion.
+// workgroup walking the list took 222 us a step at 73,000 contacts; the marks
+// take 8 us and the gathering, with the key set's insertion, 15.
 __device__ __forceinline__ bool still_overlaps(const DeviceState& d, int i) {
     const int2 pr = d.c_prox[i];
     return overlap(d.paabb[pr.x], d.paabb[pr.y]);
@@ -391,8 +391,8 @@ __device__ __forceinline__ std::uint32_t morton_code(float4 b, float4 a) {
 // The test is four comparisons, so 20,000 proxies against all of themselves
 // cost less than the tree that the search once built for each call (sort
 // 169 us and refit 133 us in one workgroup's and one climb's latency at 20,000
-// proxies, whatever had moved): 9 us with the few hundred moved proxies of
-// a settled world and about 0.1 ms with all moved.
+// proxies, whatever had moved): 5 us with nothing moved, 25 on average over a
+// settled world's searches and 0.11 ms with all moved.
 constexpr int kMovedTile = 64;
 constexpr int kMovedSplit = 16;  // grid.y: tiles in flight per proxy
 __global__ __launch_bounds__(kGrid) void k_pairs_find(DeviceState d, BigState g, int slot) {
@@ -952,7 +952,8 @@ __global__ __launch_bounds__(kGrid) void k_col_commit(DeviceState d, BigState g,
 // launches.  The lowest list position wins a claim, so a round colours a tenth
 // to a half of what is left: of 49,000 touching contacts 22,000 are left after
 // 4 rounds and 1,000 after 8, of which the rest take 6 to 8 rounds more.  With
-// 4 grid rounds this kernel took 340 us.  A round that colours nothing is the
+// 4 grid rounds this kernel took 340 us; with 8 it takes 130 over the 600 steps
+// of a drop and 230 over the last 100.  A round that colours nothing is the
 // last: the lowest position with a free colour always wins, so what is left
 // touches a body that has contacts of every colour, and is solved serially.
 constexpr int kGridRounds = 8;
